@@ -2,6 +2,8 @@
 // bias), the qkv split + RoPE pass, GeGLU, row gathers and the scorer's final dot product.
 // Each row is owned by one wavefront (reductions stay in registers and cross-lane shuffles); every
 // global access is a coalesced 16-byte vector per lane.
+#include <type_traits>
+
 #include "device.hpp"
 #include "kernels.hpp"
 
@@ -20,6 +22,14 @@ __device__ __forceinline__ void load8f(const float* __restrict__ p, float* f) {
 __device__ __forceinline__ void store8f(float* p, const float* f) {
   reinterpret_cast<float4*>(p)[0] = make_float4(f[0], f[1], f[2], f[3]);
   reinterpret_cast<float4*>(p)[1] = make_float4(f[4], f[5], f[6], f[7]);
+}
+
+// 8 results at element o of y: 16-bit of type E, or f32 where E is F32.
+struct F32;
+template <class E>
+__device__ __forceinline__ void store8(void* y, size_t o, const float* f) {
+  if constexpr (std::is_same<E, F32>::value) store8f(static_cast<float*>(y) + o, f);
+  else *reinterpret_cast<uint4*>(static_cast<uint16_t*>(y) + o) = pack8<E>(f);
 }
 
 // A hidden-state row of d floats is owned by one wavefront: lane l holds elements
@@ -152,7 +162,7 @@ template <class E, int NC, int SG = NC == 1 ? 16 : NC == 2 ? 10 : 4>
 __global__ __launch_bounds__(256) void splitk_resid_ln_kernel(const float* __restrict__ ws, int splits,
                                                              const float* __restrict__ bias, float* __restrict__ h,
                                                              const float* __restrict__ w, float eps, int T, int d,
-                                                             uint16_t* __restrict__ y, const float* __restrict__ lnb,
+                                                             void* __restrict__ y, const float* __restrict__ lnb,
                                                              const float* __restrict__ hsrc,
                                                              const int* __restrict__ hrows) {
   constexpr int PL = 8 * NC;
@@ -219,7 +229,7 @@ __global__ __launch_bounds__(256) void splitk_resid_ln_kernel(const float* __res
     float o[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) o[e] = (v[c * 8 + e] - mean) * rstd * wv[c * 8 + e] + bv[c * 8 + e];
-    *reinterpret_cast<uint4*>(y + size_t(row) * d + c * 512 + lane * 8) = pack8<E>(o);
+    store8<E>(y, size_t(row) * d + c * 512 + lane * 8, o);
   }
 }
 
@@ -568,7 +578,7 @@ void layernorm_launch(const float* x, const int* rows, const float* w, const flo
 
 template <class E>
 void splitk_resid_ln_t(const float* ws, int splits, const float* bias, float* h, const float* w, float eps, int T, int d,
-                       uint16_t* y, hipStream_t st, const float* lnb, const float* hsrc, const int* hrows) {
+                       void* y, hipStream_t st, const float* lnb, const float* hsrc, const int* hrows) {
   const int rw = row_waves(T);
   dim3 grid((T + rw - 1) / rw), block(64 * rw);
 #define S1_CALL(NC)                                                                                                \
@@ -579,9 +589,13 @@ void splitk_resid_ln_t(const float* ws, int splits, const float* bias, float* h,
 }
 
 void splitk_resid_ln_launch(const float* ws, int splits, const float* bias, float* h, const float* w, float eps, int T,
-                            int d, uint16_t* y, hipStream_t st, int elem, const float* lnb, const float* hsrc,
+                            int d, void* y, hipStream_t st, int elem, const float* lnb, const float* hsrc,
                             const int* hrows) {
   if (T <= 0) return;
+  if (elem == ELEM_F32) {
+    splitk_resid_ln_t<F32>(ws, splits, bias, h, w, eps, T, d, y, st, lnb, hsrc, hrows);
+    return;
+  }
   if (elem == ELEM_F16) splitk_resid_ln_t<F16>(ws, splits, bias, h, w, eps, T, d, y, st, lnb, hsrc, hrows);
   else splitk_resid_ln_t<Bf16>(ws, splits, bias, h, w, eps, T, d, y, st, lnb, hsrc, hrows);
 }

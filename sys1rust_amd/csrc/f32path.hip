@@ -1,104 +1,236 @@
 // Kernels of the dtype=f32 path: the reference's BackendOptions::f32 (f32 weights and compute,
-// runtime/crates/laya-core/src/backend.rs:25-27; laya-mlx/tests/parity.rs:54-65 checks it). It
-// is a numerics mode, not the serving path: plain f32 arithmetic throughout (FMA GEMMs, an exact
-// erf GELU, softmax with expf), written for clarity rather than speed.
+// runtime/crates/laya-core/src/backend.rs:25-27; laya-mlx/tests/parity.rs:54-65 checks it). Plain
+// f32 arithmetic throughout: f32 matrix instructions for the products, an exact erf GELU, f32
+// softmax.
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "device.hpp"
 #include "kernels.hpp"
+#include "lds_load.hpp"
 
 namespace s1 {
 namespace {
 
-// C[M, N] (+)= act(A[M, K] . W[N, K]^T + bias): 64 x 64 tiles, 16-deep slabs of A and W staged
-// transposed in LDS, each of the 256 threads 4 x 4 outputs (rows 4 ty .., columns 4 tx ..).
-constexpr int GT = 64, GK = 16, GP = GT + 4;
-
 __device__ __forceinline__ float gelu_exact(float x) { return 0.5f * x * (1.0f + erff(x * 0.70710678118654752f)); }
 
-__global__ __launch_bounds__(256) void gemm32_kernel(Gemm32Args g) {
-  __shared__ __attribute__((aligned(16))) float sA[GK][GP];
-  __shared__ __attribute__((aligned(16))) float sW[GK][GP];
-  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-  const int m0 = blockIdx.y * GT, n0 = blockIdx.x * GT;
-  const int lr = threadIdx.x >> 2, lk = (threadIdx.x & 3) * 4;  // this thread's float4 of each slab
-  float acc[4][4];
+__device__ __forceinline__ float act32(float v, int act) {
+  return act == ACT_RELU ? fmaxf(v, 0.0f) : act == ACT_GELU ? gelu_exact(v) : v;
+}
+
+// C[M, N] = A[M, K] . W[N, K]^T on v_mfma_f32_32x32x2_f32 (64 FLOP per clock and SIMD: the unit
+// that bounds these products). BM x BN tiles in WM x WN waves, 32-float k-tiles (128-byte rows)
+// moved global -> LDS by direct loads, STAGES deep, one barrier per k-tile; 16-byte chunk c of row
+// r sits at slot c ^ ((r / 2) % 8), so the 16 rows of one fragment read phase start in 16 distinct
+// bank groups.
+//
+// A k-step is 8 floats: lane (row l % 32, h = l / 32) reads 4 consecutive floats (chunk 2 ks + h)
+// of its row with one access, and MFMA u of the step multiplies element u, i.e. k = 8 ks + u from
+// the lanes of half 0 and k = 8 ks + 4 + u from half 1: both operands use the same order, so each
+// k is met once. W is the first operand (C^T = W . A^T): a lane holds 4 consecutive columns of one
+// row and stores them as one float4.
+template <int BM, int BN, int WM, int WN, int STAGES>
+__global__ __launch_bounds__(WM * WN * 64) void gemm32_kernel(Gemm32Args g) {
+  constexpr int NW = WM * WN, TM = BM / WM, TN = BN / WN, FM = TM / 32, FN = TN / 32;
+  constexpr int BKF = 32, ROWB = BKF * 4, CH = 8, RG = 8;
+  constexpr int AG = BM / RG, WG = BN / RG, LPW = (AG + WG) / NW;
+  constexpr int A_BYTES = BM * ROWB, STAGE_BYTES = (BM + BN) * ROWB;
+  static_assert(LPW * NW == AG + WG && AG % NW == 0, "a wave's j-th load reads one operand");
+  static_assert(TM % 32 == 0 && TN % 32 == 0, "whole fragments");
+  __shared__ __attribute__((aligned(1024))) char smem[STAGES * STAGE_BYTES];
+
+  // Tile order as in the 16-bit GEMM: XCD-contiguous runs of 4-row-tile groups across all columns.
+  constexpr int GM = 4;
+  const int mt = (g.M + BM - 1) / BM, nt = g.N / BN;
+  const int bid = xcd_remap(blockIdx.x, gridDim.x);
+  const int grp = bid / (GM * nt);
+  const int gm = min(GM, mt - grp * GM);
+  const int loc = bid - grp * GM * nt;
+  const int m0 = (grp * GM + loc % gm) * BM, n0 = loc / gm * BN;
+  const int ktiles = g.K / BKF, split = blockIdx.y;
+  const int kt0 = int((long long)split * ktiles / g.splits);
+  const int NK = int((long long)(split + 1) * ktiles / g.splits) - kt0;
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+
+  // Loads: the operands are addressed from the tile's own first row, so 32-bit offsets reach it
+  // whatever the matrix spans; rows past M repeat the last one (their results are not stored).
+  const int lrow = lane / CH, lslot = lane % CH;
+  const int mlast = g.M - 1 - m0;
+  uint32_t voff[LPW];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int j = 0; j < LPW; ++j) {
+    const int gi = wave + j * NW;
+    const bool isA = j < AG / NW;
+    const int r = (isA ? gi : gi - AG) * RG + lrow;
+    const int c = lslot ^ ((r >> 1) & 7);
+    voff[j] = (isA ? uint32_t(min(r, mlast)) * uint32_t(g.lda) : uint32_t(r) * uint32_t(g.ldw)) * 4u + c * 16;
+  }
+  const i32x4 rsrcA = buffer_rsrc(g.A + size_t(m0) * g.lda, uint32_t((size_t(min(BM - 1, mlast)) * g.lda + g.K) * 4));
+  const i32x4 rsrcW = buffer_rsrc(g.W + size_t(n0) * g.ldw, uint32_t((size_t(BN - 1) * g.ldw + g.K) * 4));
+  auto issue = [&](int stage, int kt) __attribute__((always_inline)) {
+    const int koff = __builtin_amdgcn_readfirstlane(kt * ROWB);
+    char* sb = smem + stage * STAGE_BYTES + wave * 1024;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = 0.0f;
-  for (int k0 = 0; k0 < g.K; k0 += GK) {
-    float4 av = make_float4(0.0f, 0.0f, 0.0f, 0.0f), wv = av;
-    if (m0 + lr < g.M) av = *reinterpret_cast<const float4*>(g.A + size_t(m0 + lr) * g.lda + k0 + lk);
-    if (n0 + lr < g.N) wv = *reinterpret_cast<const float4*>(g.W + size_t(n0 + lr) * g.ldw + k0 + lk);
-    __syncthreads();  // the previous slab has been read
-    sA[lk][lr] = av.x;
-    sA[lk + 1][lr] = av.y;
-    sA[lk + 2][lr] = av.z;
-    sA[lk + 3][lr] = av.w;
-    sW[lk][lr] = wv.x;
-    sW[lk + 1][lr] = wv.y;
-    sW[lk + 2][lr] = wv.z;
-    sW[lk + 3][lr] = wv.w;
-    __syncthreads();
+    for (int j = 0; j < LPW; ++j) load16_lds(j < AG / NW ? rsrcA : rsrcW, sb + j * NW * 1024, int(voff[j]), koff);
+  };
+
+  f32x16 acc[FM][FN];
 #pragma unroll
-    for (int kk = 0; kk < GK; ++kk) {
-      const float4 a = *reinterpret_cast<const float4*>(&sA[kk][ty * 4]);
-      const float4 w = *reinterpret_cast<const float4*>(&sW[kk][tx * 4]);
-      const float ar[4] = {a.x, a.y, a.z, a.w}, wr[4] = {w.x, w.y, w.z, w.w};
+  for (int i = 0; i < FM; ++i)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+    for (int j = 0; j < FN; ++j)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(ar[i], wr[j], acc[i][j]);
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+
+#pragma unroll
+  for (int s = 0; s < STAGES - 1; ++s)
+    if (s < NK) issue(s, kt0 + s);
+  const int lr = lane & 31, lh = lane >> 5;
+  int ka[4];
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) ka[ks] = lr * ROWB + (((ks * 2 + lh) ^ ((lr >> 1) & 7)) << 4);
+  for (int it = 0; it < NK; ++it) {
+    wait_ahead<LPW, STAGES - 2>(min(STAGES - 2, NK - 1 - it));
+    // Every wave's loads of k-tile `it` have landed and every wave is done with k-tile it - 1,
+    // whose buffer the next issue overwrites.
+    barrier_lds();
+    if (it + STAGES - 1 < NK) issue((it + STAGES - 1) % STAGES, kt0 + it + STAGES - 1);
+    const char* sa = smem + (it % STAGES) * STAGE_BYTES + wm * TM * ROWB;
+    const char* sw = smem + (it % STAGES) * STAGE_BYTES + A_BYTES + wn * TN * ROWB;
+    f32x4 fa[2][FM], fb[2][FN];
+    auto frag = [&](int ks, int buf) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = 0; i < FM; ++i) fa[buf][i] = *reinterpret_cast<const f32x4*>(sa + ka[ks] + i * 32 * ROWB);
+#pragma unroll
+      for (int j = 0; j < FN; ++j) fb[buf][j] = *reinterpret_cast<const f32x4*>(sw + ka[ks] + j * 32 * ROWB);
+    };
+    frag(0, 0);
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      if (ks < 3) frag(ks + 1, (ks + 1) & 1);
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < FN; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[ks & 1][j][u], fa[ks & 1][i][u], acc[i][j], 0, 0, 0);
     }
   }
+
+  // Lane: row m0 + wm TM + 32 i + l % 32, columns n0 + wn TN + 32 j + 8 q + 4 h .. + 3. A split
+  // product leaves its part of the sum in ws[split] for the reduce (splitk32_kernel, or the
+  // consumer's own).
+  const bool part = g.splits > 1;
+  float* out = part ? g.ws + size_t(split) * g.M * g.N : g.C;
+  const int ld = part ? g.N : g.ldc;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int row = m0 + ty * 4 + i;
+  for (int i = 0; i < FM; ++i) {
+    const int row = m0 + wm * TM + i * 32 + lr;
     if (row >= g.M) continue;
+    float* orow = out + size_t(row) * ld + n0 + wn * TN + 4 * lh;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int col = n0 + tx * 4 + j;
-      if (col >= g.N) continue;
-      float v = acc[i][j] + (g.bias ? g.bias[col] : 0.0f);
-      if (g.act == ACT_RELU) v = fmaxf(v, 0.0f);
-      else if (g.act == ACT_GELU) v = gelu_exact(v);
-      float* c = g.C + size_t(row) * g.ldc + col;
-      *c = g.accumulate ? *c + v : v;
-    }
+    for (int j = 0; j < FN; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        float4* o = reinterpret_cast<float4*>(orow + j * 32 + q * 8);
+        float v[4] = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+        if (!part) {
+          if (g.bias) {
+            const float4 b = *reinterpret_cast<const float4*>(g.bias + n0 + wn * TN + 4 * lh + j * 32 + q * 8);
+            v[0] += b.x;
+            v[1] += b.y;
+            v[2] += b.z;
+            v[3] += b.w;
+          }
+#pragma unroll
+          for (int r = 0; r < 4; ++r) v[r] = act32(v[r], g.act);
+          if (g.accumulate) {
+            const float4 c = *o;
+            v[0] += c.x;
+            v[1] += c.y;
+            v[2] += c.z;
+            v[3] += c.w;
+          }
+        }
+        *o = make_float4(v[0], v[1], v[2], v[3]);
+      }
   }
 }
 
+// Four consecutive elements of a product, from C itself (splits 1) or its parts [splits, plane]
+// summed in order.
+__device__ __forceinline__ float4 sum_parts(const float* p, int splits, size_t plane) {
+  float4 s = *reinterpret_cast<const float4*>(p);
+  for (int i = 1; i < splits; ++i) {
+    const float4 v = *reinterpret_cast<const float4*>(p + size_t(i) * plane);
+    s.x += v.x;
+    s.y += v.y;
+    s.z += v.z;
+    s.w += v.w;
+  }
+  return s;
+}
+
+// The end of a split product whose consumer does not sum the parts itself.
+__global__ __launch_bounds__(256) void splitk32_kernel(Gemm32Args g) {
+  const long long gid = (long long)blockIdx.x * 256 + threadIdx.x;
+  const int n4 = g.N / 4;
+  if (gid >= (long long)g.M * n4) return;
+  const int row = int(gid / n4), c = int(gid % n4) * 4;
+  const float4 s = sum_parts(g.ws + size_t(row) * g.N + c, g.splits, size_t(g.M) * g.N);
+  const float4 b = g.bias ? *reinterpret_cast<const float4*>(g.bias + c) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  float4* o = reinterpret_cast<float4*>(g.C + size_t(row) * g.ldc + c);
+  const float4 old = g.accumulate ? *o : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  *o = make_float4(old.x + act32(s.x + b.x, g.act), old.y + act32(s.y + b.y, g.act), old.z + act32(s.z + b.z, g.act),
+                   old.w + act32(s.w + b.w, g.act));
+}
+
 // qkv [T, 3d] -> q, k, v [H, T, 64], with the half-split RoPE rotation of q and k at pos[t] when
-// the tables are given (split_rope.rs:44-54). One thread per (token, head, pair i < 32).
-__global__ __launch_bounds__(256) void split32_kernel(const float* __restrict__ qkv, int T, int d, const int* __restrict__ pos,
+// the tables are given (split_rope.rs:44-54). qkv comes whole, bias added, or as the parts of a
+// split product, which are summed and given the bias here. One thread per (token, head, 4 dim
+// pairs i .. i + 3, i + 32 .. i + 35).
+__global__ __launch_bounds__(256) void split32_kernel(const float* __restrict__ qkv, int splits, const float* __restrict__ bias,
+                                                      int T, int d, const int* __restrict__ pos,
                                                       const float* __restrict__ cs, const float* __restrict__ sn,
                                                       float* __restrict__ q, float* __restrict__ k, float* __restrict__ v) {
   const long long gid = (long long)blockIdx.x * 256 + threadIdx.x;
   const int H = d / 64;
-  if (gid >= (long long)T * H * 32) return;
-  const int i = int(gid % 32), h = int((gid / 32) % H), t = int(gid / (32LL * H));
-  const float* row = qkv + size_t(t) * 3 * d + h * 64;
-  const size_t o = (size_t(h) * T + t) * 64;
-  float c = 1.0f, s = 0.0f;
+  if (gid >= (long long)T * H * 8) return;
+  const int i = int(gid % 8) * 4, h = int((gid / 8) % H), t = int(gid / (8LL * H));
+  const size_t plane = size_t(T) * 3 * d;
+  const float* row = qkv + size_t(t) * 3 * d + h * 64 + i;
+  const size_t o = (size_t(h) * T + t) * 64 + i;
   const bool rot = cs != nullptr;
+  float4 c = make_float4(1.0f, 1.0f, 1.0f, 1.0f), s = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   if (rot) {
-    c = cs[size_t(pos[t]) * 32 + i];
-    s = sn[size_t(pos[t]) * 32 + i];
+    c = *reinterpret_cast<const float4*>(cs + size_t(pos[t]) * 32 + i);
+    s = *reinterpret_cast<const float4*>(sn + size_t(pos[t]) * 32 + i);
   }
-  for (int part = 0; part < 2; ++part) {
-    const float x1 = row[part * d + i], x2 = row[part * d + i + 32];
-    float* dst = (part == 0 ? q : k) + o;
-    if (rot) {
-      dst[i] = x1 * c - x2 * s;
-      dst[i + 32] = x1 * s + x2 * c;
+#pragma unroll
+  for (int part = 0; part < 3; ++part) {
+    float4 x1 = sum_parts(row + part * d, splits, plane), x2 = sum_parts(row + part * d + 32, splits, plane);
+    if (bias) {
+      const float* bp = bias + part * d + h * 64 + i;
+      const float4 b1 = *reinterpret_cast<const float4*>(bp), b2 = *reinterpret_cast<const float4*>(bp + 32);
+      x1 = make_float4(x1.x + b1.x, x1.y + b1.y, x1.z + b1.z, x1.w + b1.w);
+      x2 = make_float4(x2.x + b2.x, x2.y + b2.y, x2.z + b2.z, x2.w + b2.w);
+    }
+    float* dst = (part == 0 ? q : part == 1 ? k : v) + o;
+    if (rot && part < 2) {
+      *reinterpret_cast<float4*>(dst) =
+          make_float4(x1.x * c.x - x2.x * s.x, x1.y * c.y - x2.y * s.y, x1.z * c.z - x2.z * s.z, x1.w * c.w - x2.w * s.w);
+      *reinterpret_cast<float4*>(dst + 32) =
+          make_float4(x1.x * s.x + x2.x * c.x, x1.y * s.y + x2.y * c.y, x1.z * s.z + x2.z * c.z, x1.w * s.w + x2.w * c.w);
     } else {
-      dst[i] = x1;
-      dst[i + 32] = x2;
+      *reinterpret_cast<float4*>(dst) = x1;
+      *reinterpret_cast<float4*>(dst + 32) = x2;
     }
   }
-  v[o + i] = row[2 * d + i];
-  v[o + i + 32] = row[2 * d + i + 32];
 }
 
 // Attention of single queries over a key set each (the entry format of attn_fallback_launch):
@@ -161,37 +293,92 @@ __global__ __launch_bounds__(64) void attn32_kernel(Attn32Args a) {
   a.out[size_t(qrow) * a.ldo + head * 64 + lane] = o / l;
 }
 
-// act[t, i] = gelu(x[t, i]) * x[t, I + i] over x [T, 2I].
-__global__ __launch_bounds__(256) void geglu32_kernel(const float* __restrict__ x, int T, int I, float* __restrict__ act) {
+// act[t, i] = gelu(x[t, i]) * x[t, I + i] over x [T, 2I], whole or the parts of a split product.
+__global__ __launch_bounds__(256) void geglu32_kernel(const float* __restrict__ x, int splits, int T, int I,
+                                                      float* __restrict__ act) {
   const long long gid = (long long)blockIdx.x * 256 + threadIdx.x;
-  if (gid >= (long long)T * I) return;
-  const int t = int(gid / I), i = int(gid % I);
-  const float* row = x + size_t(t) * 2 * I;
-  act[gid] = gelu_exact(row[i]) * row[I + i];
+  const int n4 = I / 4;
+  if (gid >= (long long)T * n4) return;
+  const int t = int(gid / n4), i = int(gid % n4) * 4;
+  const float* row = x + size_t(t) * 2 * I + i;
+  const size_t plane = size_t(T) * 2 * I;
+  const float4 a = sum_parts(row, splits, plane), g = sum_parts(row + I, splits, plane);
+  *reinterpret_cast<float4*>(act + size_t(t) * I + i) =
+      make_float4(gelu_exact(a.x) * g.x, gelu_exact(a.y) * g.y, gelu_exact(a.z) * g.z, gelu_exact(a.w) * g.w);
 }
+
+// out[r] = dot(x[r], w) + b over rows of K floats, one wave per row.
+__global__ __launch_bounds__(64) void rowdot32_kernel(const float* __restrict__ x, const float* __restrict__ w,
+                                                      const float* __restrict__ b, int K, float* __restrict__ out) {
+  const float* row = x + size_t(blockIdx.x) * K;
+  float acc = 0.0f;
+  for (int o = threadIdx.x * 4; o < K; o += 256) {
+    const float4 v = *reinterpret_cast<const float4*>(row + o), u = *reinterpret_cast<const float4*>(w + o);
+    acc = fmaf(v.x, u.x, fmaf(v.y, u.y, fmaf(v.z, u.z, fmaf(v.w, u.w, acc))));
+  }
+  acc = wave_sum(acc);
+  if (threadIdx.x == 0) out[blockIdx.x] = acc + b[0];
+}
+
+template <int BM, int BN, int WM, int WN, int STAGES>
+void gemm32_t(const Gemm32Args& g, hipStream_t st) {
+  const dim3 grid(unsigned((g.M + BM - 1) / BM) * unsigned(g.N / BN), unsigned(g.splits));
+  hipLaunchKernelGGL((gemm32_kernel<BM, BN, WM, WN, STAGES>), grid, dim3(WM * WN * 64), 0, st, g);
+}
+
+// 32-row tiles where they leave fewer rows idle than 64-row ones by a tenth of the product or more.
+bool rows32(int M) { return ((M + 31) / 32) * 32 * 11 <= ((M + 63) / 64) * 64 * 10; }
 
 }  // namespace
 
 const char* gemm32_check(const Gemm32Args& g) {
   if (g.M < 0 || g.N <= 0 || g.K <= 0) return "f32 GEMM: empty shape";
-  if (g.K % GK || g.lda % 4 || g.ldw % 4) return "f32 GEMM: K must be a multiple of 16, lda and ldw of 4";
-  if ((reinterpret_cast<uintptr_t>(g.A) | reinterpret_cast<uintptr_t>(g.W)) % 16) return "f32 GEMM: A and W must be 16-byte aligned";
-  if ((g.M + GT - 1) / GT > 65535) return "f32 GEMM: more than 65535 row tiles (4,194,240 rows)";
+  if (g.K % 32 || g.N % 128) return "f32 GEMM: K must be a multiple of 32, N of 128";
+  if (g.lda < g.K || g.ldw < g.K || g.lda % 4 || g.ldw % 4 || g.ldc % 4) return "f32 GEMM: bad leading dimension";
+  if ((reinterpret_cast<uintptr_t>(g.A) | reinterpret_cast<uintptr_t>(g.W) | reinterpret_cast<uintptr_t>(g.C) |
+       reinterpret_cast<uintptr_t>(g.bias) | reinterpret_cast<uintptr_t>(g.ws)) % 16)
+    return "f32 GEMM: operands must be 16-byte aligned";
+  if (size_t(std::max(g.lda, g.ldw)) * 128 * 4 > 0xffffffffu) return "f32 GEMM: a tile's rows must span less than 4 GiB";
+  if (g.splits < 1 || g.splits > g.K / 32) return "f32 GEMM: splits must be in 1..K/32";
+  if (g.splits > 1 && !g.ws) return "f32 GEMM: a split product needs a workspace";
   return nullptr;
+}
+
+int gemm32_splits(int M, int N, int K) {
+  if (M <= 0) return 1;
+  const int tiles = rows32(M) ? (M + 31) / 32 * (N / 128) : (M + 63) / 64 * (N / 64);
+  const int kt = K / 32;
+  // A tile's work is matrix-unit time, so a launch lasts as long as the CU with the most tiles:
+  // the split that makes that least, each part at least 4 k-tiles and the parts' planes (written
+  // and read back) no more than 8. A part costs about 3 k-tiles of start and end besides.
+  int best = 1;
+  long long least = 0;
+  for (int s = 1; s <= 8 && s <= kt / 4; ++s) {
+    const long long t = (long long)((tiles * s + 255) / 256) * ((kt + s - 1) / s + 3) + 2 * (s > 1);
+    if (s == 1 || t < least) {
+      best = s;
+      least = t;
+    }
+  }
+  return tiles >= 1024 ? 1 : best;
 }
 
 void gemm32_launch(const Gemm32Args& g, hipStream_t st) {
   if (g.M <= 0) return;
-  const dim3 grid((g.N + GT - 1) / GT, (g.M + GT - 1) / GT);
-  hipLaunchKernelGGL(gemm32_kernel, grid, dim3(256), 0, st, g);
+  if (rows32(g.M)) gemm32_t<32, 128, 1, 4, 3>(g, st);
+  else gemm32_t<64, 64, 2, 2, 3>(g, st);
+  if (g.splits > 1 && g.C) {
+    const long long n = (long long)g.M * (g.N / 4);
+    hipLaunchKernelGGL(splitk32_kernel, dim3(unsigned((n + 255) / 256)), dim3(256), 0, st, g);
+  }
 }
 
-void split32_launch(const float* qkv, int T, int d, const int* pos, const float* cos_t, const float* sin_t, float* q,
-                    float* k, float* v, hipStream_t st) {
-  const long long n = (long long)T * (d / 64) * 32;
+void split32_launch(const float* qkv, int splits, const float* bias, int T, int d, const int* pos, const float* cos_t,
+                    const float* sin_t, float* q, float* k, float* v, hipStream_t st) {
+  const long long n = (long long)T * (d / 64) * 8;
   if (n <= 0) return;
-  hipLaunchKernelGGL(split32_kernel, dim3(unsigned((n + 255) / 256)), dim3(256), 0, st, qkv, T, d, pos, cos_t, sin_t,
-                     q, k, v);
+  hipLaunchKernelGGL(split32_kernel, dim3(unsigned((n + 255) / 256)), dim3(256), 0, st, qkv, splits, bias, T, d, pos,
+                     cos_t, sin_t, q, k, v);
 }
 
 void attn32_launch(const Attn32Args& a, hipStream_t st) {
@@ -199,10 +386,15 @@ void attn32_launch(const Attn32Args& a, hipStream_t st) {
   hipLaunchKernelGGL(attn32_kernel, dim3(unsigned(a.n) * unsigned(a.heads)), dim3(64), 0, st, a);
 }
 
-void geglu32_launch(const float* x, int T, int I, float* act, hipStream_t st) {
-  const long long n = (long long)T * I;
+void geglu32_launch(const float* x, int splits, int T, int I, float* act, hipStream_t st) {
+  const long long n = (long long)T * (I / 4);
   if (n <= 0) return;
-  hipLaunchKernelGGL(geglu32_kernel, dim3(unsigned((n + 255) / 256)), dim3(256), 0, st, x, T, I, act);
+  hipLaunchKernelGGL(geglu32_kernel, dim3(unsigned((n + 255) / 256)), dim3(256), 0, st, x, splits, T, I, act);
+}
+
+void rowdot32_launch(const float* x, const float* w, const float* b, int R, int K, float* out, hipStream_t st) {
+  if (R <= 0) return;
+  hipLaunchKernelGGL(rowdot32_kernel, dim3(unsigned(R)), dim3(64), 0, st, x, w, b, K, out);
 }
 
 }  // namespace s1

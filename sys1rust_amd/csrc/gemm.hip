@@ -32,25 +32,13 @@
 
 #include "device.hpp"
 #include "kernels.hpp"
-
-// buffer_load_dwordx4 ... lds: a direct global -> LDS load (LDS address from M0, lane l at + 16 l)
-// whose global address is a buffer resource (scalar) plus a per-lane 32-bit offset and a scalar
-// offset; offsets past the resource's size read 0. The LLVM intrinsic behind it is bound by name,
-// outside any namespace so that the declaration keeps external linkage.
-typedef int i32x4 __attribute__((ext_vector_type(4)));
-__device__ void raw_buffer_load_lds(i32x4 rsrc, __attribute__((address_space(3))) void* lds, int size, int voffset,
-                                    int soffset, int offset, int aux) __asm("llvm.amdgcn.raw.buffer.load.lds");
+#include "lds_load.hpp"
 
 namespace s1 {
 
 namespace {
 
 constexpr int BK = 64;
-
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
 
 // 16 bytes from LDS at an address that is only 8-byte aligned (the staged output tiles pad their
 // rows by 8 bytes, which keeps the fragment writes free of bank conflicts but leaves every other
@@ -61,43 +49,11 @@ __device__ __forceinline__ uint4 lds_load16_a8(const char* p) {
   return make_uint4(lo.x, lo.y, hi.x, hi.y);
 }
 
-// Workgroup barrier without the memory fence of __syncthreads: the fence would make the compiler
-// drain every outstanding global->LDS load (vmcnt(0)) at each k-tile and serialise the pipeline.
-// The "memory" clobber keeps LDS accesses on their side of it; completion of the async loads is
-// awaited explicitly with wait_vmcnt before it.
-__device__ __forceinline__ void barrier_lds() { asm volatile("s_barrier" ::: "memory"); }
-
-// Raw buffer resource over [p, p + bytes): base address, no stride, the byte count, and the third
-// dword of every gfx9 buffer resource (32-bit data format, no swizzle).
-__device__ __forceinline__ i32x4 buffer_rsrc(const void* p, uint32_t bytes) {
-  const uint64_t a = reinterpret_cast<uint64_t>(p);
-  i32x4 r;
-  r.x = __builtin_amdgcn_readfirstlane(int(uint32_t(a)));
-  r.y = __builtin_amdgcn_readfirstlane(int(uint32_t(a >> 32) & 0xffff));
-  r.z = __builtin_amdgcn_readfirstlane(int(bytes));
-  r.w = 0x00020000;
-  return r;
-}
-
 // Bytes from the start of a [rows, ld] 16-bit matrix to the end of its k columns. Every launch
 // keeps both operands' spans below 4 GiB (W by gemm_check; A by gemm_launch, which runs a longer
 // A as row pieces), so a 32-bit offset reaches every element.
 __host__ __device__ inline size_t span_bytes(int rows, int ld, int k) { return (size_t(rows - 1) * ld + k) * 2; }
 constexpr size_t kMaxSpan = (size_t(1) << 32) - 1;
-
-// Wait until at most `ahead` k-tiles of this wave's loads (LPW loads each) are in flight.
-template <int LPW, int MAXA>
-__device__ __forceinline__ void wait_ahead(int ahead) {
-  if constexpr (MAXA > 0) {
-    if (ahead >= MAXA) {
-      wait_vmcnt<MAXA * LPW>();
-      return;
-    }
-    wait_ahead<LPW, MAXA - 1>(ahead);
-  } else {
-    wait_vmcnt<0>();
-  }
-}
 
 // One BM x BN output tile: the k-loop over [kt0, kt0 + NK) and the epilogue.
 //
@@ -166,10 +122,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, char* smem0, int m0
     for (int j = 0; j < LPW; ++j) {
       if (j < jlo || j >= jhi) continue;
       const bool isA = j < AG / NW;
-      raw_buffer_load_lds(isA ? rsrcA : rsrcW,
-                          reinterpret_cast<__attribute__((address_space(3))) void*>(
-                              uint32_t(reinterpret_cast<uintptr_t>(sb + j * NW * 1024))),
-                          16, int(voff[j]), koff, 0, 0);
+      load16_lds(isA ? rsrcA : rsrcW, sb + j * NW * 1024, int(voff[j]), koff);
     }
   };
 

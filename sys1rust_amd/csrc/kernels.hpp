@@ -11,7 +11,8 @@ namespace s1 {
 
 // The 16-bit type of weights and activations (every "bf16" buffer below holds this type): bf16
 // by default, f16 with the model setting dtype=f16.
-enum Elem { ELEM_BF16 = 0, ELEM_F16 = 1 };
+// ELEM_F32 is taken only where a declaration says so.
+enum Elem { ELEM_BF16 = 0, ELEM_F16 = 1, ELEM_F32 = 2 };
 
 enum GemmEpi { EPI_BF16 = 0, EPI_RESID = 1, EPI_GEGLU = 2, EPI_F32 = 3, EPI_ROPE = 4 };
 enum Act { ACT_NONE = 0, ACT_RELU = 1, ACT_GELU = 2 };
@@ -148,8 +149,9 @@ void layernorm_launch(const float* x, const int* rows, const float* w, const flo
 // ws is [splits, T, d] f32, h is [T, d] f32.
 // With hsrc, the residual of row r is row hrows[r] of hsrc (a row gather folded in); the sum
 // still goes to row r of h.
+// y is 16-bit, or f32 with elem = ELEM_F32.
 void splitk_resid_ln_launch(const float* ws, int splits, const float* bias, float* h, const float* w, float eps, int T,
-                            int d, uint16_t* y, hipStream_t st, int elem = ELEM_BF16, const float* lnb = nullptr,
+                            int d, void* y, hipStream_t st, int elem = ELEM_BF16, const float* lnb = nullptr,
                             const float* hsrc = nullptr, const int* hrows = nullptr);
 
 // End of the pruned decision head over its P = n per picked rows ([row 0, kmax scorer rows] per
@@ -185,24 +187,32 @@ void gather_f32_launch(const float* x, const int* rows, int R, int d, float* out
 void rowdot_launch(const uint16_t* x, const float* w, const float* b, int R, int d, float* out, hipStream_t st,
                    int elem = ELEM_BF16);
 
-// ---- The dtype=f32 path (BackendOptions::f32): f32 weights and activations, plain kernels.
+// ---- The dtype=f32 path (BackendOptions::f32): f32 weights and activations.
 
 // C[M, N] (+)= act(A[M, K] . W[N, K]^T + bias), all f32; accumulate adds to C (the residual).
 struct Gemm32Args {
   const float* A = nullptr;  // [M, lda]
   const float* W = nullptr;  // [N, ldw]
-  float* C = nullptr;        // [M, ldc]
+  float* C = nullptr;        // [M, ldc]; null: a split product whose consumer sums the parts
   const float* bias = nullptr;
   int M = 0, N = 0, K = 0, lda = 0, ldw = 0, ldc = 0;
   int act = ACT_NONE;
   bool accumulate = false;
+  // Split product: `splits` workgroups share each output tile, each over a part of K, and write
+  // their sums to ws [splits, M, N]; a second kernel, or the consumer, adds them in order.
+  int splits = 1;
+  float* ws = nullptr;
 };
-// Null when the shape is supported (K a multiple of 16, 16-byte aligned rows), else a message.
+// Null when the shape is supported (K a multiple of 32, N of 128, 16-byte aligned rows), else a
+// message.
 const char* gemm32_check(const Gemm32Args& g);
+// The split gemm32_launch should use for M x N x K (1: none).
+int gemm32_splits(int M, int N, int K);
 void gemm32_launch(const Gemm32Args& g, hipStream_t st);
-// qkv [T, 3d] -> q, k, v [d / 64, T, 64] f32, q and k rotated at pos[t] when cos_t is given.
-void split32_launch(const float* qkv, int T, int d, const int* pos, const float* cos_t, const float* sin_t, float* q,
-                    float* k, float* v, hipStream_t st);
+// qkv [T, 3d] (splits 1, bias null or added here) or the parts [splits, T, 3d] of its product -> q,
+// k, v [d / 64, T, 64] f32, q and k rotated at pos[t] when cos_t is given.
+void split32_launch(const float* qkv, int splits, const float* bias, int T, int d, const int* pos, const float* cos_t,
+                    const float* sin_t, float* q, float* k, float* v, hipStream_t st);
 // Attention of n single queries, each over its key set: entries of 8 int32 as attn_fallback_launch
 // takes them ({query, a0, a1, b0, b1, lo, hi, zeros}); q, k, v [heads, T, 64] f32, out [T, ldo].
 struct Attn32Args {
@@ -215,7 +225,9 @@ struct Attn32Args {
   float scale = 0.125f;
 };
 void attn32_launch(const Attn32Args& a, hipStream_t st);
-// act[t, i] = gelu(x[t, i]) * x[t, I + i] (exact erf) over x [T, 2I] f32.
-void geglu32_launch(const float* x, int T, int I, float* act, hipStream_t st);
+// act[t, i] = gelu(x[t, i]) * x[t, I + i] (exact erf) over x [T, 2I] f32, or its parts [splits, T, 2I].
+void geglu32_launch(const float* x, int splits, int T, int I, float* act, hipStream_t st);
+// out[r] = dot(x[r], w) + b[0] over rows of K floats (K a multiple of 4).
+void rowdot32_launch(const float* x, const float* w, const float* b, int R, int K, float* out, hipStream_t st);
 
 }  // namespace s1

@@ -1342,14 +1342,21 @@ void Model::encoder_hidden(const Plan& p, float* hidden) {
 // entry tables.
 
 struct Model::Acts32 {
-  float *h, *x, *qkv, *q, *k, *v, *att, *mid, *act, *enc, *hh, *sx, *s1, *logits, *pooled;
+  float *h, *x, *qkv, *q, *k, *v, *att, *mid, *act, *enc, *hh, *sx, *s1, *logits, *pooled, *ws;
 };
 
 Model::Acts32 Model::arena32(const Plan& p) {
   const size_t T = size_t(p.T), R = size_t(p.R), n = size_t(p.n);
   const size_t d = size_t(cfg.d), I = size_t(cfg.inter), S = size_t(scorer_width);
+  // Parts of the products that split K, the largest of the forward's.
+  size_t wsf = 0;
+  const size_t shapes[][3] = {{T, 3 * d, d}, {T, d, d}, {T, 2 * I, d}, {T, d, I}, {T, 4 * d, d}, {T, d, 4 * d}, {R, S, d}};
+  for (const auto& sh : shapes) {
+    const int s = gemm32_splits(int(sh[0]), int(sh[1]), int(sh[2]));
+    if (s > 1) wsf = std::max(wsf, s * sh[0] * sh[1]);
+  }
   const size_t sizes[] = {T * d, T * d, T * 3 * d, T * d, T * d, T * d, T * d, T * std::max(2 * I, 4 * d), T * I,
-                          T * d, T * d, R * d, R * S, R, n * d};
+                          T * d, T * d, R * d, R * S, R, n * d, wsf};
   constexpr int NS = sizeof(sizes) / sizeof(sizes[0]);
   size_t off[NS], total = 0;
   for (int i = 0; i < NS; ++i) {
@@ -1368,14 +1375,14 @@ Model::Acts32 Model::arena32(const Plan& p) {
   }
   float* b[NS];
   for (int i = 0; i < NS; ++i) b[i] = reinterpret_cast<float*>(static_cast<char*>(fmem) + off[i]);
-  return Acts32{b[0], b[1], b[2], b[3], b[4], b[5], b[6], b[7], b[8], b[9], b[10], b[11], b[12], b[13], b[14]};
+  return Acts32{b[0], b[1], b[2], b[3], b[4], b[5], b[6], b[7], b[8], b[9], b[10], b[11], b[12], b[13], b[14], b[15]};
 }
 
 namespace {
 
-// C (+)= act(A . W^T + bias) on the f32 GEMM, shapes checked first.
-void gemm32(const float* A, int lda, const float* W, int ldw, float* C, int ldc, const float* bias, int M, int N, int K,
-            int act, bool accumulate, hipStream_t st) {
+// C (+)= act(A . W^T + bias) on the f32 GEMM, split as planned, shapes checked.
+Gemm32Args gemm32_args(const float* A, int lda, const float* W, int ldw, float* C, int ldc, const float* bias, int M, int N,
+                       int K, int act, bool accumulate, float* ws) {
   Gemm32Args g;
   g.A = A;
   g.W = W;
@@ -1389,11 +1396,33 @@ void gemm32(const float* A, int lda, const float* W, int ldw, float* C, int ldc,
   g.ldc = ldc;
   g.act = act;
   g.accumulate = accumulate;
+  g.splits = gemm32_splits(M, N, K);
+  g.ws = ws;
   if (const char* e = gemm32_check(g)) fail(kBackend, e);
-  gemm32_launch(g, st);
+  return g;
+}
+
+// The parts of g's product only, when it splits K (the caller's next kernel sums them); else g.
+Gemm32Args parts_of(Gemm32Args g) {
+  if (g.splits > 1) g.C = nullptr;
+  return g;
 }
 
 }  // namespace
+
+// A residual product g into h, then y = LN(h) (weight w, bias b) over M rows: one kernel after the
+// product when it splits K, which sums the parts and g's bias into h first.
+void Model::resid_ln32(const char* gname, const char* lname, const Gemm32Args& g, float* h, const float* w, const float* b,
+                       float eps, float* y) {
+  const int d = cfg.d;
+  if (g.splits > 1) {
+    op(gname, [&] { gemm32_launch(parts_of(g), stream); });
+    op(lname, [&] { splitk_resid_ln_launch(g.ws, g.splits, g.bias, h, w, eps, g.M, d, y, stream, ELEM_F32, b); });
+  } else {
+    op(gname, [&] { gemm32_launch(g, stream); });
+    op(lname, [&] { layernorm_launch(h, nullptr, w, b, eps, g.M, d, nullptr, y, nullptr, nullptr, nullptr, stream, elem); });
+  }
+}
 
 // encode (lib.rs:1525-1693) in f32 over the plan's rows; a.h holds the residual stream after it.
 void Model::run_encoder32(const Plan& p, const Acts32& a) {
@@ -1409,16 +1438,13 @@ void Model::run_encoder32(const Plan& p, const Acts32& a) {
   for (int l = 0; l < cfg.layers; ++l) {
     const LayerWeights& L = layers[l];
     const int tw = L.local ? 1 : 0;
-    const float* xin = a.h;  // layer 0 attends from the embedding itself
-    if (l > 0) {
-      op("attn_norm", [&] {
-        layernorm_launch(a.h, nullptr, L.attn_norm, nullptr, eps, T, d, nullptr, a.x, nullptr, nullptr, nullptr, stream,
-                         elem);
-      });
-      xin = a.x;
-    }
-    op("wqkv", [&] { gemm32(xin, d, w32(L.wqkv), d, a.qkv, 3 * d, nullptr, T, 3 * d, d, ACT_NONE, false, stream); });
-    op("split_rope", [&] { split32_launch(a.qkv, T, d, pos, rope_cos[tw], rope_sin[tw], a.q, a.k, a.v, stream); });
+    const float* xin = l > 0 ? a.x : a.h;  // layer 0 attends from the embedding itself
+    const Gemm32Args gq = gemm32_args(xin, d, w32(L.wqkv), d, a.qkv, 3 * d, nullptr, T, 3 * d, d, ACT_NONE, false, a.ws);
+    op("wqkv", [&] { gemm32_launch(parts_of(gq), stream); });
+    op("split_rope", [&] {
+      split32_launch(gq.splits > 1 ? a.ws : a.qkv, gq.splits, nullptr, T, d, pos, rope_cos[tw], rope_sin[tw], a.q, a.k, a.v,
+                     stream);
+    });
     op(L.local ? "attn_local" : "attn_global", [&] {
       Attn32Args at;
       at.q = a.q;
@@ -1433,13 +1459,14 @@ void Model::run_encoder32(const Plan& p, const Acts32& a) {
       at.scale = 1.0f / std::sqrt(float(cfg.head_dim()));
       attn32_launch(at, stream);
     });
-    op("wo", [&] { gemm32(a.att, d, w32(L.wo), d, a.h, d, nullptr, T, d, d, ACT_NONE, true, stream); });
-    op("mlp_norm", [&] {
-      layernorm_launch(a.h, nullptr, L.mlp_norm, nullptr, eps, T, d, nullptr, a.x, nullptr, nullptr, nullptr, stream, elem);
-    });
-    op("wi", [&] { gemm32(a.x, d, w32(L.wi), d, a.mid, 2 * I, nullptr, T, 2 * I, d, ACT_NONE, false, stream); });
-    op("geglu", [&] { geglu32_launch(a.mid, T, I, a.act, stream); });
-    op("wo2", [&] { gemm32(a.act, I, w32(L.wo2), I, a.h, d, nullptr, T, d, I, ACT_NONE, true, stream); });
+    resid_ln32("wo", "mlp_norm", gemm32_args(a.att, d, w32(L.wo), d, a.h, d, nullptr, T, d, d, ACT_NONE, true, a.ws), a.h,
+               L.mlp_norm, nullptr, eps, a.x);
+    const Gemm32Args gi = gemm32_args(a.x, d, w32(L.wi), d, a.mid, 2 * I, nullptr, T, 2 * I, d, ACT_NONE, false, a.ws);
+    op("wi", [&] { gemm32_launch(parts_of(gi), stream); });
+    op("geglu", [&] { geglu32_launch(gi.splits > 1 ? a.ws : a.mid, gi.splits, T, I, a.act, stream); });
+    const Gemm32Args go = gemm32_args(a.act, I, w32(L.wo2), I, a.h, d, nullptr, T, d, I, ACT_NONE, true, a.ws);
+    if (l + 1 < cfg.layers) resid_ln32("wo2", "attn_norm", go, a.h, layers[l + 1].attn_norm, nullptr, eps, a.x);
+    else op("wo2", [&] { gemm32_launch(go, stream); });
     layer_mark();
   }
 }
@@ -1462,11 +1489,16 @@ void Model::forward32(const Plan& p, float* logits_out, float* pooled_out) {
   // head_forward (lib.rs:1698-1765): pre-norm layers with biases, ReLU FFN, every row
   for (int j = 0; j < cfg.head_layers; ++j) {
     const HeadWeights& Hw = head[j];
-    op("head_norm1", [&] {
-      layernorm_launch(a.hh, nullptr, Hw.n1w, Hw.n1b, 1e-5f, T, d, nullptr, a.x, nullptr, nullptr, nullptr, stream, elem);
+    if (j == 0)
+      op("head_norm1", [&] {
+        layernorm_launch(a.hh, nullptr, Hw.n1w, Hw.n1b, 1e-5f, T, d, nullptr, a.x, nullptr, nullptr, nullptr, stream, elem);
+      });
+    const Gemm32Args gq = gemm32_args(a.x, d, w32(Hw.in_w), d, a.qkv, 3 * d, Hw.in_b, T, 3 * d, d, ACT_NONE, false, a.ws);
+    op("head_in_proj", [&] { gemm32_launch(parts_of(gq), stream); });
+    op("head_split", [&] {  // a product that does not split adds its bias itself
+      split32_launch(gq.splits > 1 ? a.ws : a.qkv, gq.splits, gq.splits > 1 ? Hw.in_b : nullptr, T, d, nullptr, nullptr,
+                     nullptr, a.q, a.k, a.v, stream);
     });
-    op("head_in_proj", [&] { gemm32(a.x, d, w32(Hw.in_w), d, a.qkv, 3 * d, Hw.in_b, T, 3 * d, d, ACT_NONE, false, stream); });
-    op("head_split", [&] { split32_launch(a.qkv, T, d, nullptr, nullptr, nullptr, a.q, a.k, a.v, stream); });
     op("head_attn", [&] {
       Attn32Args at;
       at.q = a.q;
@@ -1481,14 +1513,15 @@ void Model::forward32(const Plan& p, float* logits_out, float* pooled_out) {
       at.scale = hscale;
       attn32_launch(at, stream);
     });
-    op("head_out_proj", [&] { gemm32(a.att, d, w32(Hw.out_w), d, a.hh, d, Hw.out_b, T, d, d, ACT_NONE, true, stream); });
-    op("head_norm2", [&] {
-      layernorm_launch(a.hh, nullptr, Hw.n2w, Hw.n2b, 1e-5f, T, d, nullptr, a.x, nullptr, nullptr, nullptr, stream, elem);
+    resid_ln32("head_out_proj", "head_norm2",
+               gemm32_args(a.att, d, w32(Hw.out_w), d, a.hh, d, Hw.out_b, T, d, d, ACT_NONE, true, a.ws), a.hh, Hw.n2w, Hw.n2b,
+               1e-5f, a.x);
+    op("head_linear1", [&] {
+      gemm32_launch(gemm32_args(a.x, d, w32(Hw.l1_w), d, a.mid, 4 * d, Hw.l1_b, T, 4 * d, d, ACT_RELU, false, a.ws), stream);
     });
-    op("head_linear1",
-       [&] { gemm32(a.x, d, w32(Hw.l1_w), d, a.mid, 4 * d, Hw.l1_b, T, 4 * d, d, ACT_RELU, false, stream); });
-    op("head_linear2",
-       [&] { gemm32(a.mid, 4 * d, w32(Hw.l2_w), 4 * d, a.hh, d, Hw.l2_b, T, d, 4 * d, ACT_NONE, true, stream); });
+    const Gemm32Args g2 = gemm32_args(a.mid, 4 * d, w32(Hw.l2_w), 4 * d, a.hh, d, Hw.l2_b, T, d, 4 * d, ACT_NONE, true, a.ws);
+    if (j + 1 < cfg.head_layers) resid_ln32("head_linear2", "head_norm1", g2, a.hh, head[j + 1].n1w, head[j + 1].n1b, 1e-5f, a.x);
+    else op("head_linear2", [&] { gemm32_launch(g2, stream); });
   }
   // score (lib.rs:1768-1800): LayerNorm with bias at the marker rows, scorer1 + exact GELU,
   // scorer3; pooled = position 0 of each row
@@ -1497,8 +1530,10 @@ void Model::forward32(const Plan& p, float* logits_out, float* pooled_out) {
       layernorm_launch(a.hh, dmeta + p.off_scorer, sc0_w, sc0_b, 1e-5f, R, d, nullptr, a.sx, nullptr, nullptr, nullptr,
                        stream, elem);
     });
-    op("scorer1", [&] { gemm32(a.sx, d, w32(sc1_w), d, a.s1, S, sc1_b, R, S, d, ACT_GELU, false, stream); });
-    op("scorer3", [&] { gemm32(a.s1, S, sc3_w, S, a.logits, 1, sc3_b, R, 1, S, ACT_NONE, false, stream); });
+    op("scorer1", [&] {
+      gemm32_launch(gemm32_args(a.sx, d, w32(sc1_w), d, a.s1, S, sc1_b, R, S, d, ACT_GELU, false, a.ws), stream);
+    });
+    op("scorer3", [&] { rowdot32_launch(a.s1, sc3_w, sc3_b, R, S, a.logits, stream); });
   }
   op("pooled", [&] { gather_f32_launch(a.hh, dmeta + p.off_pooled, n, d, a.pooled, stream); });
   hip_check(hipGetLastError(), "kernel launch");

@@ -195,6 +195,8 @@ struct Model {
   struct Acts32;
   Acts32 arena32(const Plan& p);
   void run_encoder32(const Plan& p, const Acts32& a);
+  void resid_ln32(const char* gname, const char* lname, const Gemm32Args& g, float* h, const float* w, const float* b,
+                  float eps, float* y);
   void forward32(const Plan& p, float* logits, float* pooled);
   void encoder_hidden32(const Plan& p, float* hidden);
   // The f32 GEMM weights: with dtype=f32 the 16-bit weight pointers hold f32 tensors.
