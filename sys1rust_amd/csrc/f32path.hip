@@ -233,8 +233,172 @@ __global__ __launch_bounds__(256) void split32_kernel(const float* __restrict__ 
   }
 }
 
-// Attention of single queries over a key set each (the entry format of attn_fallback_launch):
-// one wave per (entry, head), 64 keys a step, lane j scoring key j of the step against the query
+// Attention over packed rows in f32, both products on v_mfma_f32_32x32x2_f32, softmax with an
+// online maximum. A wave takes 32 queries of one row and head; the workgroup's four waves are
+// 4 / KW groups of 32 queries, and the KW waves of a group take its 32-key tiles in turn, with
+// softmax statistics of their own, merged through LDS at the end (KW 1: none to merge).
+//
+//   S^T[key, q] = K . Q^T: lane (l % 32, h = l / 32) reads 4 consecutive dims 8 j + 4 h of key row
+//   l % 32 and of query l % 32 at once, and MFMA u of the four multiplies dims 8 j + u and
+//   8 j + 4 + u. The lane then holds query l % 32 and keys 8 g + 4 h + r.
+//   O^T[dim, q] += V^T . P^T: step (g, r) takes keys 8 g + r and 8 g + 4 + r, so the operand P is
+//   the lane's own accumulator 4 g + r, and the operand V a float per lane of two key rows.
+//
+// K and V are read straight from memory: the matrix unit needs 4096 clocks for a tile of a wave,
+// and its 16 KiB, shared by the waves of the workgroup through L1, are well within what that
+// allows, so there is nothing to stage and no barrier in the loop. The next tile's K is loaded
+// before this tile's softmax. Measured at 5707 tokens in 10 rows, 16 heads, against one wave per
+// (query, head) on vector FMAs: global 1720 -> 245 us, local
+// 402 -> 74 us.
+template <int KW>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void attn32_tile_kernel(Attn32Args a) {
+  constexpr float NEG_INF = -__builtin_huge_valf();
+  __shared__ float mt[KW > 1 ? 4 * 64 : 1], lt[KW > 1 ? 4 * 64 : 1], ot[KW > 1 ? 4 * 32 * 64 : 1];
+  const int lid = xcd_remap(blockIdx.x, gridDim.x);
+  const int head = lid / a.n;
+  const AttnTile tl = a.tiles[lid - head * a.n];
+  const int lane = threadIdx.x & 63, col = lane & 31, hl = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wk = wave % KW;
+  const float* __restrict__ Qh = a.q + size_t(head) * a.T * 64;
+  const float* __restrict__ Kh = a.k + size_t(head) * a.T * 64;
+  const float* __restrict__ Vh = a.v + size_t(head) * a.T * 64;
+
+  const int wq0 = tl.q0 + wave / KW * 32;
+  const bool active = wq0 < tl.q1;
+  const int qi = wq0 + col, qld = min(qi, tl.q1 - 1);
+  const int qk = active ? (a.qkey ? a.qkey[qld] : qld) : tl.k0;  // q row and key index of this query
+  int k0 = tl.k0, k1 = tl.k1;
+  if (a.window >= 0) {  // no qkey: slots are key indices
+    k0 = max(k0, wq0 - a.window);
+    k1 = min(k1, min(wq0 + 31, tl.q1 - 1) + a.window + 1);
+  }
+  if (!active) k1 = k0;
+  k0 = __builtin_amdgcn_readfirstlane(k0);
+  k1 = __builtin_amdgcn_readfirstlane(k1);
+  f32x4 qf[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) qf[j] = *reinterpret_cast<const f32x4*>(Qh + size_t(qk) * 64 + j * 8 + hl * 4);
+
+  const float sl2 = a.scale * 1.4426950408889634f;
+  float m = NEG_INF, l = 0.0f;
+  f32x16 o[2];
+#pragma unroll
+  for (int e = 0; e < 16; ++e) o[0][e] = o[1][e] = 0.0f;
+  f32x4 kf[8];
+  auto loadk = [&](int kb) __attribute__((always_inline)) {  // rows past the range repeat its last key
+    const float* kr = Kh + size_t(min(kb + col, k1 - 1)) * 64 + hl * 4;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) kf[j] = *reinterpret_cast<const f32x4*>(kr + j * 8);
+  };
+  if (k0 + wk * 32 < k1) loadk(k0 + wk * 32);
+  for (int kb = k0 + wk * 32; kb < k1; kb += KW * 32) {
+    float v[2][16];
+    const bool whole = kb + 32 <= k1;
+    const float* vr = Vh + size_t(kb + 4 * hl) * 64 + col;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const int off = (e >> 2) * 8 + (e & 3);
+      const float* p = whole ? vr + off * 64 : Vh + size_t(min(kb + 4 * hl + off, k1 - 1)) * 64 + col;
+      v[0][e] = p[0];
+      v[1][e] = p[32];
+    }
+    f32x16 s;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) s[e] = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[j][u], qf[j][u], s, 0, 0, 0);
+    if (kb + KW * 32 < k1) loadk(kb + KW * 32);
+    // Masks where the tile crosses the range's end or some query's window.
+    const int kbase = kb + 4 * hl;
+    int lo = 0, hi = k1 - kbase;
+    bool edge = !whole;
+    if (a.window >= 0) {
+      lo = qk - a.window - kbase;
+      hi = min(hi, qk + a.window + 1 - kbase);
+      edge = edge || kb < wq0 + 31 - a.window || kb + 32 > wq0 + a.window + 1;
+    }
+    if (edge) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int off = (e >> 2) * 8 + (e & 3);
+        s[e] = off >= lo && off < hi ? s[e] : NEG_INF;
+      }
+    }
+    float mx = s[0];
+#pragma unroll
+    for (int e = 1; e < 16; ++e) mx = fmaxf(mx, s[e]);
+    const float mn = fmaxf(m, half_max(mx) * sl2);
+    const float ms = mn == NEG_INF ? 0.0f : mn;  // nothing visible yet
+    const float alpha = __builtin_amdgcn_exp2f(m - ms);
+    float psum = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      s[e] = __builtin_amdgcn_exp2f(fmaf(s[e], sl2, -ms));
+      psum += s[e];
+    }
+    l = l * alpha + psum;
+    m = mn;
+    if (alpha != 1.0f) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        o[0][e] *= alpha;
+        o[1][e] *= alpha;
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      o[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(v[0][e], s[e], o[0], 0, 0, 0);
+      o[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(v[1][e], s[e], o[1], 0, 0, 0);
+    }
+  }
+  l = half_sum(l);
+  float L = l, f[KW];
+  if constexpr (KW > 1) {
+    mt[wave * 64 + lane] = m;
+    lt[wave * 64 + lane] = l;
+#pragma unroll
+    for (int e = 0; e < 32; ++e) ot[(wave * 32 + e) * 64 + lane] = o[e >> 4][e & 15];
+    __syncthreads();
+    if (wk != 0) return;
+    float M = m;
+#pragma unroll
+    for (int w = 1; w < KW; ++w) M = fmaxf(M, mt[(wave + w) * 64 + lane]);
+    L = 0.0f;
+#pragma unroll
+    for (int w = 0; w < KW; ++w) {
+      const float mw = mt[(wave + w) * 64 + lane];
+      f[w] = mw == NEG_INF ? 0.0f : __builtin_amdgcn_exp2f(mw - M);
+      L += lt[(wave + w) * 64 + lane] * f[w];
+    }
+  }
+  if (!active || qi >= tl.q1) return;
+  const float inv = 1.0f / L;
+  float* orow = a.out + size_t(qi) * a.ldo + head * 64 + hl * 4;
+#pragma unroll
+  for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      float r4[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int e = g * 4 + r;
+        float acc = o[dt][e];
+        if constexpr (KW > 1) {
+          acc *= f[0];
+#pragma unroll
+          for (int w = 1; w < KW; ++w) acc += ot[((wave + w) * 32 + dt * 16 + e) * 64 + lane] * f[w];
+        }
+        r4[r] = acc * inv;
+      }
+      *reinterpret_cast<float4*>(orow + dt * 32 + g * 8) = make_float4(r4[0], r4[1], r4[2], r4[3]);
+    }
+}
+
+// Attention of single queries over a key set each (the padded layout's far padding queries, in the
+// entry format of attn_fallback_launch): one wave per (entry, head), 64 keys a step, lane j scoring key j of the step against the query
 // held in LDS, lane c accumulating output dim c; softmax with expf.
 __global__ __launch_bounds__(64) void attn32_kernel(Attn32Args a) {
   __shared__ float sq[64];
@@ -326,8 +490,14 @@ void gemm32_t(const Gemm32Args& g, hipStream_t st) {
   hipLaunchKernelGGL((gemm32_kernel<BM, BN, WM, WN, STAGES>), grid, dim3(WM * WN * 64), 0, st, g);
 }
 
-// 32-row tiles where they leave fewer rows idle than 64-row ones by a tenth of the product or more.
+// Tiles by rows and columns: 64 x 128 once there are two for every CU, else 64 x 64, or 32 x 128
+// where those leave fewer rows idle by a tenth of the product or more (193 rows: 224 instead of
+// 256). At 5707 rows the 64 x 128 tiles in two stages (48 KiB, three workgroups per CU) run the
+// five products of a layer and the head at 128-131 TFLOP/s, 64 x 64 ones at 125, and larger
+// tiles, three or four stages, or the next fragments read across the barrier less: what counts is
+// waves per SIMD to issue matrix instructions while others wait.
 bool rows32(int M) { return ((M + 31) / 32) * 32 * 11 <= ((M + 63) / 64) * 64 * 10; }
+bool wide32(int M, int N) { return (long long)((M + 63) / 64) * (N / 128) >= 512; }
 
 }  // namespace
 
@@ -345,28 +515,30 @@ const char* gemm32_check(const Gemm32Args& g) {
 }
 
 int gemm32_splits(int M, int N, int K) {
-  if (M <= 0) return 1;
+  if (M <= 0 || wide32(M, N)) return 1;
   const int tiles = rows32(M) ? (M + 31) / 32 * (N / 128) : (M + 63) / 64 * (N / 64);
   const int kt = K / 32;
-  // A tile's work is matrix-unit time, so a launch lasts as long as the CU with the most tiles:
-  // the split that makes that least, each part at least 4 k-tiles and the parts' planes (written
-  // and read back) no more than 8. A part costs about 3 k-tiles of start and end besides.
+  // A tile is matrix-unit time, so a launch lasts as long as the CU with the most parts of tiles:
+  // the split that makes that least, each part at least 4 k-tiles, its start and end counted as 4
+  // more, at most 8 parts (they are written and read back). At 193 rows of width 1024, against no
+  // split: q|k|v 26 -> 18 us (3 parts), Wo 25 -> 9.4 (4), Wi 39 -> 30 (3), Wo2 57 -> 18 (4).
   int best = 1;
   long long least = 0;
   for (int s = 1; s <= 8 && s <= kt / 4; ++s) {
-    const long long t = (long long)((tiles * s + 255) / 256) * ((kt + s - 1) / s + 3) + 2 * (s > 1);
+    const long long t = (long long)((tiles * s + 255) / 256) * ((kt + s - 1) / s + 4) + 2 * (s > 1);
     if (s == 1 || t < least) {
       best = s;
       least = t;
     }
   }
-  return tiles >= 1024 ? 1 : best;
+  return best;
 }
 
 void gemm32_launch(const Gemm32Args& g, hipStream_t st) {
   if (g.M <= 0) return;
-  if (rows32(g.M)) gemm32_t<32, 128, 1, 4, 3>(g, st);
-  else gemm32_t<64, 64, 2, 2, 3>(g, st);
+  if (wide32(g.M, g.N)) gemm32_t<64, 128, 2, 2, 2>(g, st);
+  else if (rows32(g.M)) gemm32_t<32, 128, 1, 4, 2>(g, st);
+  else gemm32_t<64, 64, 2, 2, 2>(g, st);
   if (g.splits > 1 && g.C) {
     const long long n = (long long)g.M * (g.N / 4);
     hipLaunchKernelGGL(splitk32_kernel, dim3(unsigned((n + 255) / 256)), dim3(256), 0, st, g);
@@ -381,9 +553,37 @@ void split32_launch(const float* qkv, int splits, const float* bias, int T, int 
                      cos_t, sin_t, q, k, v);
 }
 
+int attn32_plan_tiles(const int* row_start, int n, int heads, int window, std::vector<int>& out, const int* q_end,
+                      const int* k_end) {
+  auto queries = [&](int r) { return (q_end ? q_end[r] : row_start[r + 1]) - row_start[r]; };
+  // 128 queries per workgroup while that gives two workgroups per CU or more, else 64 or 32, whose
+  // keys two or four waves share: the chain of key tiles is what a short batch waits for.
+  int qb = 32;
+  for (int c : {128, 64}) {
+    long long tiles = 0;
+    for (int r = 0; r < n; ++r) tiles += (queries(r) + c - 1) / c;
+    if (tiles * heads >= 512) {
+      qb = c;
+      break;
+    }
+  }
+  for (int r = 0; r < n; ++r) {
+    const int rs = row_start[r], qe = rs + queries(r), ke = k_end ? k_end[r] : row_start[r + 1];
+    for (int q0 = rs; q0 < qe; q0 += qb) {
+      const int t[4] = {q0, std::min(q0 + qb, qe), rs, ke};
+      out.insert(out.end(), t, t + 4);
+    }
+  }
+  return qb;
+}
+
 void attn32_launch(const Attn32Args& a, hipStream_t st) {
   if (a.n <= 0) return;
-  hipLaunchKernelGGL(attn32_kernel, dim3(unsigned(a.n) * unsigned(a.heads)), dim3(64), 0, st, a);
+  const dim3 grid(unsigned(a.n) * unsigned(a.heads));
+  if (a.entries) hipLaunchKernelGGL(attn32_kernel, grid, dim3(64), 0, st, a);
+  else if (a.tile_q == 128) hipLaunchKernelGGL(attn32_tile_kernel<1>, grid, dim3(256), 0, st, a);
+  else if (a.tile_q == 64) hipLaunchKernelGGL(attn32_tile_kernel<2>, grid, dim3(256), 0, st, a);
+  else hipLaunchKernelGGL(attn32_tile_kernel<4>, grid, dim3(256), 0, st, a);
 }
 
 void geglu32_launch(const float* x, int splits, int T, int I, float* act, hipStream_t st) {

@@ -213,17 +213,27 @@ void gemm32_launch(const Gemm32Args& g, hipStream_t st);
 // k, v [d / 64, T, 64] f32, q and k rotated at pos[t] when cos_t is given.
 void split32_launch(const float* qkv, int splits, const float* bias, int T, int d, const int* pos, const float* cos_t,
                     const float* sin_t, float* q, float* k, float* v, hipStream_t st);
-// Attention of n single queries, each over its key set: entries of 8 int32 as attn_fallback_launch
-// takes them ({query, a0, a1, b0, b1, lo, hi, zeros}); q, k, v [heads, T, 64] f32, out [T, ldo].
+// f32 attention, q, k, v [heads, T, 64], out [slots, ldo]: over n work tiles as AttnArgs describes
+// them (up to tile_q slots of one row each, its key range, the window tested per query, qkey), or,
+// with `entries`, of n single queries over a key set each: entries of 8 int32 as
+// attn_fallback_launch takes them ({query, a0, a1, b0, b1, lo, hi, zeros}).
 struct Attn32Args {
   const float* q = nullptr;
   const float* k = nullptr;
   const float* v = nullptr;
   float* out = nullptr;
+  const AttnTile* tiles = nullptr;
   const int* entries = nullptr;
+  const int* qkey = nullptr;  // global attention only
   int n = 0, heads = 0, T = 0, ldo = 0;
+  int tile_q = 32;  // 128, 64 or 32
+  int window = -1;
   float scale = 0.125f;
 };
+// Appends the rows' work tiles to out and returns the queries per tile (Attn32Args::tile_q); q_end
+// and k_end as attn_plan_tiles takes them.
+int attn32_plan_tiles(const int* row_start, int n, int heads, int window, std::vector<int>& out,
+                      const int* q_end = nullptr, const int* k_end = nullptr);
 void attn32_launch(const Attn32Args& a, hipStream_t st);
 // act[t, i] = gelu(x[t, i]) * x[t, I + i] (exact erf) over x [T, 2I] f32, or its parts [splits, T, 2I].
 void geglu32_launch(const float* x, int splits, int T, int I, float* act, hipStream_t st);

@@ -167,10 +167,9 @@ void Model::init(const SafeTensors& st, const std::string& enc_json, const std::
   // headprune prunes the last head layer; with no head layers the scorer reads the encoder's
   // stream whole, as head_forward's loop then leaves it (lib.rs:1726-1765).
   if (cfg.head_layers == 0) set.headprune = false;
-  // dtype=f32 runs the plain f32 kernels: no fused kernels, and the head's last layer over every
-  // row (headprune skips only rows nobody reads, so the outputs are the same). fuserope keeps its
-  // other meaning there: with `band` it chooses the banded local attention (lib.rs:330-361).
-  if (set.f32) set.fusegeglu = set.fuseln = set.headprune = false;
+  // dtype=f32 runs the f32 kernels, none of them fused. fuserope keeps its other meaning there:
+  // with `band` it chooses the banded local attention (lib.rs:330-361).
+  if (set.f32) set.fusegeglu = set.fuseln = false;
   elem = set.f16 ? ELEM_F16 : ELEM_BF16;
   // The forwards `warm` runs at load (warm_buckets) are checked before any device work.
   if (std::any_of(set.warm.begin(), set.warm.end(), [](size_t n) { return n > 0; }))
@@ -542,19 +541,21 @@ Plan Model::plan(uint32_t n, uint32_t len, uint32_t kmax, const uint32_t* ids, c
   // of 8 waves), or 128 or 32 for a short batch; for local ones 128 (4 waves; their keys are only
   // the window), or 32 for a short batch.
   p.off_tiles = m.size();
-  p.gq = attn_plan_tiles(p.row_start.data(), int(n), cfg.heads, -1, m);
+  const auto tiles = set.f32 ? attn32_plan_tiles : attn_plan_tiles;
+  p.gq = tiles(p.row_start.data(), int(n), cfg.heads, -1, m, nullptr, nullptr);
   p.ntiles = int(m.size() - p.off_tiles) / 4;
   p.off_ltiles = m.size();
-  p.lq = attn_plan_tiles(p.row_start.data(), int(n), cfg.heads, cfg.window(), m);
+  p.lq = tiles(p.row_start.data(), int(n), cfg.heads, cfg.window(), m, nullptr, nullptr);
   p.nltiles = int(m.size() - p.off_ltiles) / 4;
   const int per = 1 + int(kmax);
   if (set.headprune) {
     p.off_ptiles = m.size();
     for (uint32_t r = 0; r < n; ++r) {
       const int s0 = int(r) * per, s1 = s0 + per;
-      for (int q0 = s0; q0 < s1; q0 += 128) {
+      const int step = set.f32 ? 32 : 128;
+      for (int q0 = s0; q0 < s1; q0 += step) {
         m.push_back(q0);
-        m.push_back(std::min(q0 + 128, s1));
+        m.push_back(std::min(q0 + step, s1));
         m.push_back(p.row_start[r]);
         m.push_back(p.row_start[r + 1]);
         ++p.nptiles;
@@ -574,23 +575,6 @@ Plan Model::plan(uint32_t n, uint32_t len, uint32_t kmax, const uint32_t* ids, c
   p.off_pooled = m.size();
   for (uint32_t r = 0; r < n; ++r) m.push_back(set.headprune ? int(r) * per : p.row_start[r]);
   pad4();
-  if (set.f32) {
-    // Every token's keys: its row (global layers), the row within the window (local layers).
-    const int W = cfg.window();
-    auto entries = [&](bool local) {
-      for (uint32_t r = 0; r < n; ++r) {
-        const int rs = p.row_start[r], re = p.row_start[r + 1];
-        for (int t = rs; t < re; ++t) {
-          const int e[8] = {t, local ? std::max(rs, t - W) : rs, local ? std::min(re, t + W + 1) : re, rs, rs, 0, 0, 0};
-          m.insert(m.end(), e, e + 8);
-        }
-      }
-    };
-    p.off_eg = m.size();
-    entries(false);
-    p.off_el = m.size();
-    entries(true);
-  }
   return p;
 }
 
@@ -677,37 +661,15 @@ Plan Model::plan_padded(uint32_t n, uint32_t len, const uint32_t* ids, const uin
     }
   }
   p.off_tiles = m.size();
-  p.gq = attn_plan_tiles(p.row_start.data(), int(n), cfg.heads, -1, m, nullptr, kend.data());
+  const auto tiles = set.f32 ? attn32_plan_tiles : attn_plan_tiles;
+  p.gq = tiles(p.row_start.data(), int(n), cfg.heads, -1, m, nullptr, kend.data());
   p.ntiles = int(m.size() - p.off_tiles) / 4;
   p.off_ltiles = m.size();
-  p.lq = attn_plan_tiles(p.row_start.data(), int(n), cfg.heads, W, m, lqend.data(), kend.data());
+  p.lq = tiles(p.row_start.data(), int(n), cfg.heads, W, m, lqend.data(), kend.data());
   p.nltiles = int(m.size() - p.off_ltiles) / 4;
   p.off_far = m.size();
   m.insert(m.end(), far.begin(), far.end());
   p.nfar = int(far.size() / 8);
-  if (set.f32) {
-    // Every position's keys in one table per layer kind: the real keys (global), the real keys
-    // of the window or, past lqend, the far entry above (local).
-    p.off_eg = m.size();
-    for (uint32_t r = 0; r < n; ++r)
-      for (int t = p.row_start[r]; t < p.row_start[r + 1]; ++t) {
-        const int e[8] = {t, p.row_start[r], kend[r], p.row_start[r], p.row_start[r], 0, 0, 0};
-        m.insert(m.end(), e, e + 8);
-      }
-    p.off_el = m.size();
-    size_t fi = 0;
-    for (uint32_t r = 0; r < n; ++r)
-      for (int t = p.row_start[r]; t < p.row_start[r + 1]; ++t) {
-        if (t < lqend[r]) {
-          const int e[8] = {t, std::max(p.row_start[r], t - W), std::min(kend[r], t + W + 1), p.row_start[r],
-                            p.row_start[r], 0, 0, 0};
-          m.insert(m.end(), e, e + 8);
-        } else {
-          m.insert(m.end(), far.begin() + fi, far.begin() + fi + 8);
-          fi += 8;
-        }
-      }
-  }
   p.off_scorer = p.off_pooled = m.size();
   return p;
 }
@@ -1337,26 +1299,26 @@ void Model::encoder_hidden(const Plan& p, float* hidden) {
 }
 
 // ---- dtype=f32 (BackendOptions::f32, backend.rs:25-27): the same graph with f32 weights and
-// activations on the plain f32 kernels, eagerly enqueued (no graphs, no fused kernels, the
-// head's last layer over every row). Every attention query reads its key set from the plan's
-// entry tables.
+// activations on the f32 kernels, eagerly enqueued (no graphs; what is fused is only the sum of a
+// split product's parts into the kernel after it).
 
 struct Model::Acts32 {
-  float *h, *x, *qkv, *q, *k, *v, *att, *mid, *act, *enc, *hh, *sx, *s1, *logits, *pooled, *ws;
+  float *h, *x, *qkv, *q, *k, *v, *att, *mid, *act, *enc, *hh, *sx, *s1, *logits, *pooled, *ws, *hp;
 };
 
 Model::Acts32 Model::arena32(const Plan& p) {
-  const size_t T = size_t(p.T), R = size_t(p.R), n = size_t(p.n);
+  const size_t T = size_t(p.T), P = size_t(p.P), R = size_t(p.R), n = size_t(p.n);
   const size_t d = size_t(cfg.d), I = size_t(cfg.inter), S = size_t(scorer_width);
   // Parts of the products that split K, the largest of the forward's.
   size_t wsf = 0;
-  const size_t shapes[][3] = {{T, 3 * d, d}, {T, d, d}, {T, 2 * I, d}, {T, d, I}, {T, 4 * d, d}, {T, d, 4 * d}, {R, S, d}};
+  const size_t shapes[][3] = {{T, 3 * d, d}, {T, d, d}, {T, 2 * I, d}, {T, d, I}, {T, 4 * d, d}, {T, d, 4 * d}, {P, d, d}, {P, 4 * d, d}, {P, d, 4 * d}, {R, S, d}};
   for (const auto& sh : shapes) {
     const int s = gemm32_splits(int(sh[0]), int(sh[1]), int(sh[2]));
     if (s > 1) wsf = std::max(wsf, s * sh[0] * sh[1]);
   }
-  const size_t sizes[] = {T * d, T * d, T * 3 * d, T * d, T * d, T * d, T * d, T * std::max(2 * I, 4 * d), T * I,
-                          T * d, T * d, R * d, R * S, R, n * d, wsf};
+  const size_t Tp = std::max(T, P);  // the pruned head layer's rows may outnumber the tokens
+  const size_t sizes[] = {T * d, Tp * d, T * 3 * d, T * d, T * d, T * d, Tp * d, Tp * std::max(2 * I, 4 * d), T * I,
+                          T * d, T * d, R * d, R * S, R, n * d, wsf, P * d};
   constexpr int NS = sizeof(sizes) / sizeof(sizes[0]);
   size_t off[NS], total = 0;
   for (int i = 0; i < NS; ++i) {
@@ -1375,7 +1337,7 @@ Model::Acts32 Model::arena32(const Plan& p) {
   }
   float* b[NS];
   for (int i = 0; i < NS; ++i) b[i] = reinterpret_cast<float*>(static_cast<char*>(fmem) + off[i]);
-  return Acts32{b[0], b[1], b[2], b[3], b[4], b[5], b[6], b[7], b[8], b[9], b[10], b[11], b[12], b[13], b[14], b[15]};
+  return Acts32{b[0], b[1], b[2], b[3], b[4], b[5], b[6], b[7], b[8], b[9], b[10], b[11], b[12], b[13], b[14], b[15], b[16]};
 }
 
 namespace {
@@ -1451,13 +1413,20 @@ void Model::run_encoder32(const Plan& p, const Acts32& a) {
       at.k = a.k;
       at.v = a.v;
       at.out = a.att;
-      at.entries = dmeta + (L.local ? p.off_el : p.off_eg);
-      at.n = T;
+      at.tiles = reinterpret_cast<const AttnTile*>(dmeta + (L.local ? p.off_ltiles : p.off_tiles));
+      at.n = L.local ? p.nltiles : p.ntiles;
+      at.tile_q = L.local ? p.lq : p.gq;
+      at.window = L.local ? cfg.window() : -1;
       at.heads = H;
       at.T = T;
       at.ldo = d;
       at.scale = 1.0f / std::sqrt(float(cfg.head_dim()));
       attn32_launch(at, stream);
+      if (L.local && p.nfar > 0) {  // the padding queries that the tiles do not take
+        at.entries = dmeta + p.off_far;
+        at.n = p.nfar;
+        attn32_launch(at, stream);
+      }
     });
     resid_ln32("wo", "mlp_norm", gemm32_args(a.att, d, w32(L.wo), d, a.h, d, nullptr, T, d, d, ACT_NONE, true, a.ws), a.h,
                L.mlp_norm, nullptr, eps, a.x);
@@ -1499,35 +1468,44 @@ void Model::forward32(const Plan& p, float* logits_out, float* pooled_out) {
       split32_launch(gq.splits > 1 ? a.ws : a.qkv, gq.splits, gq.splits > 1 ? Hw.in_b : nullptr, T, d, nullptr, nullptr,
                      nullptr, a.q, a.k, a.v, stream);
     });
+    // headprune (lib.rs:1728-1748): the last layer's queries and all after them at the picked rows.
+    const bool pruned = set.headprune && j + 1 == cfg.head_layers;
+    const int* picked = dmeta + p.off_picked;
+    const int M = pruned ? p.P : T;
+    float* hj = pruned ? a.hp : a.hh;
     op("head_attn", [&] {
       Attn32Args at;
       at.q = a.q;
       at.k = a.k;
       at.v = a.v;
       at.out = a.att;
-      at.entries = dmeta + p.off_eg;
-      at.n = T;
+      at.tiles = reinterpret_cast<const AttnTile*>(dmeta + (pruned ? p.off_ptiles : p.off_tiles));
+      at.n = pruned ? p.nptiles : p.ntiles;
+      at.tile_q = pruned ? 32 : p.gq;
+      at.qkey = pruned ? picked : nullptr;
       at.heads = Hh;
       at.T = T;
       at.ldo = d;
       at.scale = hscale;
       attn32_launch(at, stream);
     });
+    if (pruned) op("head_pick", [&] { gather_f32_launch(a.hh, picked, M, d, hj, stream); });
     resid_ln32("head_out_proj", "head_norm2",
-               gemm32_args(a.att, d, w32(Hw.out_w), d, a.hh, d, Hw.out_b, T, d, d, ACT_NONE, true, a.ws), a.hh, Hw.n2w, Hw.n2b,
+               gemm32_args(a.att, d, w32(Hw.out_w), d, hj, d, Hw.out_b, M, d, d, ACT_NONE, true, a.ws), hj, Hw.n2w, Hw.n2b,
                1e-5f, a.x);
     op("head_linear1", [&] {
-      gemm32_launch(gemm32_args(a.x, d, w32(Hw.l1_w), d, a.mid, 4 * d, Hw.l1_b, T, 4 * d, d, ACT_RELU, false, a.ws), stream);
+      gemm32_launch(gemm32_args(a.x, d, w32(Hw.l1_w), d, a.mid, 4 * d, Hw.l1_b, M, 4 * d, d, ACT_RELU, false, a.ws), stream);
     });
-    const Gemm32Args g2 = gemm32_args(a.mid, 4 * d, w32(Hw.l2_w), 4 * d, a.hh, d, Hw.l2_b, T, d, 4 * d, ACT_NONE, true, a.ws);
-    if (j + 1 < cfg.head_layers) resid_ln32("head_linear2", "head_norm1", g2, a.hh, head[j + 1].n1w, head[j + 1].n1b, 1e-5f, a.x);
+    const Gemm32Args g2 = gemm32_args(a.mid, 4 * d, w32(Hw.l2_w), 4 * d, hj, d, Hw.l2_b, M, d, 4 * d, ACT_NONE, true, a.ws);
+    if (j + 1 < cfg.head_layers) resid_ln32("head_linear2", "head_norm1", g2, hj, head[j + 1].n1w, head[j + 1].n1b, 1e-5f, a.x);
     else op("head_linear2", [&] { gemm32_launch(g2, stream); });
   }
+  const float* hs = set.headprune ? a.hp : a.hh;  // the rows that off_scorer and off_pooled index
   // score (lib.rs:1768-1800): LayerNorm with bias at the marker rows, scorer1 + exact GELU,
   // scorer3; pooled = position 0 of each row
   if (R > 0) {
     op("scorer_norm", [&] {
-      layernorm_launch(a.hh, dmeta + p.off_scorer, sc0_w, sc0_b, 1e-5f, R, d, nullptr, a.sx, nullptr, nullptr, nullptr,
+      layernorm_launch(hs, dmeta + p.off_scorer, sc0_w, sc0_b, 1e-5f, R, d, nullptr, a.sx, nullptr, nullptr, nullptr,
                        stream, elem);
     });
     op("scorer1", [&] {
@@ -1535,7 +1513,7 @@ void Model::forward32(const Plan& p, float* logits_out, float* pooled_out) {
     });
     op("scorer3", [&] { rowdot32_launch(a.s1, sc3_w, sc3_b, R, S, a.logits, stream); });
   }
-  op("pooled", [&] { gather_f32_launch(a.hh, dmeta + p.off_pooled, n, d, a.pooled, stream); });
+  op("pooled", [&] { gather_f32_launch(hs, dmeta + p.off_pooled, n, d, a.pooled, stream); });
   hip_check(hipGetLastError(), "kernel launch");
   if (R > 0) hip_check(hipMemcpyAsync(logits_out, a.logits, size_t(R) * 4, hipMemcpyDeviceToHost, stream), "download logits");
   hip_check(hipMemcpyAsync(pooled_out, a.pooled, size_t(n) * d * 4, hipMemcpyDeviceToHost, stream), "download pooled");

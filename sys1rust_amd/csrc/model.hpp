@@ -108,9 +108,6 @@ struct Plan {
   bool padded = false;
   size_t off_far = 0;
   int nfar = 0;
-  // dtype=f32: every query's key set in attn32_launch's entry format, for global (off_eg) and
-  // local (off_el) layers, T entries each.
-  size_t off_eg = 0, off_el = 0;
 };
 
 struct Model {

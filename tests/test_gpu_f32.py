@@ -193,3 +193,40 @@ def test_f32_random_batches(small):
         lg, pl = o.forward(b, ref)
         gate_f32(m, b, ref, lg, pl, act, f"f32 random {case} n={b.n} len={b.len} kmax={b.kmax}")
     m.close()
+
+
+# Rows at the edges of the f32 kernels' tiles (32, 64 and 128 rows of a product, 32-key and 32- to
+# 128-query attention tiles), alone and in batches, the largest on the tiles of a long batch; a
+# window of 32 keys on each side; more answer slots than tokens.
+EDGES = [([1], 0), ([31], 1), ([33, 64], 2), ([65, 1, 32], 3), ([127, 129, 128], 2), ([193], 3), ([600] * 9 + [37], 4),
+         ([3, 5], 9)]
+
+
+@pytest.mark.parametrize("lens,kmax", EDGES)
+def test_f32_tile_edges(lens, kmax):
+    from oracle.oracle import Oracle
+    from sys1rust_amd.workloads import collate, small_config
+
+    cfg = small_config(layers=3, vocab=1024, local_attention=64)
+    cfg["pad_token_id"] = 1002
+    rng = np.random.default_rng(sum(lens) + kmax)
+    items = []
+    for L in lens:
+        markers = sorted(rng.integers(0, L, kmax).tolist())
+        items.append((rng.integers(0, 1000, L).tolist(), markers, int(rng.integers(0, 3))))
+    b = collate(items, pad_id=1002)
+    st = synth_checkpoint(json.dumps(cfg), json.dumps(AGENT), seed=5, scorer_width=256)
+    m = HipBackend(st, json.dumps(cfg), json.dumps(AGENT), settings=DEFAULT_TUNING + ",dtype=f32", device=0)
+    o = TorchOracle(Oracle(st, cfg, AGENT), "cuda")
+    ref = np.zeros((b.n, b.len, 512), np.float32)
+    for r, L in enumerate(lens):  # the packed forward: each row by itself
+        one = Batch(1, L, 0, b.input_ids.reshape(b.n, -1)[r, :L], np.ones(L, np.uint32), np.array([L], np.uint64),
+                    np.zeros(0, np.uint32), np.zeros(1, np.uint64), b.qtype[r: r + 1])
+        ref[r, :L] = o.encoder_hidden(one)[0]
+    lg, pl = o.forward(b, ref)
+    out = m.forward(b)
+    say(f"f32 rows {lens} slots {kmax}")
+    if kmax:
+        assert float(np.abs(out.logits - lg).max()) <= LOGIT_ABS_F32
+    pg, pr = out.pooled.reshape(b.n, -1), pl.reshape(b.n, -1)
+    assert float((np.linalg.norm(pg - pr, axis=-1) / np.linalg.norm(pr, axis=-1)).max()) <= POOLED_REL_F32
