@@ -719,65 +719,148 @@ __global__ __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
 // the window. Each entry names the set, as the host works it out from the masks
 // (lib.rs:1241-1310): {query, a0, a1, b0, b1, lo, hi, zeros} = keys [a0, a1) and [b0, b1) (packed
 // indices), key a0 counted 1 + lo times, the last key of the last non-empty range 1 + hi times
-// (gathered slots clamped to one key), and `zeros` slots of zero key and value (score 0, value
-// 0). One wave per (entry, head), 64 keys a step: lane j scores key j of the step in f32, lane d
-// accumulates output dim d.
+// (gathered slots clamped to one key), and `zeros` slots of zero key and value (score 0, value 0).
+//
+// A workgroup takes a tile of up to 32 consecutive entries of one row and one head; its four waves
+// take the 32-key tiles of the entries' key ranges (their unions, from the host) in turn and merge
+// through LDS, and each lane masks the keys that its own query's entry does not name. The weights
+// stay in f32: the scores come from the 16-bit MFMA (S^T = K . Q^T) and the weighted sum from the
+// f32 one (v_mfma_f32_32x32x2: step 4g + r takes keys 8g + r and 8g + 4 + r, so its second operand
+// is the lane's own weight). Loads go straight to registers: the sets are a few hundred keys that
+// the tiles of a row share through L2, and what bounds the kernel is each wave's chain of about
+// three key tiles. Measured at 1780 entries of 64 to 320 keys, 16 heads, against one wave per
+// (entry, head) on vector FMAs: @FAR@.
 template <class E>
-__global__ __launch_bounds__(64) void attn_fallback_kernel(FallbackArgs a) {
-  __shared__ float sp[64];
-  const int fi = blockIdx.x / a.heads, head = blockIdx.x % a.heads;
-  const int4 f0 = reinterpret_cast<const int4*>(a.far)[2 * fi];      // query, a0, a1, b0
-  const int4 f1 = reinterpret_cast<const int4*>(a.far)[2 * fi + 1];  // b1, lo, hi, zeros
-  const int lane = threadIdx.x;
+__global__ __launch_bounds__(256) void attn_far_kernel(FallbackArgs a) {
+  typedef typename E::v8 v8;
+  constexpr int KW = 4;
+  __shared__ float mt[KW * 64], lt[KW * 64], ot[KW * 32 * 64];
+  const int lid = xcd_remap(blockIdx.x, gridDim.x);
+  const int head = lid / a.ntiles;
+  const int* tile = a.tiles + size_t(lid - head * a.ntiles) * 8;
+  const int e0 = tile[0], e1 = tile[1];
+  const int lane = threadIdx.x & 63, hl = lane >> 5, col = lane & 31;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int ei = min(e0 + col, e1 - 1);
+  const int4 f0 = reinterpret_cast<const int4*>(a.far)[2 * ei];      // query, a0, a1, b0
+  const int4 f1 = reinterpret_cast<const int4*>(a.far)[2 * ei + 1];  // b1, lo, hi, zeros
   const uint16_t* __restrict__ Qh = a.q + size_t(head) * a.T * 64;
   const uint16_t* __restrict__ Kh = a.k + size_t(head) * a.T * 64;
   const uint16_t* __restrict__ Vt = a.v + size_t(head) * 64 * a.ldv;
-  float qv[64];
+  v8 qf[4];
 #pragma unroll
-  for (int c = 0; c < 8; ++c) unpack8<E>(*reinterpret_cast<const uint4*>(Qh + size_t(f0.x) * 64 + c * 8), qv + c * 8);
+  for (int kb = 0; kb < 4; ++kb)
+    qf[kb] = *reinterpret_cast<const v8*>(Qh + size_t(f0.x) * 64 + kb * 16 + hl * 8);
   const float sl2 = a.scale * 1.4426950408889634f;
   // Repeated keys: the weight of n copies is exp2(s + log2 n).
   const int klo = f0.y, khi = (f1.x > f0.w ? f1.x : f0.z) - 1;
-  const float llo = log2f(float(1 + f1.y)), lhi = log2f(float(1 + f1.z));
-  float m = NEG_INF, l = 0.0f, o = 0.0f;
-  auto keys = [&](int j0, int j1) {
-    for (int b = j0; b < j1; b += 64) {
-      const int j = b + lane;
-      float s = NEG_INF;
-      if (j < j1) {
-        float kv[8], dot = 0.0f;
+  const float llo = __builtin_amdgcn_logf(float(1 + f1.y)), lhi = __builtin_amdgcn_logf(float(1 + f1.z));
+  float m = NEG_INF, l = 0.0f;
+  f32x16 o[2];
 #pragma unroll
-        for (int c = 0; c < 8; ++c) {
-          unpack8<E>(*reinterpret_cast<const uint4*>(Kh + size_t(j) * 64 + c * 8), kv);
+  for (int e = 0; e < 16; ++e) o[0][e] = o[1][e] = 0.0f;
+  // 32-key tiles start 8-aligned, so V^T is read in aligned pieces of 4 keys; pieces past the range
+  // repeat the one of its last key (finite values that meet weights of 0).
+  const int first[2] = {tile[2] & ~7, tile[4] & ~7}, end[2] = {tile[3], tile[5]};
+  const int na = (end[0] - first[0] + 31) >> 5, nb = (end[1] - first[1] + 31) >> 5;
+  for (int t = wave; t < na + nb; t += KW) {
+    const bool isb = t >= na;
+    const int kb = isb ? first[1] + (t - na) * 32 : first[0] + t * 32, last = (isb ? end[1] : end[0]) - 1;
+    const int r0 = isb ? f0.w : f0.y, r1 = isb ? f1.x : f0.z;  // this query's keys of the range
+    const uint16_t* kr = Kh + size_t(min(kb + col, last)) * 64 + hl * 8;
+    v8 kf[4];
+    uint2 vr[2][4];
 #pragma unroll
-          for (int e = 0; e < 8; ++e) dot = fmaf(qv[c * 8 + e], kv[e], dot);
-        }
-        s = dot * sl2 + (j == klo ? llo : 0.0f) + (j == khi ? lhi : 0.0f);
-      }
-      const float mn = fmaxf(m, wave_max(s));
-      const float p = j < j1 ? __builtin_amdgcn_exp2f(s - mn) : 0.0f;
-      const float alpha = m == NEG_INF ? 0.0f : __builtin_amdgcn_exp2f(m - mn);
-      l = l * alpha + wave_sum(p);
-      o *= alpha;
-      m = mn;
-      sp[lane] = p;
-      __syncthreads();
-      const uint16_t* vr = Vt + size_t(lane) * a.ldv + b;  // dim `lane`, keys b ..
-      const int cnt = min(64, j1 - b);
-      for (int t = 0; t < cnt; ++t) o = fmaf(sp[t], E::f32(vr[t]), o);
-      __syncthreads();
+    for (int j = 0; j < 4; ++j) kf[j] = *reinterpret_cast<const v8*>(kr + j * 16);
+#pragma unroll
+    for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        vr[dt][g] = *reinterpret_cast<const uint2*>(Vt + size_t(dt * 32 + col) * a.ldv + min(kb + 8 * g + 4 * hl, last & ~3));
+    f32x16 s;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) s[e] = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) s = E::mfma(kf[j], qf[j], s);
+    const int kbase = kb + 4 * hl;
+    float mx = NEG_INF;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const int key = kbase + (e >> 2) * 8 + (e & 3);
+      s[e] = fmaf(s[e], sl2, (key == klo ? llo : 0.0f) + (key == khi ? lhi : 0.0f));
+      s[e] = key >= r0 && key < r1 ? s[e] : NEG_INF;
+      mx = fmaxf(mx, s[e]);
     }
-  };
-  keys(f0.y, f0.z);
-  keys(f0.w, f1.x);
-  if (f1.w > 0) {  // zero slots: score 0, value 0, weight `zeros`
-    const float sz = log2f(float(f1.w));
-    const float mn = fmaxf(m, sz);
-    const float alpha = m == NEG_INF ? 0.0f : __builtin_amdgcn_exp2f(m - mn);
-    l = l * alpha + __builtin_amdgcn_exp2f(sz - mn);
-    o *= alpha;
+    const float mn = fmaxf(m, half_max(mx));
+    const float ms = mn == NEG_INF ? 0.0f : mn;  // nothing visible yet
+    const float alpha = __builtin_amdgcn_exp2f(m - ms);
+    float psum = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      s[e] = __builtin_amdgcn_exp2f(s[e] - ms);
+      psum += s[e];
+    }
+    l = l * alpha + psum;
+    m = mn;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      o[0][e] *= alpha;
+      o[1][e] *= alpha;
+    }
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+#pragma unroll
+      for (int dt = 0; dt < 2; ++dt) {
+        const uint32_t w = (e & 2) ? vr[dt][e >> 2].y : vr[dt][e >> 2].x;
+        const float v = E::f32(uint16_t((e & 1) ? w >> 16 : w));
+        o[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(v, s[e], o[dt], 0, 0, 0);
+      }
+    }
   }
-  a.out[size_t(f0.x) * a.ldo + head * 64 + lane] = E::bits(o / l);
+  l = half_sum(l);
+  if (wave == 0 && f1.w > 0) {  // zero slots: score 0, value 0, weight `zeros`
+    const float sz = __builtin_amdgcn_logf(float(f1.w));
+    const float mn = fmaxf(m, sz);
+    const float alpha = __builtin_amdgcn_exp2f(m - mn);
+    l = l * alpha + __builtin_amdgcn_exp2f(sz - mn);
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      o[0][e] *= alpha;
+      o[1][e] *= alpha;
+    }
+    m = mn;
+  }
+  mt[wave * 64 + lane] = m;
+  lt[wave * 64 + lane] = l;
+#pragma unroll
+  for (int e = 0; e < 32; ++e) ot[(wave * 32 + e) * 64 + lane] = o[e >> 4][e & 15];
+  __syncthreads();
+  // Wave w combines and stores dims 8 w .. 8 w + 7 of both halves' pieces: g = w of each 32 dims.
+  if (e0 + col >= e1) return;
+  float M = NEG_INF;
+#pragma unroll
+  for (int w = 0; w < KW; ++w) M = fmaxf(M, mt[w * 64 + lane]);
+  float f[KW], L = 0.0f;
+#pragma unroll
+  for (int w = 0; w < KW; ++w) {
+    f[w] = __builtin_amdgcn_exp2f(mt[w * 64 + lane] - M);
+    L += lt[w * 64 + lane] * f[w];
+  }
+  const float inv = 1.0f / L;
+  uint16_t* orow = a.out + size_t(f0.x) * a.ldo + head * 64 + wave * 8 + hl * 4;
+#pragma unroll
+  for (int dt = 0; dt < 2; ++dt) {
+    float v[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int e = dt * 16 + wave * 4 + r;
+      float acc = 0.0f;
+#pragma unroll
+      for (int w = 0; w < KW; ++w) acc += ot[(w * 32 + e) * 64 + lane] * f[w];
+      v[r] = acc * inv;
+    }
+    *reinterpret_cast<uint2*>(orow + dt * 32) = make_uint2(E::pack2(v[0], v[1]), E::pack2(v[2], v[3]));
+  }
 }
 
 }  // namespace
@@ -865,10 +948,30 @@ void attn_launch(const AttnArgs& a, hipStream_t st) {
 }
 
 void attn_fallback_launch(const FallbackArgs& a, hipStream_t st) {
-  if (a.nfar <= 0) return;
-  const dim3 grid(unsigned(a.nfar) * unsigned(a.heads));
-  if (a.elem == ELEM_F16) hipLaunchKernelGGL(attn_fallback_kernel<F16>, grid, dim3(64), 0, st, a);
-  else hipLaunchKernelGGL(attn_fallback_kernel<Bf16>, grid, dim3(64), 0, st, a);
+  if (a.ntiles <= 0) return;
+  const dim3 grid(unsigned(a.ntiles) * unsigned(a.heads));
+  if (a.elem == ELEM_F16) hipLaunchKernelGGL(attn_far_kernel<F16>, grid, dim3(256), 0, st, a);
+  else hipLaunchKernelGGL(attn_far_kernel<Bf16>, grid, dim3(256), 0, st, a);
+}
+
+void attn_far_tiles(const std::vector<int>& far, const int* row_far, int n, std::vector<int>& out) {
+  for (int r = 0; r < n; ++r)
+    for (int e0 = row_far[r]; e0 < row_far[r + 1]; e0 += 32) {
+      const int e1 = std::min(e0 + 32, row_far[r + 1]);
+      int u[4] = {0, 0, 0, 0};  // union of the entries' non-empty a ranges, then of their b ranges
+      for (int i = 0; i < 2; ++i) {
+        bool any = false;
+        for (int e = e0; e < e1; ++e) {
+          const int k0 = far[size_t(e) * 8 + 1 + 2 * i], k1 = far[size_t(e) * 8 + 2 + 2 * i];
+          if (k1 <= k0) continue;
+          u[2 * i] = any ? std::min(u[2 * i], k0) : k0;
+          u[2 * i + 1] = any ? std::max(u[2 * i + 1], k1) : k1;
+          any = true;
+        }
+      }
+      const int t[8] = {e0, e1, u[0], u[1], u[2], u[3], 0, 0};
+      out.insert(out.end(), t, t + 8);
+    }
 }
 
 }  // namespace s1

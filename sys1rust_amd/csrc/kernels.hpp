@@ -116,17 +116,23 @@ int attn_plan_tiles(const int* row_start, int n, int heads, int window, std::vec
 // window. far: nfar entries of 8 int32 (device, 16-byte aligned) {query, a0, a1, b0, b1, lo, hi,
 // zeros}: keys [a0, a1) and [b0, b1), key a0 counted 1 + lo times, the last key of the last
 // non-empty range 1 + hi times, plus `zeros` slots of zero key and value. Every entry has a key.
+// tiles: ntiles work tiles of 8 int32 as attn_far_tiles lists them.
 struct FallbackArgs {
   const uint16_t* q = nullptr;
   const uint16_t* k = nullptr;
   const uint16_t* v = nullptr;  // transposed, [H, 64, ldv]
   uint16_t* out = nullptr;      // [T, ldo]
   const int* far = nullptr;
-  int nfar = 0, heads = 0, T = 0, ldv = 0, ldo = 0;
+  const int* tiles = nullptr;
+  int ntiles = 0, heads = 0, T = 0, ldv = 0, ldo = 0;
   float scale = 0.125f;
   int elem = ELEM_BF16;
 };
 void attn_fallback_launch(const FallbackArgs& a, hipStream_t st);
+// Appends the work tiles of entries `far` to out: {e0, e1, A0, A1, B0, B1, 0, 0} = up to 32 entries
+// [e0, e1) of one row (row r has entries [row_far[r], row_far[r + 1])) and the unions of their key
+// ranges (0, 0 where all are empty).
+void attn_far_tiles(const std::vector<int>& far, const int* row_far, int n, std::vector<int>& out);
 // The query step that cuts a row of len tokens into tiles of at most qb queries: as many tiles
 // as qb needs, of even sizes rounded up to whole waves (570 tokens at 256: 192, 192, 186), so a
 // row's last tile is not a nearly idle workgroup beside full ones.

@@ -632,8 +632,9 @@ Plan Model::plan_padded(uint32_t n, uint32_t len, const uint32_t* ids, const uin
   const long dense_upto = set.dense_upto >= 0 ? set.dense_upto : 4L * W;
   const bool banded = set.band > 0 && set.fuserope && !set.bool_mask && len >= set.band;
   const bool chunked = banded || (set.windowed && long(len) > dense_upto);
-  std::vector<int> kend(n), lqend(n), far;
+  std::vector<int> kend(n), lqend(n), far, row_far(n + 1);
   for (uint32_t r = 0; r < n; ++r) {
+    row_far[r] = int(far.size() / 8);
     const int rs = p.row_start[r], L = int(seq_lens[r]), ln = int(len);
     kend[r] = rs + L;
     lqend[r] = rs + (set.bool_mask ? L : std::min(ln, L + W));
@@ -669,7 +670,10 @@ Plan Model::plan_padded(uint32_t n, uint32_t len, const uint32_t* ids, const uin
   p.nltiles = int(m.size() - p.off_ltiles) / 4;
   p.off_far = m.size();
   m.insert(m.end(), far.begin(), far.end());
-  p.nfar = int(far.size() / 8);
+  p.nfar = row_far[n] = int(far.size() / 8);
+  p.off_ftiles = m.size();
+  attn_far_tiles(far, row_far.data(), int(n), m);
+  p.nftiles = int(m.size() - p.off_ftiles) / 8;
   p.off_scorer = p.off_pooled = m.size();
   return p;
 }
@@ -937,7 +941,8 @@ int Model::run_encoder(const Plan& p, const Acts& a, bool fold_last) {
         fa.v = a.v;
         fa.out = a.att;
         fa.far = dmeta + p.off_far;
-        fa.nfar = p.nfar;
+        fa.tiles = dmeta + p.off_ftiles;
+        fa.ntiles = p.nftiles;
         fa.heads = H;
         fa.T = T;
         fa.ldv = vt_ld(T);
@@ -1002,7 +1007,7 @@ void Model::run(const Plan& p, int kind, F&& enqueue) {
   std::vector<int64_t> key = {kind, p.T, p.n, p.kmax, p.gq, p.lq, p.ntiles, p.nltiles, p.nptiles, p.P, p.R, int64_t(p.off_ltiles),
                               int64_t(p.off_ids), int64_t(p.off_pos), int64_t(p.off_seg), int64_t(p.off_tiles),
                               int64_t(p.off_ptiles), int64_t(p.off_picked), int64_t(p.off_scorer),
-                              int64_t(p.off_pooled), int64_t(p.off_far), p.nfar, int64_t(p.padded),
+                              int64_t(p.off_pooled), int64_t(p.off_far), p.nfar, p.nftiles, int64_t(p.padded),
                               int64_t(reinterpret_cast<intptr_t>(amem)),
                               int64_t(reinterpret_cast<intptr_t>(dmeta))};
   ++graph_clock;

@@ -104,10 +104,11 @@ struct Plan {
   // The padded layout (encoder_hidden): every one of the n * len positions is a row of the
   // forward (T = n * len). The local-attention tiles take the real tokens and the padding
   // queries whose keys are the real keys of their window; the other padding queries of local
-  // layers are listed at off_far with their key sets (attn_fallback_launch's entries).
+  // layers are listed at off_far with their key sets (attn_fallback_launch's entries) and at
+  // off_ftiles as its work tiles.
   bool padded = false;
-  size_t off_far = 0;
-  int nfar = 0;
+  size_t off_far = 0, off_ftiles = 0;
+  int nfar = 0, nftiles = 0;
 };
 
 struct Model {

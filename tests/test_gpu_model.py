@@ -110,6 +110,33 @@ def test_encoder_hidden_padding_positions(small_model, settings):
     m.close()
 
 
+@pytest.mark.parametrize("settings", ["", "mask=bool,dense_upto=0", "band=1,fuserope,dtype=f16"])
+def test_encoder_hidden_far_padding_tiles(small_model, settings):
+    """Far padding queries around the edges of their 32-query tiles: rows with 0, 1, 31, 32, 33 and
+    all but one of their positions past the last real token's window, under dense, gathered and
+    zero-slot key sets. The weights are f32, so only the 16-bit layers around them differ from
+    the oracle, as everywhere."""
+    cfg, agent, st, _, _ = small_model
+    W = cfg["local_attention"] // 2
+    L = 3 * 32 + W + 1
+    lens = [L - W - f for f in (0, 1, 31, 32, 33)] + [1]
+    rng = np.random.default_rng(17)
+    ids = rng.integers(5, 1000, size=(len(lens), L)).astype(np.uint32)
+    am = np.zeros((len(lens), L), np.uint32)
+    for r, l in enumerate(lens):
+        am[r, :l] = 1
+        ids[r, l:] = 1002
+    b = Batch(len(lens), L, 0, ids.reshape(-1), am.reshape(-1), np.array(lens, np.uint64), np.zeros(0, np.uint32),
+              np.zeros(len(lens), np.uint64), np.zeros(len(lens), np.uint32))
+    m = HipBackend(st, json.dumps(cfg), json.dumps(agent), settings=settings)
+    say(f"far padding {settings!r}: n={b.n} len={b.len}")
+    ref = O.Oracle(st, cfg, agent, settings=settings).encoder_hidden(b)
+    rel = hidden_rel(m.encoder_hidden(b).reshape(b.n, b.len, -1), ref, b, padding=True)
+    say(f"far padding {settings!r}: hidden rel at every position {rel:.2e}")
+    assert rel <= HIDDEN_REL_GATE, (settings, rel)
+    m.close()
+
+
 @pytest.mark.parametrize("head_layers", [0, 1])
 def test_decision_head_depths(small_model, head_layers):
     """Agents with no decision-head layer (the scorer reads the encoder's stream, which headprune
