@@ -66,6 +66,34 @@ struct F16 {
   }
 };
 
+// A split f32 value: hi + lo / 2048, two f16 (hi the value rounded, lo what that leaves, scaled up so
+// that it keeps its bits below the smallest hi): 2^-24 relative, as f32 itself, for values down to
+// 2^-28 of f16's largest. Operands of the f32 products are held so, times a power of two that keeps
+// them in range; a row keeps its bytes, [32 hi | 32 lo] for every 32 elements: element e of a
+// matrix (rows a multiple of 32) has hi at 16-bit index split_at(e) and lo 32 after it.
+__host__ __device__ inline size_t split_at(size_t e) { return (e & ~size_t(31)) * 2 + (e & 31); }
+template <int N>  // N consecutive values (a multiple of 2), scaled by sc
+__device__ __forceinline__ void split_f16(const float* v, float sc, uint32_t* hi, uint32_t* lo) {
+#pragma unroll
+  for (int i = 0; i < N / 2; ++i) {
+    float x[2], r[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) x[e] = v[2 * i + e] * sc;
+    hi[i] = F16::pack2(x[0], x[1]);
+#pragma unroll
+    for (int e = 0; e < 2; ++e) r[e] = (x[e] - F16::f32(uint16_t(e ? hi[i] >> 16 : hi[i]))) * 2048.0f;
+    lo[i] = F16::pack2(r[0], r[1]);
+  }
+}
+// Four values at element e (a multiple of 4) of a split matrix.
+__device__ __forceinline__ void store4_split(void* m, size_t e, const float* v, float sc) {
+  uint32_t hi[2], lo[2];
+  split_f16<4>(v, sc, hi, lo);
+  uint16_t* o = static_cast<uint16_t*>(m) + split_at(e);
+  *reinterpret_cast<uint2*>(o) = make_uint2(hi[0], hi[1]);
+  *reinterpret_cast<uint2*>(o + 32) = make_uint2(lo[0], lo[1]);
+}
+
 // 8 elements of type E held in a uint4 <-> floats.
 template <class E>
 __device__ __forceinline__ void unpack8(const uint4& v, float* f) {

@@ -24,12 +24,19 @@ __device__ __forceinline__ void store8f(float* p, const float* f) {
   reinterpret_cast<float4*>(p)[1] = make_float4(f[4], f[5], f[6], f[7]);
 }
 
-// 8 results at element o of y: 16-bit of type E, or f32 where E is F32.
-struct F32;
+// 8 results at element o of y: 16-bit of type E, or split f32 times sc where E is Split.
+struct Split;
 template <class E>
-__device__ __forceinline__ void store8(void* y, size_t o, const float* f) {
-  if constexpr (std::is_same<E, F32>::value) store8f(static_cast<float*>(y) + o, f);
-  else *reinterpret_cast<uint4*>(static_cast<uint16_t*>(y) + o) = pack8<E>(f);
+__device__ __forceinline__ void store8(void* y, size_t o, const float* f, float sc) {
+  if constexpr (std::is_same<E, Split>::value) {
+    uint32_t hi[4], lo[4];
+    split_f16<8>(f, sc, hi, lo);
+    uint16_t* p = static_cast<uint16_t*>(y) + split_at(o);
+    *reinterpret_cast<uint4*>(p) = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+    *reinterpret_cast<uint4*>(p + 32) = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+  } else {
+    *reinterpret_cast<uint4*>(static_cast<uint16_t*>(y) + o) = pack8<E>(f);
+  }
 }
 
 // A hidden-state row of d floats is owned by one wavefront: lane l holds elements
@@ -111,9 +118,9 @@ __global__ __launch_bounds__(256) void embed_ln_kernel(const uint16_t* __restric
 template <class E, int NC>
 __global__ __launch_bounds__(256) void layernorm_kernel(const float* __restrict__ x, const int* __restrict__ rows,
                                                        const float* __restrict__ w, const float* __restrict__ b,
-                                                       float eps, int T, int d, uint16_t* __restrict__ yb,
+                                                       float eps, int T, int d, void* __restrict__ yb,
                                                        float* __restrict__ yf, const float* __restrict__ addv,
-                                                       const int* __restrict__ seg, float* __restrict__ yplus) {
+                                                       const int* __restrict__ seg, float* __restrict__ yplus, float ys) {
   const int row = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (row >= T) return;
@@ -141,7 +148,7 @@ __global__ __launch_bounds__(256) void layernorm_kernel(const float* __restrict_
     float y[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) y[e] = (v[c * 8 + e] - mean) * rstd * wv[c * 8 + e] + bv[c * 8 + e];
-    if (yb) *reinterpret_cast<uint4*>(yb + size_t(row) * d + o) = pack8<E>(y);
+    if (yb) store8<E>(yb, size_t(row) * d + o, y, ys);
     if (yf) store8f(yf + size_t(row) * d + o, y);
     if (yplus) {
       float z[8];
@@ -164,7 +171,7 @@ __global__ __launch_bounds__(256) void splitk_resid_ln_kernel(const float* __res
                                                              const float* __restrict__ w, float eps, int T, int d,
                                                              void* __restrict__ y, const float* __restrict__ lnb,
                                                              const float* __restrict__ hsrc,
-                                                             const int* __restrict__ hrows) {
+                                                             const int* __restrict__ hrows, float ys) {
   constexpr int PL = 8 * NC;
   const int row = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
@@ -229,7 +236,7 @@ __global__ __launch_bounds__(256) void splitk_resid_ln_kernel(const float* __res
     float o[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) o[e] = (v[c * 8 + e] - mean) * rstd * wv[c * 8 + e] + bv[c * 8 + e];
-    store8<E>(y, size_t(row) * d + c * 512 + lane * 8, o);
+    store8<E>(y, size_t(row) * d + c * 512 + lane * 8, o, ys);
   }
 }
 
@@ -557,47 +564,45 @@ void embed_ln_launch(const uint16_t* tok_emb, const int* ids, const float* w, fl
 }
 
 template <class E>
-void layernorm_t(const float* x, const int* rows, const float* w, const float* b, float eps, int T, int d,
-                 uint16_t* y_bf16, float* y_f32, const float* add_rowvec, const int* seg, float* y_plus, hipStream_t st) {
+void layernorm_t(const float* x, const int* rows, const float* w, const float* b, float eps, int T, int d, void* y,
+                 float* y_f32, const float* add_rowvec, const int* seg, float* y_plus, hipStream_t st, float ys) {
   const int rw = row_waves(T);
   dim3 grid((T + rw - 1) / rw), block(64 * rw);
-#define S1_CALL(NC)                                                                                                   \
-  hipLaunchKernelGGL((layernorm_kernel<E, NC>), grid, block, 0, st, x, rows, w, b, eps, T, d, y_bf16, y_f32, add_rowvec, \
-                     seg, y_plus)
+#define S1_CALL(NC)                                                                                              \
+  hipLaunchKernelGGL((layernorm_kernel<E, NC>), grid, block, 0, st, x, rows, w, b, eps, T, d, y, y_f32, add_rowvec, \
+                     seg, y_plus, ys)
   S1_ROWS_BY_NC(d, S1_CALL)
 #undef S1_CALL
 }
 
-void layernorm_launch(const float* x, const int* rows, const float* w, const float* b, float eps, int T, int d,
-                      uint16_t* y_bf16, float* y_f32, const float* add_rowvec, const int* seg, float* y_plus,
-                      hipStream_t st, int elem) {
+void layernorm_launch(const float* x, const int* rows, const float* w, const float* b, float eps, int T, int d, void* y,
+                      float* y_f32, const float* add_rowvec, const int* seg, float* y_plus, hipStream_t st, int elem,
+                      float ys) {
   if (T <= 0) return;
-  if (elem == ELEM_F16) layernorm_t<F16>(x, rows, w, b, eps, T, d, y_bf16, y_f32, add_rowvec, seg, y_plus, st);
-  else layernorm_t<Bf16>(x, rows, w, b, eps, T, d, y_bf16, y_f32, add_rowvec, seg, y_plus, st);
+  if (elem == ELEM_F32) layernorm_t<Split>(x, rows, w, b, eps, T, d, y, y_f32, add_rowvec, seg, y_plus, st, ys);
+  else if (elem == ELEM_F16) layernorm_t<F16>(x, rows, w, b, eps, T, d, y, y_f32, add_rowvec, seg, y_plus, st, ys);
+  else layernorm_t<Bf16>(x, rows, w, b, eps, T, d, y, y_f32, add_rowvec, seg, y_plus, st, ys);
 }
 
 template <class E>
 void splitk_resid_ln_t(const float* ws, int splits, const float* bias, float* h, const float* w, float eps, int T, int d,
-                       void* y, hipStream_t st, const float* lnb, const float* hsrc, const int* hrows) {
+                       void* y, hipStream_t st, const float* lnb, const float* hsrc, const int* hrows, float ys) {
   const int rw = row_waves(T);
   dim3 grid((T + rw - 1) / rw), block(64 * rw);
 #define S1_CALL(NC)                                                                                                \
   hipLaunchKernelGGL((splitk_resid_ln_kernel<E, NC>), grid, block, 0, st, ws, splits, bias, h, w, eps, T, d, y, lnb, \
-                     hsrc, hrows)
+                     hsrc, hrows, ys)
   S1_ROWS_BY_NC(d, S1_CALL)
 #undef S1_CALL
 }
 
 void splitk_resid_ln_launch(const float* ws, int splits, const float* bias, float* h, const float* w, float eps, int T,
                             int d, void* y, hipStream_t st, int elem, const float* lnb, const float* hsrc,
-                            const int* hrows) {
+                            const int* hrows, float ys) {
   if (T <= 0) return;
-  if (elem == ELEM_F32) {
-    splitk_resid_ln_t<F32>(ws, splits, bias, h, w, eps, T, d, y, st, lnb, hsrc, hrows);
-    return;
-  }
-  if (elem == ELEM_F16) splitk_resid_ln_t<F16>(ws, splits, bias, h, w, eps, T, d, y, st, lnb, hsrc, hrows);
-  else splitk_resid_ln_t<Bf16>(ws, splits, bias, h, w, eps, T, d, y, st, lnb, hsrc, hrows);
+  if (elem == ELEM_F32) splitk_resid_ln_t<Split>(ws, splits, bias, h, w, eps, T, d, y, st, lnb, hsrc, hrows, ys);
+  else if (elem == ELEM_F16) splitk_resid_ln_t<F16>(ws, splits, bias, h, w, eps, T, d, y, st, lnb, hsrc, hrows, ys);
+  else splitk_resid_ln_t<Bf16>(ws, splits, bias, h, w, eps, T, d, y, st, lnb, hsrc, hrows, ys);
 }
 
 template <class E>

@@ -1,7 +1,7 @@
 // Kernels of the dtype=f32 path: the reference's BackendOptions::f32 (f32 weights and compute,
 // runtime/crates/laya-core/src/backend.rs:25-27; laya-mlx/tests/parity.rs:54-65 checks it). Plain
-// f32 arithmetic throughout: f32 matrix instructions for the products, an exact erf GELU, f32
-// softmax.
+// f32 arithmetic throughout: products of operands split into two f16 with f32 sums, f32 matrix
+// instructions for attention, an exact erf GELU, f32 softmax.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -19,17 +19,21 @@ __device__ __forceinline__ float act32(float v, int act) {
   return act == ACT_RELU ? fmaxf(v, 0.0f) : act == ACT_GELU ? gelu_exact(v) : v;
 }
 
-// C[M, N] = A[M, K] . W[N, K]^T on v_mfma_f32_32x32x2_f32 (64 FLOP per clock and SIMD: the unit
-// that bounds these products). BM x BN tiles in WM x WN waves, 32-float k-tiles (128-byte rows)
-// moved global -> LDS by direct loads, STAGES deep, one barrier per k-tile; 16-byte chunk c of row
-// r sits at slot c ^ ((r / 2) % 8), so the 16 rows of one fragment read phase start in 16 distinct
-// bank groups.
+// C[M, N] = A[M, K] . W[N, K]^T of split operands: hi hi + (hi lo + lo hi) / 2048 on
+// v_mfma_f32_32x32x16_f16, each product exact and summed in f32, the two orders of magnitude in
+// accumulators of their own. Three 16-deep instructions take 96 clocks of a SIMD where the f32 matrix
+// instruction takes 512; what bounds these products is the power that they draw (the same launch on
+// zeros runs 1.4 times as fast). Against v_mfma_f32_32x32x2_f32 on the same tiles, M 5707:
+// N 3072, K 1024 330 -> 119 us (302 TFLOP/s); 1024, 1024 112 -> 39; 5248, 1024 524 -> 224; 1024, 2624
+// 279 -> 92; 4096, 1024 417 -> 168; 1024, 4096 425 -> 149, and the error against float64 from 5.7e-7 to
+// 2.2e-7 at K 1024, 1.2e-6 to 4.3e-7 at 4096 (fewer roundings of the sum). Splitting into three bf16
+// and six products: 239 us for the first of them.
 //
-// A k-step is 8 floats: lane (row l % 32, h = l / 32) reads 4 consecutive floats (chunk 2 ks + h)
-// of its row with one access, and MFMA u of the step multiplies element u, i.e. k = 8 ks + u from
-// the lanes of half 0 and k = 8 ks + 4 + u from half 1: both operands use the same order, so each
-// k is met once. W is the first operand (C^T = W . A^T): a lane holds 4 consecutive columns of one
-// row and stores them as one float4.
+// BM x BN tiles in WM x WN waves, 32-deep k-tiles (128-byte rows, [32 hi | 32 lo]) moved global -> LDS
+// by direct loads, STAGES deep, one barrier per k-tile; 16-byte chunk c of row r sits at slot
+// c ^ ((r / 2) % 8), so the 16 rows of one fragment read phase start in 16 distinct bank groups. W is
+// the first operand (C^T = W . A^T): a lane holds 4 consecutive columns of one row and stores them as
+// one float4.
 template <int BM, int BN, int WM, int WN, int STAGES>
 __global__ __launch_bounds__(WM * WN * 64) void gemm32_kernel(Gemm32Args g) {
   constexpr int NW = WM * WN, TM = BM / WM, TN = BN / WN, FM = TM / 32, FN = TN / 32;
@@ -71,54 +75,62 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm32_kernel(Gemm32Args g) {
   }
   const i32x4 rsrcA = buffer_rsrc(g.A + size_t(m0) * g.lda, uint32_t((size_t(min(BM - 1, mlast)) * g.lda + g.K) * 4));
   const i32x4 rsrcW = buffer_rsrc(g.W + size_t(n0) * g.ldw, uint32_t((size_t(BN - 1) * g.ldw + g.K) * 4));
-  auto issue = [&](int stage, int kt) __attribute__((always_inline)) {
+  auto issue = [&](int stage, int kt, int jlo, int jhi) __attribute__((always_inline)) {  // this wave's loads [jlo, jhi)
     const int koff = __builtin_amdgcn_readfirstlane(kt * ROWB);
     char* sb = smem + stage * STAGE_BYTES + wave * 1024;
 #pragma unroll
-    for (int j = 0; j < LPW; ++j) load16_lds(j < AG / NW ? rsrcA : rsrcW, sb + j * NW * 1024, int(voff[j]), koff);
+    for (int j = 0; j < LPW; ++j)
+      if (j >= jlo && j < jhi) load16_lds(j < AG / NW ? rsrcA : rsrcW, sb + j * NW * 1024, int(voff[j]), koff);
   };
 
-  f32x16 acc[FM][FN];
+  f32x16 acc[FM][FN], acx[FM][FN];
 #pragma unroll
   for (int i = 0; i < FM; ++i)
 #pragma unroll
     for (int j = 0; j < FN; ++j)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = acx[i][j][e] = 0.0f;
 
 #pragma unroll
   for (int s = 0; s < STAGES - 1; ++s)
-    if (s < NK) issue(s, kt0 + s);
+    if (s < NK) issue(s, kt0 + s, 0, LPW);
   const int lr = lane & 31, lh = lane >> 5;
-  int ka[4];
+  int ka[4];  // fragments of k-steps 0 and 1: hi, then lo
 #pragma unroll
-  for (int ks = 0; ks < 4; ++ks) ka[ks] = lr * ROWB + (((ks * 2 + lh) ^ ((lr >> 1) & 7)) << 4);
+  for (int c = 0; c < 4; ++c) ka[c] = lr * ROWB + (((c * 2 + lh) ^ ((lr >> 1) & 7)) << 4);
   for (int it = 0; it < NK; ++it) {
     wait_ahead<LPW, STAGES - 2>(min(STAGES - 2, NK - 1 - it));
     // Every wave's loads of k-tile `it` have landed and every wave is done with k-tile it - 1,
     // whose buffer the next issue overwrites.
     barrier_lds();
-    if (it + STAGES - 1 < NK) issue((it + STAGES - 1) % STAGES, kt0 + it + STAGES - 1);
+    const bool pre = it + STAGES - 1 < NK;
     const char* sa = smem + (it % STAGES) * STAGE_BYTES + wm * TM * ROWB;
     const char* sw = smem + (it % STAGES) * STAGE_BYTES + A_BYTES + wn * TN * ROWB;
-    f32x4 fa[2][FM], fb[2][FN];
-    auto frag = [&](int ks, int buf) __attribute__((always_inline)) {
+    typedef typename F16::v8 v8;
+    v8 fa[2][2][FM], fb[2][2][FN];
+    auto frag = [&](int s) __attribute__((always_inline)) {
 #pragma unroll
-      for (int i = 0; i < FM; ++i) fa[buf][i] = *reinterpret_cast<const f32x4*>(sa + ka[ks] + i * 32 * ROWB);
+      for (int p = 0; p < 2; ++p) {
 #pragma unroll
-      for (int j = 0; j < FN; ++j) fb[buf][j] = *reinterpret_cast<const f32x4*>(sw + ka[ks] + j * 32 * ROWB);
+        for (int i = 0; i < FM; ++i) fa[s][p][i] = *reinterpret_cast<const v8*>(sa + ka[2 * p + s] + i * 32 * ROWB);
+#pragma unroll
+        for (int j = 0; j < FN; ++j) fb[s][p][j] = *reinterpret_cast<const v8*>(sw + ka[2 * p + s] + j * 32 * ROWB);
+      }
     };
-    frag(0, 0);
+    frag(0);
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      if (ks < 3) frag(ks + 1, (ks + 1) & 1);
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
+    for (int s = 0; s < 2; ++s) {
+      if (pre) issue((it + STAGES - 1) % STAGES, kt0 + it + STAGES - 1, s * LPW / 2, (s + 1) * LPW / 2);
+      if (s == 0) frag(1);
+      auto mm = [&](int pw, int pa, f32x16 (&c)[FM][FN]) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < FM; ++i)
 #pragma unroll
-          for (int j = 0; j < FN; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[ks & 1][j][u], fa[ks & 1][i][u], acc[i][j], 0, 0, 0);
+          for (int j = 0; j < FN; ++j) c[i][j] = F16::mfma(fb[s][pw][j], fa[s][pa][i], c[i][j]);
+      };
+      mm(0, 0, acc);
+      mm(1, 0, acx);
+      mm(0, 1, acx);
     }
   }
 
@@ -138,7 +150,11 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm32_kernel(Gemm32Args g) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         float4* o = reinterpret_cast<float4*>(orow + j * 32 + q * 8);
-        float v[4] = {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+        const float4 inv = *reinterpret_cast<const float4*>(g.inv + n0 + wn * TN + 4 * lh + j * 32 + q * 8);
+        const float iv[4] = {inv.x, inv.y, inv.z, inv.w};
+        float v[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = fmaf(acx[i][j][4 * q + r], 1.0f / 2048.0f, acc[i][j][4 * q + r]) * iv[r];
         if (!part) {
           if (g.bias) {
             const float4 b = *reinterpret_cast<const float4*>(g.bias + n0 + wn * TN + 4 * lh + j * 32 + q * 8);
@@ -155,6 +171,10 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm32_kernel(Gemm32Args g) {
             v[1] += c.y;
             v[2] += c.z;
             v[3] += c.w;
+          }
+          if (g.cs > 0.0f) {
+            store4_split(g.C, size_t(row) * ld + n0 + wn * TN + 4 * lh + j * 32 + q * 8, v, g.cs);
+            continue;
           }
         }
         *o = make_float4(v[0], v[1], v[2], v[3]);
@@ -186,8 +206,52 @@ __global__ __launch_bounds__(256) void splitk32_kernel(Gemm32Args g) {
   const float4 b = g.bias ? *reinterpret_cast<const float4*>(g.bias + c) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   float4* o = reinterpret_cast<float4*>(g.C + size_t(row) * g.ldc + c);
   const float4 old = g.accumulate ? *o : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  *o = make_float4(old.x + act32(s.x + b.x, g.act), old.y + act32(s.y + b.y, g.act), old.z + act32(s.z + b.z, g.act),
-                   old.w + act32(s.w + b.w, g.act));
+  const float v[4] = {old.x + act32(s.x + b.x, g.act), old.y + act32(s.y + b.y, g.act), old.z + act32(s.z + b.z, g.act),
+                      old.w + act32(s.w + b.w, g.act)};
+  if (g.cs > 0.0f) store4_split(g.C, size_t(row) * g.ldc + c, v, g.cs);
+  else *o = make_float4(v[0], v[1], v[2], v[3]);
+}
+
+// A weight matrix into split f32 in place, each row times the power of two that puts its largest
+// element (bounds[2 row]) at 2^14 to 2^15: a wave reads its 64 elements of one row, then writes their
+// bytes. inv[row] undoes the row's scale and the input's.
+__global__ __launch_bounds__(256) void split_weight_kernel(float* w, size_t n, int K, const float* __restrict__ bounds,
+                                                           float a, float* __restrict__ inv) {
+  const size_t e = size_t(blockIdx.x) * 256 + threadIdx.x;
+  if (e >= n) return;
+  const size_t row = e / K;
+  const float m = bounds[2 * row];
+  int ex = 0;
+  if (m > 0.0f && m < __builtin_huge_valf()) (void)frexpf(m, &ex);
+  const float sc = ldexpf(1.0f, 15 - min(max(ex, -40), 60));  // products of two scales stay normal
+  if (e % K == 0) inv[row] = 1.0f / (sc * a);
+  const float x[2] = {w[e], 0.0f};
+  uint32_t hi, lo;
+  split_f16<2>(x, sc, &hi, &lo);
+  uint16_t* o = reinterpret_cast<uint16_t*>(w) + split_at(e);
+  o[0] = uint16_t(hi);
+  o[32] = uint16_t(lo);
+}
+
+// One wave per row of W (weight_bound_launch): |W_r . (z * lw + lb) + bias| <= sqrt(K) |W_r * lw|_2 +
+// |W_r . lb + bias| by the Cauchy-Schwarz inequality.
+__global__ __launch_bounds__(64) void weight_bound_kernel(const float* __restrict__ W, const float* __restrict__ lw,
+                                                          const float* __restrict__ lb, const float* __restrict__ bias, int K,
+                                                          float* __restrict__ out) {
+  const float* row = W + size_t(blockIdx.x) * K;
+  float mx = 0.0f, sq = 0.0f, dot = 0.0f;
+  for (int k = threadIdx.x; k < K; k += 64) {
+    const float w = row[k], x = lw ? w * lw[k] : w;
+    mx = fmaxf(mx, fabsf(w));
+    sq = fmaf(x, x, sq);
+    if (lb) dot = fmaf(w, lb[k], dot);
+  }
+  mx = wave_max(mx);
+  sq = wave_sum(sq);
+  dot = wave_sum(dot);
+  if (threadIdx.x) return;
+  out[2 * blockIdx.x] = mx;
+  out[2 * blockIdx.x + 1] = sqrtf(float(K)) * sqrtf(sq) + fabsf(dot + (bias ? bias[blockIdx.x] : 0.0f));
 }
 
 // qkv [T, 3d] -> q, k, v [H, T, 64], with the half-split RoPE rotation of q and k at pos[t] when
@@ -376,7 +440,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
   }
   if (!active || qi >= tl.q1) return;
   const float inv = 1.0f / L;
-  float* orow = a.out + size_t(qi) * a.ldo + head * 64 + hl * 4;
+  const size_t oe = size_t(qi) * a.ldo + head * 64 + hl * 4;
 #pragma unroll
   for (int dt = 0; dt < 2; ++dt)
 #pragma unroll
@@ -393,7 +457,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
         }
         r4[r] = acc * inv;
       }
-      *reinterpret_cast<float4*>(orow + dt * 32 + g * 8) = make_float4(r4[0], r4[1], r4[2], r4[3]);
+      store4_split(a.out, oe + dt * 32 + g * 8, r4, a.os);
     }
 }
 
@@ -454,12 +518,17 @@ __global__ __launch_bounds__(64) void attn32_kernel(Attn32Args a) {
     l = l * alpha + expf(sz - mn);
     o *= alpha;
   }
-  a.out[size_t(qrow) * a.ldo + head * 64 + lane] = o / l;
+  const float r[2] = {o / l, 0.0f};
+  uint32_t h16, l16;
+  split_f16<2>(r, a.os, &h16, &l16);
+  uint16_t* out = reinterpret_cast<uint16_t*>(a.out) + split_at(size_t(qrow) * a.ldo + head * 64 + lane);
+  out[0] = uint16_t(h16);
+  out[32] = uint16_t(l16);
 }
 
 // act[t, i] = gelu(x[t, i]) * x[t, I + i] over x [T, 2I], whole or the parts of a split product.
 __global__ __launch_bounds__(256) void geglu32_kernel(const float* __restrict__ x, int splits, int T, int I,
-                                                      float* __restrict__ act) {
+                                                      float* __restrict__ act, float as) {
   const long long gid = (long long)blockIdx.x * 256 + threadIdx.x;
   const int n4 = I / 4;
   if (gid >= (long long)T * n4) return;
@@ -467,8 +536,8 @@ __global__ __launch_bounds__(256) void geglu32_kernel(const float* __restrict__ 
   const float* row = x + size_t(t) * 2 * I + i;
   const size_t plane = size_t(T) * 2 * I;
   const float4 a = sum_parts(row, splits, plane), g = sum_parts(row + I, splits, plane);
-  *reinterpret_cast<float4*>(act + size_t(t) * I + i) =
-      make_float4(gelu_exact(a.x) * g.x, gelu_exact(a.y) * g.y, gelu_exact(a.z) * g.z, gelu_exact(a.w) * g.w);
+  const float v[4] = {gelu_exact(a.x) * g.x, gelu_exact(a.y) * g.y, gelu_exact(a.z) * g.z, gelu_exact(a.w) * g.w};
+  store4_split(act, size_t(t) * I + i, v, as);
 }
 
 // out[r] = dot(x[r], w) + b over rows of K floats, one wave per row.
@@ -490,23 +559,20 @@ void gemm32_t(const Gemm32Args& g, hipStream_t st) {
   hipLaunchKernelGGL((gemm32_kernel<BM, BN, WM, WN, STAGES>), grid, dim3(WM * WN * 64), 0, st, g);
 }
 
-// Tiles by rows and columns: 64 x 128 once there are two for every CU, else 64 x 64, or 32 x 128
-// where those leave fewer rows idle by a tenth of the product or more (193 rows: 224 instead of
-// 256). At 5707 rows the 64 x 128 tiles in two stages (48 KiB, three workgroups per CU) run the
-// five products of a layer and the head at 128-131 TFLOP/s, 64 x 64 ones at 125, and larger
-// tiles, three or four stages, or the next fragments read across the barrier less: what counts is
-// waves per SIMD to issue matrix instructions while others wait.
-bool rows32(int M) { return ((M + 31) / 32) * 32 * 11 <= ((M + 63) / 64) * 64 * 10; }
+// 64 x 128 tiles in two stages (48 KiB, three workgroups per CU) once there are two for every CU, else
+// 64 x 64 in three. At 5707 rows, q|k|v: 64 x 128 119 us, in three stages 129, 192 x 128 119, 128 x 128
+// 155, 256 x 128 in 8 waves 138. At 193 rows 32-row tiles gain at most 1 us in 10 and lose as much
+// elsewhere.
 bool wide32(int M, int N) { return (long long)((M + 63) / 64) * (N / 128) >= 512; }
 
 }  // namespace
 
 const char* gemm32_check(const Gemm32Args& g) {
   if (g.M < 0 || g.N <= 0 || g.K <= 0) return "f32 GEMM: empty shape";
-  if (g.K % 32 || g.N % 128) return "f32 GEMM: K must be a multiple of 32, N of 128";
-  if (g.lda < g.K || g.ldw < g.K || g.lda % 4 || g.ldw % 4 || g.ldc % 4) return "f32 GEMM: bad leading dimension";
+  if (g.K % 32 || g.N % 128 || g.lda % 32 || g.ldw % 32 || g.ldc % 32) return "f32 GEMM: K and leading dimensions must be multiples of 32, N of 128";
+  if (g.lda < g.K || g.ldw < g.K) return "f32 GEMM: bad leading dimension";
   if ((reinterpret_cast<uintptr_t>(g.A) | reinterpret_cast<uintptr_t>(g.W) | reinterpret_cast<uintptr_t>(g.C) |
-       reinterpret_cast<uintptr_t>(g.bias) | reinterpret_cast<uintptr_t>(g.ws)) % 16)
+       reinterpret_cast<uintptr_t>(g.bias) | reinterpret_cast<uintptr_t>(g.ws) | reinterpret_cast<uintptr_t>(g.inv)) % 16)
     return "f32 GEMM: operands must be 16-byte aligned";
   if (size_t(std::max(g.lda, g.ldw)) * 128 * 4 > 0xffffffffu) return "f32 GEMM: a tile's rows must span less than 4 GiB";
   if (g.splits < 1 || g.splits > g.K / 32) return "f32 GEMM: splits must be in 1..K/32";
@@ -516,16 +582,17 @@ const char* gemm32_check(const Gemm32Args& g) {
 
 int gemm32_splits(int M, int N, int K) {
   if (M <= 0 || wide32(M, N)) return 1;
-  const int tiles = rows32(M) ? (M + 31) / 32 * (N / 128) : (M + 63) / 64 * (N / 64);
+  const int tiles = (M + 63) / 64 * (N / 64);
   const int kt = K / 32;
-  // A tile is matrix-unit time, so a launch lasts as long as the CU with the most parts of tiles:
-  // the split that makes that least, each part at least 4 k-tiles, its start and end counted as 4
-  // more, at most 8 parts (they are written and read back). At 193 rows of width 1024, against no
-  // split: q|k|v 26 -> 18 us (3 parts), Wo 25 -> 9.4 (4), Wi 39 -> 30 (3), Wo2 57 -> 18 (4).
+  // Three workgroups of 64 x 64 tiles share a CU, and a launch lasts as long as the CU with the most
+  // parts of tiles: the split that makes that least, each part at least 4 k-tiles, its start and end
+  // counted as 4 more, at most 8 parts, each counted as one k-tile where they are read back. At 193
+  // rows of width 1024, against no split: q|k|v 14.0 -> 10.2 us (4 parts), Wo 10.2 -> 5.5 (4), Wo2 20.2 -> 9.0 (8);
+  // Wi, 328 tiles, takes two rounds either way.
   int best = 1;
   long long least = 0;
   for (int s = 1; s <= 8 && s <= kt / 4; ++s) {
-    const long long t = (long long)((tiles * s + 255) / 256) * ((kt + s - 1) / s + 4) + 2 * (s > 1);
+    const long long t = (long long)((tiles * s + 767) / 768) * ((kt + s - 1) / s + 4) + s;
     if (s == 1 || t < least) {
       best = s;
       least = t;
@@ -537,8 +604,7 @@ int gemm32_splits(int M, int N, int K) {
 void gemm32_launch(const Gemm32Args& g, hipStream_t st) {
   if (g.M <= 0) return;
   if (wide32(g.M, g.N)) gemm32_t<64, 128, 2, 2, 2>(g, st);
-  else if (rows32(g.M)) gemm32_t<32, 128, 1, 4, 2>(g, st);
-  else gemm32_t<64, 64, 2, 2, 2>(g, st);
+  else gemm32_t<64, 64, 2, 2, 3>(g, st);
   if (g.splits > 1 && g.C) {
     const long long n = (long long)g.M * (g.N / 4);
     hipLaunchKernelGGL(splitk32_kernel, dim3(unsigned((n + 255) / 256)), dim3(256), 0, st, g);
@@ -586,10 +652,20 @@ void attn32_launch(const Attn32Args& a, hipStream_t st) {
   else hipLaunchKernelGGL(attn32_tile_kernel<4>, grid, dim3(256), 0, st, a);
 }
 
-void geglu32_launch(const float* x, int splits, int T, int I, float* act, hipStream_t st) {
+void split_weight_launch(float* W, int N, int K, const float* bounds, float a, float* inv, hipStream_t st) {
+  const size_t n = size_t(N) * K;
+  hipLaunchKernelGGL(split_weight_kernel, dim3(unsigned((n + 255) / 256)), dim3(256), 0, st, W, n, K, bounds, a, inv);
+}
+
+void weight_bound_launch(const float* W, const float* lw, const float* lb, const float* bias, int N, int K, float* out,
+                         hipStream_t st) {
+  hipLaunchKernelGGL(weight_bound_kernel, dim3(unsigned(N)), dim3(64), 0, st, W, lw, lb, bias, K, out);
+}
+
+void geglu32_launch(const float* x, int splits, int T, int I, float* act, float as, hipStream_t st) {
   const long long n = (long long)T * (I / 4);
   if (n <= 0) return;
-  hipLaunchKernelGGL(geglu32_kernel, dim3(unsigned((n + 255) / 256)), dim3(256), 0, st, x, splits, T, I, act);
+  hipLaunchKernelGGL(geglu32_kernel, dim3(unsigned((n + 255) / 256)), dim3(256), 0, st, x, splits, T, I, act, as);
 }
 
 void rowdot32_launch(const float* x, const float* w, const float* b, int R, int K, float* out, hipStream_t st) {

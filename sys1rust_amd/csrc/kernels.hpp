@@ -142,12 +142,13 @@ int attn_row_step(int len, int qb);
 void embed_ln_launch(const uint16_t* tok_emb, const int* ids, const float* w, float eps, int T, int d, float* h_out,
                      uint16_t* x_out, hipStream_t st, int elem = ELEM_BF16);
 
-// y = LN(x) (optional bias) over rows of d, x f32; y bf16 and/or f32 (null to skip). With
-// `rows` the input row of output row t is rows[t]. With `add_rowvec`, the f32 output also gets
-// add_rowvec[seg[t]] (the type embedding of the row's question), used to start the head stream.
-void layernorm_launch(const float* x, const int* rows, const float* w, const float* b, float eps, int T, int d,
-                      uint16_t* y_bf16, float* y_f32, const float* add_rowvec, const int* seg, float* y_plus,
-                      hipStream_t st, int elem = ELEM_BF16);
+// y = LN(x) (optional bias) over rows of d, x f32; y 16-bit (or, with elem = ELEM_F32, split f32
+// times ys) and/or f32 (null to skip). With `rows` the input row of output row t is rows[t]. With
+// `add_rowvec`, y_plus gets the f32 result plus add_rowvec[seg[t]] (the type embedding of the row's
+// question), used to start the head stream.
+void layernorm_launch(const float* x, const int* rows, const float* w, const float* b, float eps, int T, int d, void* y,
+                      float* y_f32, const float* add_rowvec, const int* seg, float* y_plus, hipStream_t st,
+                      int elem = ELEM_BF16, float ys = 1.0f);
 
 // The end of a split-K residual GEMM and the LayerNorm after it, one wave per row:
 // h[t] += (sum over s of ws[s, t] in split order) + bias, then y[t] = LN(h[t]) (weight w, bias
@@ -155,10 +156,10 @@ void layernorm_launch(const float* x, const int* rows, const float* w, const flo
 // ws is [splits, T, d] f32, h is [T, d] f32.
 // With hsrc, the residual of row r is row hrows[r] of hsrc (a row gather folded in); the sum
 // still goes to row r of h.
-// y is 16-bit, or f32 with elem = ELEM_F32.
+// y is 16-bit, or split f32 times ys with elem = ELEM_F32.
 void splitk_resid_ln_launch(const float* ws, int splits, const float* bias, float* h, const float* w, float eps, int T,
                             int d, void* y, hipStream_t st, int elem = ELEM_BF16, const float* lnb = nullptr,
-                            const float* hsrc = nullptr, const int* hrows = nullptr);
+                            const float* hsrc = nullptr, const int* hrows = nullptr, float ys = 1.0f);
 
 // End of the pruned decision head over its P = n per picked rows ([row 0, kmax scorer rows] per
 // request, per = 1 + kmax): h (+ the sum of `splits` f32 partials in ws [splits, P, d] and then
@@ -193,15 +194,19 @@ void gather_f32_launch(const float* x, const int* rows, int R, int d, float* out
 void rowdot_launch(const uint16_t* x, const float* w, const float* b, int R, int d, float* out, hipStream_t st,
                    int elem = ELEM_BF16);
 
-// ---- The dtype=f32 path (BackendOptions::f32): f32 weights and activations.
+// ---- The dtype=f32 path (BackendOptions::f32): f32 weights and activations. The products' operands
+// are split f32 (device.hpp's split_f16), activations times a power of two, weights a row each.
 
-// C[M, N] (+)= act(A[M, K] . W[N, K]^T + bias), all f32; accumulate adds to C (the residual).
+// C[M, N] (+)= act(A[M, K] . W[N, K]^T * inv + bias): A and W split, inv[n] = 1 / (A's scale, W row n's),
+// C f32, or with cs > 0 split times cs; accumulate adds to an f32 C (the residual).
 struct Gemm32Args {
   const float* A = nullptr;  // [M, lda]
   const float* W = nullptr;  // [N, ldw]
   float* C = nullptr;        // [M, ldc]; null: a split product whose consumer sums the parts
   const float* bias = nullptr;
   int M = 0, N = 0, K = 0, lda = 0, ldw = 0, ldc = 0;
+  const float* inv = nullptr;  // [N]
+  float cs = 0.0f;
   int act = ACT_NONE;
   bool accumulate = false;
   // Split product: `splits` workgroups share each output tile, each over a part of K, and write
@@ -209,8 +214,8 @@ struct Gemm32Args {
   int splits = 1;
   float* ws = nullptr;
 };
-// Null when the shape is supported (K a multiple of 32, N of 128, 16-byte aligned rows), else a
-// message.
+// Null when the shape is supported (K and leading dimensions multiples of 32, N of 128, aligned
+// operands), else a message.
 const char* gemm32_check(const Gemm32Args& g);
 // The split gemm32_launch should use for M x N x K (1: none).
 int gemm32_splits(int M, int N, int K);
@@ -219,7 +224,15 @@ void gemm32_launch(const Gemm32Args& g, hipStream_t st);
 // k, v [d / 64, T, 64] f32, q and k rotated at pos[t] when cos_t is given.
 void split32_launch(const float* qkv, int splits, const float* bias, int T, int d, const int* pos, const float* cos_t,
                     const float* sin_t, float* q, float* k, float* v, hipStream_t st);
-// f32 attention, q, k, v [heads, T, 64], out [slots, ldo]: over n work tiles as AttnArgs describes
+// Splits W [N, K] (K a multiple of 64) in place, each row times a power of two by its largest element
+// in `bounds` (weight_bound_launch's), and fills inv [N] for inputs that are held times a.
+void split_weight_launch(float* W, int N, int K, const float* bounds, float a, float* inv, hipStream_t st);
+// Bounds for the scales: for each row r of W [N, K] f32, out[2 r] = its largest |element| and
+// out[2 r + 1] = the most |W_r . x + bias_r| can be over all x = z * lw + lb with |z|_2 <= sqrt(K), what a
+// LayerNorm with weight lw and bias lb (or none) gives.
+void weight_bound_launch(const float* W, const float* lw, const float* lb, const float* bias, int N, int K, float* out,
+                         hipStream_t st);
+// f32 attention, q, k, v [heads, T, 64], out [slots, ldo] split f32 times os: over n work tiles as AttnArgs describes
 // them (up to tile_q slots of one row each, its key range, the window tested per query, qkey), or,
 // with `entries`, of n single queries over a key set each: entries of 8 int32 as
 // attn_fallback_launch takes them ({query, a0, a1, b0, b1, lo, hi, zeros}).
@@ -235,14 +248,16 @@ struct Attn32Args {
   int tile_q = 32;  // 128, 64 or 32
   int window = -1;
   float scale = 0.125f;
+  float os = 1.0f;
 };
 // Appends the rows' work tiles to out and returns the queries per tile (Attn32Args::tile_q); q_end
 // and k_end as attn_plan_tiles takes them.
 int attn32_plan_tiles(const int* row_start, int n, int heads, int window, std::vector<int>& out,
                       const int* q_end = nullptr, const int* k_end = nullptr);
 void attn32_launch(const Attn32Args& a, hipStream_t st);
-// act[t, i] = gelu(x[t, i]) * x[t, I + i] (exact erf) over x [T, 2I] f32, or its parts [splits, T, 2I].
-void geglu32_launch(const float* x, int splits, int T, int I, float* act, hipStream_t st);
+// act[t, i] = gelu(x[t, i]) * x[t, I + i] (exact erf), split f32 times as, over x [T, 2I] f32, or its
+// parts [splits, T, 2I].
+void geglu32_launch(const float* x, int splits, int T, int I, float* act, float as, hipStream_t st);
 // out[r] = dot(x[r], w) + b[0] over rows of K floats (K a multiple of 4).
 void rowdot32_launch(const float* x, const float* w, const float* b, int R, int K, float* out, hipStream_t st);
 

@@ -374,6 +374,8 @@ void Model::init(const SafeTensors& st, const std::string& enc_json, const std::
     hip_check(hipMemcpy(dptr, hb.data(), n * 2, hipMemcpyHostToDevice), "upload weight");
   }
 
+  if (set.f32) split_weights32();
+
   char nb[64];
   std::snprintf(nb, sizeof nb, "hip(gfx950,%s)", set.f32 ? "f32" : set.f16 ? "f16" : "bf16");
   name = nb;
@@ -403,13 +405,14 @@ void Model::teardown() {
   if (rmem) (void)hipFree(rmem);
   if (amem) (void)hipFree(amem);
   if (fmem) (void)hipFree(fmem);
+  if (imem) (void)hipFree(imem);
   if (dmeta) (void)hipFree(dmeta);
   if (hmeta) (void)hipHostFree(hmeta);
   if (hout) (void)hipHostFree(hout);
   if (stream) (void)hipStreamDestroy(stream);
   pending.clear();
   event_pool.clear();
-  wmem = rmem = amem = fmem = nullptr;
+  wmem = rmem = amem = fmem = imem = nullptr;
   dmeta = nullptr;
   hmeta = hout = nullptr;
   stream = nullptr;
@@ -1348,9 +1351,11 @@ Model::Acts32 Model::arena32(const Plan& p) {
 namespace {
 
 // C (+)= act(A . W^T + bias) on the f32 GEMM, split as planned, shapes checked.
-Gemm32Args gemm32_args(const float* A, int lda, const float* W, int ldw, float* C, int ldc, const float* bias, int M, int N,
-                       int K, int act, bool accumulate, float* ws) {
+Gemm32Args gemm32_args(const Scales32& sc, const float* A, int lda, const float* W, int ldw, float* C, int ldc,
+                       const float* bias, int M, int N, int K, int act, bool accumulate, float* ws, float cs = 0.0f) {
   Gemm32Args g;
+  g.inv = sc.inv;
+  g.cs = cs;
   g.A = A;
   g.W = W;
   g.C = C;
@@ -1377,17 +1382,82 @@ Gemm32Args parts_of(Gemm32Args g) {
 
 }  // namespace
 
+// The f32 products' scales and split weights, at load. An operand's scale is the power of two that puts
+// the most it can reach at 2^14 to 2^15 (f16 goes to 65504): a weight row's largest element, or for
+// activations a bound that holds for every input. A LayerNorm's output is z * w + b with
+// |z|_2 <= sqrt(d), so each element and each product of it with a weight row is bounded
+// (weight_bound_launch); attention returns averages of v rows; |gelu(x) g| <= |x| |g|. Operands that stay
+// far below their bound lose nothing: a split value keeps f32's precision down to 2^-27 of it.
+void Model::split_weights32() {
+  const int d = cfg.d, I = cfg.inter;
+  const size_t most = size_t(std::max({3 * d, 2 * I, 4 * d, scorer_width}));
+  const size_t rows = size_t(cfg.layers) * (5 * d + 2 * I) + size_t(cfg.head_layers) * 9 * d + scorer_width;
+  hip_check(hipMalloc(&imem, (rows + most * 2) * 4), "hipMalloc(scales)");
+  float* inv = static_cast<float*>(imem);
+  float* const db = inv + rows;  // bounds of the weight at hand
+  std::vector<float> b(most * 2), hw(d), hb(d);
+  auto pow2 = [](double bound) {
+    int e = 0;
+    if (bound > 0.0 && std::isfinite(bound)) (void)std::frexp(bound, &e);  // bound <= 2^e
+    return float(std::ldexp(1.0, 15 - std::min(std::max(e, -40), 60)));
+  };
+  // What LayerNorm (lw, lb) can give, per element.
+  auto norm = [&](const float* lw, const float* lb) {
+    hip_check(hipMemcpy(hw.data(), lw, size_t(d) * 4, hipMemcpyDeviceToHost), "read norm");
+    if (lb) hip_check(hipMemcpy(hb.data(), lb, size_t(d) * 4, hipMemcpyDeviceToHost), "read norm");
+    double m = 0.0;
+    for (int k = 0; k < d; ++k) m = std::max(m, std::sqrt(double(d)) * std::fabs(hw[k]) + (lb ? std::fabs(hb[k]) : 0.0f));
+    return m;
+  };
+  // Splits w [N, K], whose input is held times a, after reading its rows' bounds on an input of
+  // LayerNorm (lw, lb) into b.
+  auto weight = [&](uint16_t* w, int N, int K, double bound, const float* lw, const float* lb, const float* bias) {
+    Scales32 sc{pow2(bound), inv};
+    float* W = const_cast<float*>(w32(w));
+    weight_bound_launch(W, lw, lb, bias, N, K, db, stream);
+    hip_check(hipGetLastError(), "weight bounds");
+    hip_check(hipMemcpyAsync(b.data(), db, size_t(N) * 8, hipMemcpyDeviceToHost, stream), "read bounds");
+    split_weight_launch(W, N, K, db, sc.a, inv, stream);
+    hip_check(hipGetLastError(), "split weight");
+    hip_check(hipStreamSynchronize(stream), "split weight");
+    inv += N;
+    return sc;
+  };
+  auto most_of = [&](int r0, int r1) {
+    double m = 0.0;
+    for (int r = r0; r < r1; ++r) m = std::max(m, double(b[2 * r + 1]));
+    return m;
+  };
+  for (int l = 0; l < cfg.layers; ++l) {
+    LayerWeights& L = layers[l];
+    const float* n1 = l ? L.attn_norm : emb_norm;
+    L.s_qkv = weight(L.wqkv, 3 * d, d, norm(n1, nullptr), n1, nullptr, nullptr);
+    L.s_wo = weight(L.wo, d, d, most_of(2 * d, 3 * d), nullptr, nullptr, nullptr);
+    L.s_wi = weight(L.wi, 2 * I, d, norm(L.mlp_norm, nullptr), L.mlp_norm, nullptr, nullptr);
+    double m = 0.0;
+    for (int j = 0; j < I; ++j) m = std::max(m, double(b[2 * j + 1]) * b[2 * (I + j) + 1]);
+    L.s_wo2 = weight(L.wo2, d, I, m, nullptr, nullptr, nullptr);
+  }
+  for (HeadWeights& H : head) {
+    H.s_in = weight(H.in_w, 3 * d, d, norm(H.n1w, H.n1b), H.n1w, H.n1b, H.in_b);
+    H.s_out = weight(H.out_w, d, d, most_of(2 * d, 3 * d), nullptr, nullptr, nullptr);
+    H.s_l1 = weight(H.l1_w, 4 * d, d, norm(H.n2w, H.n2b), H.n2w, H.n2b, H.l1_b);
+    H.s_l2 = weight(H.l2_w, d, 4 * d, most_of(0, 4 * d), nullptr, nullptr, nullptr);
+  }
+  s_sc1 = weight(sc1_w, scorer_width, d, norm(sc0_w, sc0_b), sc0_w, sc0_b, sc1_b);
+}
+
 // A residual product g into h, then y = LN(h) (weight w, bias b) over M rows: one kernel after the
 // product when it splits K, which sums the parts and g's bias into h first.
 void Model::resid_ln32(const char* gname, const char* lname, const Gemm32Args& g, float* h, const float* w, const float* b,
-                       float eps, float* y) {
+                       float eps, float* y, float ys) {
   const int d = cfg.d;
   if (g.splits > 1) {
     op(gname, [&] { gemm32_launch(parts_of(g), stream); });
-    op(lname, [&] { splitk_resid_ln_launch(g.ws, g.splits, g.bias, h, w, eps, g.M, d, y, stream, ELEM_F32, b); });
+    op(lname, [&] { splitk_resid_ln_launch(g.ws, g.splits, g.bias, h, w, eps, g.M, d, y, stream, ELEM_F32, b, nullptr, nullptr, ys); });
   } else {
     op(gname, [&] { gemm32_launch(g, stream); });
-    op(lname, [&] { layernorm_launch(h, nullptr, w, b, eps, g.M, d, nullptr, y, nullptr, nullptr, nullptr, stream, elem); });
+    op(lname, [&] { layernorm_launch(h, nullptr, w, b, eps, g.M, d, y, nullptr, nullptr, nullptr, nullptr, stream, ELEM_F32, ys); });
   }
 }
 
@@ -1399,14 +1469,14 @@ void Model::run_encoder32(const Plan& p, const Acts32& a) {
   const int* pos = dmeta + p.off_pos;
   // h = LN(tok_emb[ids]) (lib.rs:1534-1551)
   op("embed", [&] {
-    gather_f32_launch(w32(tok_emb), ids, T, d, a.x, stream);
-    layernorm_launch(a.x, nullptr, emb_norm, nullptr, eps, T, d, nullptr, a.h, nullptr, nullptr, nullptr, stream, elem);
+    gather_f32_launch(w32(tok_emb), ids, T, d, a.att, stream);
+    layernorm_launch(a.att, nullptr, emb_norm, nullptr, eps, T, d, a.x, a.h, nullptr, nullptr, nullptr, stream, ELEM_F32,
+                     layers[0].s_qkv.a);
   });
   for (int l = 0; l < cfg.layers; ++l) {
     const LayerWeights& L = layers[l];
     const int tw = L.local ? 1 : 0;
-    const float* xin = l > 0 ? a.x : a.h;  // layer 0 attends from the embedding itself
-    const Gemm32Args gq = gemm32_args(xin, d, w32(L.wqkv), d, a.qkv, 3 * d, nullptr, T, 3 * d, d, ACT_NONE, false, a.ws);
+    const Gemm32Args gq = gemm32_args(L.s_qkv, a.x, d, w32(L.wqkv), d, a.qkv, 3 * d, nullptr, T, 3 * d, d, ACT_NONE, false, a.ws);
     op("wqkv", [&] { gemm32_launch(parts_of(gq), stream); });
     op("split_rope", [&] {
       split32_launch(gq.splits > 1 ? a.ws : a.qkv, gq.splits, nullptr, T, d, pos, rope_cos[tw], rope_sin[tw], a.q, a.k, a.v,
@@ -1426,6 +1496,7 @@ void Model::run_encoder32(const Plan& p, const Acts32& a) {
       at.T = T;
       at.ldo = d;
       at.scale = 1.0f / std::sqrt(float(cfg.head_dim()));
+      at.os = L.s_wo.a;
       attn32_launch(at, stream);
       if (L.local && p.nfar > 0) {  // the padding queries that the tiles do not take
         at.entries = dmeta + p.off_far;
@@ -1433,13 +1504,13 @@ void Model::run_encoder32(const Plan& p, const Acts32& a) {
         attn32_launch(at, stream);
       }
     });
-    resid_ln32("wo", "mlp_norm", gemm32_args(a.att, d, w32(L.wo), d, a.h, d, nullptr, T, d, d, ACT_NONE, true, a.ws), a.h,
-               L.mlp_norm, nullptr, eps, a.x);
-    const Gemm32Args gi = gemm32_args(a.x, d, w32(L.wi), d, a.mid, 2 * I, nullptr, T, 2 * I, d, ACT_NONE, false, a.ws);
+    resid_ln32("wo", "mlp_norm", gemm32_args(L.s_wo, a.att, d, w32(L.wo), d, a.h, d, nullptr, T, d, d, ACT_NONE, true, a.ws),
+               a.h, L.mlp_norm, nullptr, eps, a.x, L.s_wi.a);
+    const Gemm32Args gi = gemm32_args(L.s_wi, a.x, d, w32(L.wi), d, a.mid, 2 * I, nullptr, T, 2 * I, d, ACT_NONE, false, a.ws);
     op("wi", [&] { gemm32_launch(parts_of(gi), stream); });
-    op("geglu", [&] { geglu32_launch(gi.splits > 1 ? a.ws : a.mid, gi.splits, T, I, a.act, stream); });
-    const Gemm32Args go = gemm32_args(a.act, I, w32(L.wo2), I, a.h, d, nullptr, T, d, I, ACT_NONE, true, a.ws);
-    if (l + 1 < cfg.layers) resid_ln32("wo2", "attn_norm", go, a.h, layers[l + 1].attn_norm, nullptr, eps, a.x);
+    op("geglu", [&] { geglu32_launch(gi.splits > 1 ? a.ws : a.mid, gi.splits, T, I, a.act, L.s_wo2.a, stream); });
+    const Gemm32Args go = gemm32_args(L.s_wo2, a.act, I, w32(L.wo2), I, a.h, d, nullptr, T, d, I, ACT_NONE, true, a.ws);
+    if (l + 1 < cfg.layers) resid_ln32("wo2", "attn_norm", go, a.h, layers[l + 1].attn_norm, nullptr, eps, a.x, layers[l + 1].s_qkv.a);
     else op("wo2", [&] { gemm32_launch(go, stream); });
     layer_mark();
   }
@@ -1465,9 +1536,10 @@ void Model::forward32(const Plan& p, float* logits_out, float* pooled_out) {
     const HeadWeights& Hw = head[j];
     if (j == 0)
       op("head_norm1", [&] {
-        layernorm_launch(a.hh, nullptr, Hw.n1w, Hw.n1b, 1e-5f, T, d, nullptr, a.x, nullptr, nullptr, nullptr, stream, elem);
+        layernorm_launch(a.hh, nullptr, Hw.n1w, Hw.n1b, 1e-5f, T, d, a.x, nullptr, nullptr, nullptr, nullptr, stream, ELEM_F32,
+                         Hw.s_in.a);
       });
-    const Gemm32Args gq = gemm32_args(a.x, d, w32(Hw.in_w), d, a.qkv, 3 * d, Hw.in_b, T, 3 * d, d, ACT_NONE, false, a.ws);
+    const Gemm32Args gq = gemm32_args(Hw.s_in, a.x, d, w32(Hw.in_w), d, a.qkv, 3 * d, Hw.in_b, T, 3 * d, d, ACT_NONE, false, a.ws);
     op("head_in_proj", [&] { gemm32_launch(parts_of(gq), stream); });
     op("head_split", [&] {  // a product that does not split adds its bias itself
       split32_launch(gq.splits > 1 ? a.ws : a.qkv, gq.splits, gq.splits > 1 ? Hw.in_b : nullptr, T, d, nullptr, nullptr,
@@ -1492,17 +1564,21 @@ void Model::forward32(const Plan& p, float* logits_out, float* pooled_out) {
       at.T = T;
       at.ldo = d;
       at.scale = hscale;
+      at.os = Hw.s_out.a;
       attn32_launch(at, stream);
     });
     if (pruned) op("head_pick", [&] { gather_f32_launch(a.hh, picked, M, d, hj, stream); });
     resid_ln32("head_out_proj", "head_norm2",
-               gemm32_args(a.att, d, w32(Hw.out_w), d, hj, d, Hw.out_b, M, d, d, ACT_NONE, true, a.ws), hj, Hw.n2w, Hw.n2b,
-               1e-5f, a.x);
+               gemm32_args(Hw.s_out, a.att, d, w32(Hw.out_w), d, hj, d, Hw.out_b, M, d, d, ACT_NONE, true, a.ws), hj, Hw.n2w,
+               Hw.n2b, 1e-5f, a.x, Hw.s_l1.a);
     op("head_linear1", [&] {
-      gemm32_launch(gemm32_args(a.x, d, w32(Hw.l1_w), d, a.mid, 4 * d, Hw.l1_b, M, 4 * d, d, ACT_RELU, false, a.ws), stream);
+      gemm32_launch(gemm32_args(Hw.s_l1, a.x, d, w32(Hw.l1_w), d, a.mid, 4 * d, Hw.l1_b, M, 4 * d, d, ACT_RELU, false, a.ws,
+                                Hw.s_l2.a),
+                    stream);
     });
-    const Gemm32Args g2 = gemm32_args(a.mid, 4 * d, w32(Hw.l2_w), 4 * d, hj, d, Hw.l2_b, M, d, 4 * d, ACT_NONE, true, a.ws);
-    if (j + 1 < cfg.head_layers) resid_ln32("head_linear2", "head_norm1", g2, hj, head[j + 1].n1w, head[j + 1].n1b, 1e-5f, a.x);
+    const Gemm32Args g2 = gemm32_args(Hw.s_l2, a.mid, 4 * d, w32(Hw.l2_w), 4 * d, hj, d, Hw.l2_b, M, d, 4 * d, ACT_NONE, true, a.ws);
+    if (j + 1 < cfg.head_layers) resid_ln32("head_linear2", "head_norm1", g2, hj, head[j + 1].n1w, head[j + 1].n1b, 1e-5f, a.x,
+                                       head[j + 1].s_in.a);
     else op("head_linear2", [&] { gemm32_launch(g2, stream); });
   }
   const float* hs = set.headprune ? a.hp : a.hh;  // the rows that off_scorer and off_pooled index
@@ -1510,11 +1586,11 @@ void Model::forward32(const Plan& p, float* logits_out, float* pooled_out) {
   // scorer3; pooled = position 0 of each row
   if (R > 0) {
     op("scorer_norm", [&] {
-      layernorm_launch(hs, dmeta + p.off_scorer, sc0_w, sc0_b, 1e-5f, R, d, nullptr, a.sx, nullptr, nullptr, nullptr,
-                       stream, elem);
+      layernorm_launch(hs, dmeta + p.off_scorer, sc0_w, sc0_b, 1e-5f, R, d, a.sx, nullptr, nullptr, nullptr, nullptr,
+                       stream, ELEM_F32, s_sc1.a);
     });
     op("scorer1", [&] {
-      gemm32_launch(gemm32_args(a.sx, d, w32(sc1_w), d, a.s1, S, sc1_b, R, S, d, ACT_GELU, false, a.ws), stream);
+      gemm32_launch(gemm32_args(s_sc1, a.sx, d, w32(sc1_w), d, a.s1, S, sc1_b, R, S, d, ACT_GELU, false, a.ws), stream);
     });
     op("scorer3", [&] { rowdot32_launch(a.s1, sc3_w, sc3_b, R, S, a.logits, stream); });
   }

@@ -52,6 +52,13 @@ struct Settings {
   static Settings parse(const std::string& spec);
 };
 
+// dtype=f32: the power of two that a product's input is held times (split f32), and per output column
+// what undoes it and the weight row's.
+struct Scales32 {
+  float a = 1.0f;
+  const float* inv = nullptr;
+};
+
 struct LayerWeights {
   uint16_t* wqkv = nullptr;  // [3d, d]
   uint16_t* wo = nullptr;    // [d, d]
@@ -60,9 +67,11 @@ struct LayerWeights {
   float* attn_norm = nullptr;  // null for layer 0
   float* mlp_norm = nullptr;
   bool local = false;
+  Scales32 s_qkv, s_wo, s_wi, s_wo2;
 };
 
 struct HeadWeights {
+  Scales32 s_in, s_out, s_l1, s_l2;
   float *n1w, *n1b, *n2w, *n2b;
   uint16_t* in_w;
   float* in_b;
@@ -134,6 +143,7 @@ struct Model {
   float* sc1_b = nullptr;
   float* sc3_w = nullptr;
   float* sc3_b = nullptr;
+  Scales32 s_sc1;
   float* rope_cos[2] = {nullptr, nullptr};  // [max_pos, hd/2] for global (0) and local (1)
   float* rope_sin[2] = {nullptr, nullptr};
 
@@ -142,6 +152,7 @@ struct Model {
   size_t acap = 0;
   // the dtype=f32 path's activation arena
   void* fmem = nullptr;
+  void* imem = nullptr;  // the f32 products' inv arrays
   size_t fcap = 0;
   // pinned host staging
   void* hmeta = nullptr;
@@ -194,7 +205,8 @@ struct Model {
   Acts32 arena32(const Plan& p);
   void run_encoder32(const Plan& p, const Acts32& a);
   void resid_ln32(const char* gname, const char* lname, const Gemm32Args& g, float* h, const float* w, const float* b,
-                  float eps, float* y);
+                  float eps, float* y, float ys);
+  void split_weights32();
   void forward32(const Plan& p, float* logits, float* pooled);
   void encoder_hidden32(const Plan& p, float* hidden);
   // The f32 GEMM weights: with dtype=f32 the 16-bit weight pointers hold f32 tensors.

@@ -230,3 +230,56 @@ def test_f32_tile_edges(lens, kmax):
         assert float(np.abs(out.logits - lg).max()) <= LOGIT_ABS_F32
     pg, pr = out.pooled.reshape(b.n, -1), pl.reshape(b.n, -1)
     assert float((np.linalg.norm(pg - pr, axis=-1) / np.linalg.norm(pr, axis=-1)).max()) <= POOLED_REL_F32
+
+
+def _rescaled(st: bytes, cfg: dict, span: int) -> bytes:
+    """The same model in exact arithmetic, its operands spread over 2 * span powers of two: channel k
+    of mlp_norm times 2^e_k and column k of Wi divided by it, gate row j of Wi times 2^f_j and column
+    j of Wo divided by it."""
+    import struct
+
+    n = struct.unpack("<Q", st[:8])[0]
+    header, out = json.loads(st[8:8 + n]), bytearray(st)
+    rng = np.random.default_rng(8)
+
+    def scale(name, s):
+        a, z = (8 + n + o for o in header[name]["data_offsets"])
+        assert header[name]["dtype"] == "BF16"
+        w = (np.frombuffer(bytes(out[a:z]), np.uint16).astype(np.uint32) << 16).view(np.float32)
+        w = (w.reshape(header[name]["shape"]) * s.astype(np.float32)).reshape(-1)
+        out[a:z] = (w.view(np.uint32) >> 16).astype(np.uint16).tobytes()
+
+    inter = cfg["intermediate_size"]
+    for l in range(cfg["num_hidden_layers"]):
+        p = f"encoder.layers.{l}.mlp"
+        e = 2.0 ** rng.integers(-span, span + 1, cfg["hidden_size"])
+        f = 2.0 ** rng.integers(-span, span + 1, inter)
+        scale(p + "_norm.weight", e)
+        scale(p + ".Wi.weight", np.concatenate([np.ones(inter), f])[:, None] / e[None, :])
+        scale(p + ".Wo.weight", 1.0 / f[None, :])
+    return bytes(out)
+
+
+@pytest.mark.parametrize("span", [6, 10])
+def test_f32_wide_operand_range(span):
+    """The split operands keep f32's precision over a wide range of magnitudes: a model whose MLP
+    operands are spread over 2^12 and 2^20 gives the plain model's results. Each value is held to 2^-24
+    relative either way and a sum of K = 1024 rounds to at most K 2^-24, typically its root (2e-6);
+    three layers of two such products, doubled for the two models: 2e-5 relative. An operand rounded
+    to one f16 would be off by 2e-4 or more."""
+    from sys1rust_amd.workloads import collate, small_config
+
+    cfg = small_config(layers=3, vocab=1024)
+    cfg["pad_token_id"] = 1002
+    rng = np.random.default_rng(3)
+    b = collate([(rng.integers(0, 1000, L).tolist(), [1, L // 2], 0) for L in (70, 200, 33)], pad_id=1002)
+    st = synth_checkpoint(json.dumps(cfg), json.dumps(AGENT), seed=6, scorer_width=256)
+    outs = []
+    for image in (st, _rescaled(st, cfg, span)):
+        m = HipBackend(image, json.dumps(cfg), json.dumps(AGENT), settings=DEFAULT_TUNING + ",dtype=f32", device=0)
+        outs.append((m.encoder_hidden(b), m.forward(b)))
+        m.close()
+    rel = [float(np.linalg.norm(x - y) / np.linalg.norm(x)) for x, y in
+           ((outs[0][0], outs[1][0]), (outs[0][1].pooled, outs[1][1].pooled), (outs[0][1].logits, outs[1][1].logits))]
+    say(f"f32 operands over 2^{2 * span}: hidden, pooled, logits rel {rel}")
+    assert max(rel) <= 2e-5, rel
