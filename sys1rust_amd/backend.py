@@ -152,7 +152,7 @@ class HipBackend:
 
     def encoder_hidden(self, b: Batch) -> np.ndarray:
         ids, am, sl, mp, mc, qt = _batch_arrays(b)
-        hidden = np.zeros(max(b.n * b.len * self.d, 1), dtype=np.float32)
+        hidden = np.empty(max(b.n * b.len * self.d, 1), dtype=np.float32)  # written whole
         check(_lib.lib().s1_encoder_hidden(self._h, b.n, b.len, b.kmax, _ptr(ids, u32p), _ptr(am, u32p),
                                            _ptr(sl, u64p), _ptr(mp, u32p), _ptr(mc, u64p), _ptr(qt, u32p),
                                            _ptr(hidden, f32p)))

@@ -161,6 +161,11 @@ struct Model {
   size_t hout_cap = 0;
   int* dmeta = nullptr;
   size_t dmeta_cap = 0;
+  // pinned staging of a large download: a piece for each of kCopiers threads
+  static constexpr size_t kPiece = size_t(2) << 20;
+  static constexpr int kCopiers = 4;
+  void* hring = nullptr;
+  hipEvent_t ring_ev[kCopiers] = {};
 
   // per-kernel timing (Settings::ops)
   struct OpRec {
@@ -216,6 +221,8 @@ struct Model {
   void teardown();
   Acts arena(const Plan& p);
   void upload(const Plan& p);
+  // Copies device memory to the caller's pageable memory behind the work enqueued so far, and waits.
+  void download(void* dst, const void* src, size_t bytes, const char* what);
   // Enqueues the encoder; with fold_last, the last layer's Wo2 may leave its split-K partials in
   // the workspace for the caller's next kernel: returns their count then (else 0).
   int run_encoder(const Plan& p, const Acts& a, bool fold_last = false);

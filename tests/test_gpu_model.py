@@ -137,6 +137,29 @@ def test_encoder_hidden_far_padding_tiles(small_model, settings):
     m.close()
 
 
+@pytest.mark.parametrize("rows", [31, 32, 33, 130])
+def test_encoder_hidden_download_pieces(small_model, rows):
+    """encoder_hidden's output around the size from which it is downloaded in 2 MiB pieces by several
+    threads (4 MiB), and past a second round of pieces: every row is that of the batch of one, alone,
+    wherever its piece falls, within the 16-bit layers' gate (a batch may take other tiles), and the same
+    call again is the same bits."""
+    cfg, agent, st, _, _ = small_model
+    d, L = cfg["hidden_size"], (4 << 20) // 4 // 32 // cfg["hidden_size"]
+    rng = np.random.default_rng(5)
+    ids = rng.integers(5, 1000, size=(rows, L)).astype(np.uint32)
+    batch = lambda x: Batch(len(x), L, 0, x.reshape(-1), np.ones(x.size, np.uint32), np.full(len(x), L, np.uint64),
+                            np.zeros(0, np.uint32), np.zeros(len(x), np.uint64), np.zeros(len(x), np.uint32))
+    m = HipBackend(st, json.dumps(cfg), json.dumps(agent))
+    say(f"download of {rows} rows x {L} x {d}")
+    hid = m.encoder_hidden(batch(ids)).reshape(rows, L, d)
+    assert np.array_equal(hid, m.encoder_hidden(batch(ids)).reshape(rows, L, d))
+    for r in (0, rows // 2, rows - 1):
+        one = m.encoder_hidden(batch(ids[r: r + 1])).reshape(L, d)
+        rel = np.linalg.norm(hid[r] - one, axis=-1) / np.linalg.norm(one, axis=-1)
+        assert float(rel.max()) <= HIDDEN_REL_GATE, (rows, r, float(rel.max()))
+    m.close()
+
+
 @pytest.mark.parametrize("head_layers", [0, 1])
 def test_decision_head_depths(small_model, head_layers):
     """Agents with no decision-head layer (the scorer reads the encoder's stream, which headprune
