@@ -80,16 +80,18 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, char* smem0, int m0
   static_assert((STAGES - 2) * LPW < 64, "vmcnt range");
 
   // KG > 1 (k-groups): the workgroup holds KG groups of NW waves; group k runs k-tiles
-  // [kt0 + k NK / KG, kt0 + (k + 1) NK / KG) on stage buffers of its own (NK divides by KG, so
-  // every group passes the same barriers), and group 0 adds the other groups' accumulators, in
+  // [kt0 + k NK / KG, kt0 + (k + 1) NK / KG) on stage buffers of its own (a group with a k-tile
+  // less passes the last one's barrier all the same), and group 0 adds the other groups' accumulators, in
   // group order, from LDS and runs the epilogue alone. A short GEMM's chain of dependent k-tiles
   // is then KG times shorter on the same tiles.
   const int grp = KG > 1 ? __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6) / NW : 0;
   const int tid = threadIdx.x - grp * NW * 64;
   char* const smem = smem0 + grp * STAGES * STAGE_BYTES;
+  const int NKmax = (NK + KG - 1) / KG;
   if constexpr (KG > 1) {
-    kt0 += grp * (NK / KG);
-    NK /= KG;
+    const int b = grp * NK / KG;
+    kt0 += b;
+    NK = (grp + 1) * NK / KG - b;
   }
   const int lane = tid & 63;
   // Wave-uniform, so everything derived from it (load row groups, LDS destinations) is scalar.
@@ -264,6 +266,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, char* smem0, int m0
   }
 
   if constexpr (KG > 1) {
+    if (NK < NKmax) barrier_lds();
     // Groups 1.. leave their accumulators in their own stage buffers, in register order (float4
     // e4 of fragment (i, j) of wave w at ((w FM + i) FN + j) 4 + e4, 64 lanes apart), and end;
     // waves that have ended take no part in the barriers that follow.
@@ -694,12 +697,13 @@ void launch_te(const GemmArgs& g, hipStream_t st) {
       // Except for the k-groups below, the k-loop order is the same for every tile, so the results
       // are the same bits. The q|k|v product takes 64 x 64 tiles while they fit one workgroup per
       // CU (a third fewer bytes per k-tile, twice the workgroups): at 174 tokens 13.0 -> 12.2 µs
-      // per launch (the GeGLU product lost 2% that way). A GEMM with a 16-bit epilogue whose
-      // 64 x 64 tiles fit one workgroup per CU runs them in two k-groups of 4 waves (8 k-tiles
-      // each where there were 16): at 174 tokens q|k|v 9.9 -> 8.9 µs and GeGLU 9.8 -> 8.2 µs
-      // (GeGLU on twice the workgroups of its 64 x 128 tiles), weights cold in HBM.
-      constexpr bool KGOK = EPI != EPI_RESID && EPI != EPI_F32;
-      if (KGOK && g.splits == 1 && (g.K / BK) % 2 == 0 && (long long)((g.M + 63) / 64) * (g.N / 64) <= 256)
+      // per launch (the GeGLU product lost 2% that way). An unsplit GEMM whose
+      // 64 x 64 tiles fit one workgroup per CU runs them in two k-groups (8 k-tiles each where
+      // there were 16): at 174 tokens q|k|v 9.9 -> 8.9 µs and GeGLU 9.8 -> 8.2 µs (GeGLU on twice
+      // the workgroups of its 64 x 128 tiles), weights cold in HBM; a residual product of 563 x
+      // 1024 x 2624, a chain of 41 k-tiles on 72 CUs before, 18.5 -> 12.4 µs.
+      constexpr bool KGOK = EPI != EPI_F32;
+      if (KGOK && g.splits == 1 && g.K >= 2 * BK && (long long)((g.M + 63) / 64) * (g.N / 64) <= 256)
         launch_t<E, 64, 64, 64, 4, 2, 1, EPI, KGOK ? 2 : 1>(g, st);
       else if (EPI == EPI_ROPE && (long long)((g.M + 63) / 64) * (g.N / 64) * g.splits <= 256)
         launch_t<E, 64, 64, 64, 4, 2, 1, EPI>(g, st);

@@ -122,6 +122,26 @@ def test_gemm_epilogues_bias_relu_gelu_residual_geglu(dev, M, N):
     assert bool(((act - r).abs() <= r.abs() * 2 ** -7 + 1e-4).all()), float((act - r).abs().max())
 
 
+# 64 x 64 tiles in two k-groups: one k-tile each, one and two, an odd number of many, with partial
+# row tiles and at the 256 tiles that still run so
+@pytest.mark.parametrize("M,K", [(705, 128), (563, 192), (1024, 192), (300, 320), (563, 2624)])
+def test_gemm_k_groups_of_any_k(dev, M, K):
+    N = 1024
+    say(f"k-groups M={M} K={K}")
+    g = torch.Generator(device="cpu").manual_seed(M + K)
+    A = bf16_bits(torch.randn(M, K, generator=g)).to(dev)
+    W = bf16_bits(torch.randn(N, K, generator=g) * 0.02).to(dev)
+    bias = (torch.randn(N, generator=g) * 0.1).to(dev)
+    ref = (as_f32(A).double() @ as_f32(W).double().T + bias).float()
+    scale = float(ref.abs().max())
+    ob = as_f32(gemm(A, W, M, N, K, epi=0, bias=bias))
+    assert bool(((ob - ref).abs() <= ref.abs() * 2 ** -8 + 1e-5 * scale).all())
+    h0 = torch.randn(M, N, generator=g).to(dev)
+    h = h0.clone()
+    gemm(A, W, M, N, K, epi=1, bias=bias, C_out=h)
+    assert float((h - (h0 + ref)).abs().max()) <= 2e-5 * scale + 1e-5
+
+
 @pytest.mark.parametrize("M", [5686, 5000])
 def test_gemm_long_k_one_round_pipelined(dev, M):
     """One round of 192 x 128 tiles (200 to 256 of them) with K >= 2048 takes the pipelined
