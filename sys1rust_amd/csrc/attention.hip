@@ -10,8 +10,8 @@
 // packed layout at all.
 //
 // Work split: a workgroup of NW wavefronts takes up to 32 NW queries of one sequence and one
-// head; each wave owns 32 queries. Keys stream through LDS in chunks of 64 (double-buffered on
-// global layers): K as [key][dim] and V as [dim][key], copied with 16-byte accesses from the
+// head; each wave owns 32 queries (64 in attn_wide_kernel, the global layers of batches that fill
+// the GPU). Keys stream through LDS in chunks of 64 (double-buffered on global layers): K as [key][dim] and V as [dim][key], copied with 16-byte accesses from the
 // transposed v buffer. On local layers waves skip chunks, and 32-key halves, outside their
 // window, and only chunks that cross a window or row edge pay for masking. Short batches (fewer
 // tiles than CUs) take 32-query tiles whose keys several waves split and merge at the end
@@ -36,6 +36,7 @@
 
 #include "device.hpp"
 #include "kernels.hpp"
+#include "lds_load.hpp"
 
 namespace s1 {
 
@@ -317,6 +318,222 @@ void attn_kernel(AttnArgs a) {
     }
 }
 
+// Global layers of batches that fill the GPU: a wave owns 64 queries, as two halves of 32, and a
+// workgroup of 4 waves the same 256 queries that 8 waves of 32 would. Each K and V^T fragment read
+// from LDS then feeds two MFMAs, and half 1's softmax weights are computed beside half 0's V^T P^T
+// products. Two waves per SIMD: by counters a SIMD spends 477k cycles on VALU issue (an exp2 costs
+// two FMAs) and 262k on MFMAs at 8192 keys and 16 heads, and at equal priority a launch took their
+// sum. The priority raised over the weights and the V^T P^T products lets one wave's vector work
+// go ahead while the other's K Q^T products run (raised over K Q^T, or from the row maximum on, it
+// gains nothing). With this and the order of the tiles, against 8 waves of 32 queries, 16 heads:
+// 8192 keys 336 -> 310 µs (890 TFLOP/s), 10 rows of 547 to 579 tokens 34.1 -> 30.6, 12 of 300 to
+// 1100 61.3 -> 51.8, 48 of 215 to 2038 510 -> 481. The same work with 32 queries per wave and four
+// waves per SIMD (128 registers, 10 spilled) is 2 to 7% slower, and V^T in its own order in LDS, by direct loads, with a
+// lane's 8 keys read as two 8-byte halves, 1 to 6%. For 128-query tiles, about one wave per SIMD,
+// attn_kernel is faster (6 rows of 286 to 391 tokens, 12 heads: 11.6 against 13.8 µs with two
+// waves of 64).
+//
+// The next chunk's loads run during this one's math; layouts and sums are attn_kernel's (the same
+// bits).
+//
+// Workgroup b takes head b % heads of tile b / heads; the tiles come longest key range first
+// (attn_plan_tiles), so that the short ones fill what the long ones leave at the end. Workgroups
+// go round the 8 XCDs, so a head stays on one XCD's L2 (on two where heads are a multiple of 4 only).
+constexpr int WQ = 256;  // queries per workgroup
+template <class E>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void attn_wide_kernel(AttnArgs a) {
+  typedef typename E::v8 v8;
+  constexpr int QH = 2;        // query halves of a wave
+  constexpr int CB = KC * 64;  // elements of a staged chunk
+  __shared__ __attribute__((aligned(1024))) uint16_t smem[4 * CB];  // [K0 | V0 | K1 | V1]
+
+  const AttnTile tl = a.tiles[blockIdx.x / a.heads];
+  const int head = blockIdx.x % a.heads;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
+  const int hl = lane >> 5, col = lane & 31;
+  const uint16_t* __restrict__ Qh = a.q + size_t(head) * a.Tq * 64;
+  const uint16_t* __restrict__ Kh = a.k + size_t(head) * a.Tk * 64;
+  const uint16_t* __restrict__ Vt = a.v + size_t(head) * 64 * a.ldv;
+
+  const int wq0 = tl.q0 + wave * QH * 32;
+  const bool wave_active = wq0 < tl.q1;
+  const int kb0 = tl.k0, kb1 = tl.k1;
+  const int cstart = kb0 & ~7;  // V^T rows are read in aligned pieces of 8 keys
+  const int vlast = cstart + (((kb1 - 1) - cstart) & ~7);
+
+  v8 qf[QH][4];  // dims 16 kb + 8 h .. + 7 of this lane's two queries
+#pragma unroll
+  for (int qh = 0; qh < QH; ++qh) {
+    const int qi = min(wq0 + qh * 32 + col, tl.q1 - 1);
+    const uint16_t* qp = Qh + size_t(a.qkey ? a.qkey[qi] : qi) * 64 + hl * 8;
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) qf[qh][kb] = *reinterpret_cast<const v8*>(qp + kb * 16);
+  }
+
+  // A chunk's 16 KiB: wave w moves row groups 2w and 2w + 1 of K and of V^T (8 rows of 128 bytes
+  // each), K by direct global -> LDS loads, V^T through registers. K rows past kb1 repeat the last key; V^T pieces past it repeat the piece that holds it,
+  // which may hold up to 7 keys past kb1: the next row's, or the zeros that every writer of v
+  // leaves up to a multiple of 8 tokens. Those meet weights of 0.
+  const int r8 = lane >> 3, slot = lane & 7;
+  uint4 vreg[2];
+  auto stage = [&](int c0, int buf) __attribute__((always_inline)) {
+    char* dst = reinterpret_cast<char*>(smem + buf * 2 * CB);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int gi = wave * 2 + i, row = gi * 8 + r8;
+      __builtin_amdgcn_global_load_lds(Kh + size_t(min(c0 + row, kb1 - 1)) * 64 + kslot(row, slot) * 8, dst + gi * 1024,
+                                       16, 0, 0);
+      vreg[i] = *reinterpret_cast<const uint4*>(Vt + size_t(row) * a.ldv + min(c0 + slot * 8, vlast));
+    }
+  };
+  auto vstore = [&](int buf) __attribute__((always_inline)) {
+    uint16_t* sv = smem + buf * 2 * CB + CB;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int row = (wave * 2 + i) * 8 + r8;
+      uint16_t* p = sv + row * 64 + (slot & 1) * 4;
+      *reinterpret_cast<uint2*>(p + kslot(row, slot & ~1) * 8) = make_uint2(vreg[i].x, vreg[i].y);
+      *reinterpret_cast<uint2*>(p + kslot(row, slot | 1) * 8) = make_uint2(vreg[i].z, vreg[i].w);
+    }
+  };
+
+  const float sl2 = a.scale * 1.4426950408889634f;  // exp(x) = exp2(x log2 e)
+  float m[QH], l[QH];
+  f32x16 o[QH][2];
+#pragma unroll
+  for (int qh = 0; qh < QH; ++qh) {
+    m[qh] = NEG_INF;
+    l[qh] = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) o[qh][0][e] = o[qh][1][e] = 0.0f;
+  }
+
+  int fo[4];  // LDS element offsets of this lane's fragments, of K and of V^T alike
+#pragma unroll
+  for (int i = 0; i < 4; ++i) fo[i] = col * 64 + kslot(col, i * 2 + hl) * 8;
+
+  auto chunk = [&](int c0, int buf) __attribute__((always_inline)) {
+    const bool edge = c0 < kb0 || c0 + KC > kb1;
+    const uint16_t* sk = smem + buf * 2 * CB;
+    const uint16_t* sv = sk + CB;
+    v8 kf[2][4];
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) kf[t][kb] = *reinterpret_cast<const v8*>(sk + t * 32 * 64 + fo[kb]);
+    f32x16 s[QH][2];
+#pragma unroll
+    for (int qh = 0; qh < QH; ++qh) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) s[qh][t][e] = 0.0f;
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) s[qh][t] = E::mfma(kf[t][kb], qf[qh][kb], s[qh][t]);
+    }
+    if (edge) {  // only the first and the last chunk hold keys outside the range
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const int kbase = c0 + t * 32 + hl * 4, lo = kb0 - kbase, hi = kb1 - kbase;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int off = (e >> 2) * 8 + (e & 3);
+          const bool in = off >= lo && off < hi;
+#pragma unroll
+          for (int qh = 0; qh < QH; ++qh) s[qh][t][e] = in ? s[qh][t][e] : NEG_INF;
+        }
+      }
+    }
+    float alpha[QH], ms[QH];
+#pragma unroll
+    for (int qh = 0; qh < QH; ++qh) {
+      float mx = NEG_INF;
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) mx = fmaxf(mx, s[qh][t][e]);
+      const float mn = fmaxf(m[qh], half_max(mx) * sl2);
+      ms[qh] = mn == NEG_INF ? 0.0f : mn;  // nothing visible yet: every p is exp2(-inf) = 0
+      alpha[qh] = __builtin_amdgcn_exp2f(m[qh] - ms[qh]);
+      m[qh] = mn;
+    }
+    if (alpha[0] != 1.0f || alpha[QH - 1] != 1.0f) {  // skipped by the wave once its maxima have settled
+#pragma unroll
+      for (int qh = 0; qh < QH; ++qh) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          o[qh][0][e] *= alpha[qh];
+          o[qh][1][e] *= alpha[qh];
+        }
+      }
+    }
+    __builtin_amdgcn_s_setprio(1);
+    v8 vf[2][4], pf[4];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+      for (int dt = 0; dt < 2; ++dt) vf[dt][ks] = *reinterpret_cast<const v8*>(sv + dt * 32 * 64 + fo[ks]);
+#pragma unroll
+    for (int qh = 0; qh < QH; ++qh) {
+      float psum = 0.0f;
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const float p = __builtin_amdgcn_exp2f(fmaf(s[qh][t][e], sl2, -ms[qh]));
+          psum += p;
+          pf[t * 2 + (e >> 3)][e & 7] = typename E::scalar(p);
+        }
+      l[qh] = l[qh] * alpha[qh] + psum;
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+        for (int dt = 0; dt < 2; ++dt) o[qh][dt] = E::mfma(vf[dt][ks], pf[ks], o[qh][dt]);
+    }
+    __builtin_amdgcn_s_setprio(0);
+  };
+
+  stage(cstart, 0);
+  vstore(0);
+  wait_vmcnt<0>();
+  __syncthreads();
+  int buf = 0;
+  for (int c0 = cstart; c0 < kb1; c0 += KC, buf ^= 1) {
+    const bool more = c0 + KC < kb1;
+    if (more) stage(c0 + KC, buf ^ 1);  // that buffer was last read before the last barrier
+    if (wave_active) chunk(c0, buf);
+    if (more) vstore(buf ^ 1);
+    wait_vmcnt<0>();
+    __syncthreads();
+  }
+
+  if (!wave_active) return;
+  // The wave's 64 rows leave through its own 8 KiB of LDS (every wave is past its last read), so
+  // that a store writes whole 128-byte rows: chunk c of row r at slot c ^ (r % 8).
+  uint16_t* st = smem + wave * QH * 32 * 64;
+#pragma unroll
+  for (int qh = 0; qh < QH; ++qh) {
+    const float inv = 1.0f / half_sum(l[qh]);
+#pragma unroll
+    for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const uint2 w = make_uint2(E::pack2(o[qh][dt][g * 4 + 0] * inv, o[qh][dt][g * 4 + 1] * inv),
+                                   E::pack2(o[qh][dt][g * 4 + 2] * inv, o[qh][dt][g * 4 + 3] * inv));
+        *reinterpret_cast<uint2*>(st + (qh * 32 + col) * 64 + ((dt * 4 + g) ^ (col & 7)) * 8 + hl * 4) = w;
+      }
+  }
+#pragma unroll
+  for (int i = 0; i < QH * 4; ++i) {
+    const int r = i * 8 + r8;
+    const uint4 v = *reinterpret_cast<const uint4*>(st + r * 64 + (slot ^ (r & 7)) * 8);
+    if (wq0 + r < tl.q1) *reinterpret_cast<uint4*>(a.out + size_t(wq0 + r) * a.ldo + head * 64 + slot * 8) = v;
+  }
+}
+
 // Local layers with a window of at most 64 keys: a workgroup's 128 queries see at most
 // 128 + 2 * 64 keys, so the whole key range is staged in LDS at once (every load of the
 // workgroup in flight together, one barrier) and each wave then runs its queries' softmax over
@@ -506,7 +723,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
       *reinterpret_cast<uint2*>(orow + dim) = w;
     }
 }
-
 
 // Global attention for a short batch (one request): a workgroup of KW waves takes 32 queries of
 // one row and head, and wave w visits the row's key chunks w, w + KW, ... with softmax statistics
@@ -886,11 +1102,12 @@ int attn_local_tile(const int* row_start, int n, int heads, int window) {
 int attn_row_step(int len, int qb) {
   if (qb <= 32) return qb;
   const int nt = (len + qb - 1) / qb;
-  return std::min(qb, ((len + nt - 1) / nt + 31) / 32 * 32);
+  const int wave = qb == WQ ? 64 : 32;  // queries of a wave
+  return std::min(qb, ((len + nt - 1) / nt + wave - 1) / wave * wave);
 }
 
-// 256-query tiles (8 waves, every K/V chunk shared by 256 queries) while they give at least one
-// workgroup per CU; then 128 (4 waves) while they give 128 workgroups; a shorter batch takes
+// 256-query tiles (attn_wide_kernel, every K/V chunk shared by 256 queries) while they give at
+// least one workgroup per CU; then 128 (4 waves) while they give 128 workgroups; a shorter batch takes
 // 32-query tiles whose keys are split over 4 waves (attn_ksplit_kernel).
 static int global_tile(const int* row_start, const int* q_end, int n, int heads) {
   auto count = [&](int qb) {
@@ -907,18 +1124,20 @@ int attn_global_tile(const int* row_start, int n, int heads) { return global_til
 int attn_plan_tiles(const int* row_start, int n, int heads, int window, std::vector<int>& out, const int* q_end,
                     const int* k_end) {
   const int qb = window >= 0 ? local_tile(row_start, q_end, n, heads, window) : global_tile(row_start, q_end, n, heads);
+  std::vector<AttnTile> tiles;
   for (int r = 0; r < n; ++r) {
     const int rs = row_start[r], qe = q_end ? q_end[r] : row_start[r + 1], ke = k_end ? k_end[r] : row_start[r + 1];
     const int step = attn_row_step(qe - rs, qb);
     for (int q0 = rs; q0 < qe; q0 += step) {
       const int q1 = std::min(q0 + step, qe);
       const bool win = window >= 0 && qb == 32;
-      out.push_back(q0);
-      out.push_back(q1);
-      out.push_back(win ? std::max(rs, q0 - window) : rs);
-      out.push_back(win ? std::min(ke, q1 + window) : ke);
+      tiles.push_back({q0, q1, win ? std::max(rs, q0 - window) : rs, win ? std::min(ke, q1 + window) : ke});
     }
   }
+  if (window < 0 && qb == WQ)  // attn_wide_kernel: most keys first
+    std::stable_sort(tiles.begin(), tiles.end(),
+                     [](const AttnTile& x, const AttnTile& y) { return x.k1 - x.k0 > y.k1 - y.k0; });
+  for (const AttnTile& t : tiles) out.insert(out.end(), {t.q0, t.q1, t.k0, t.k1});
   return qb;
 }
 
@@ -932,7 +1151,7 @@ void attn_launch_t(const AttnArgs& a, hipStream_t st) {
   else if (a.window >= 0)
     hipLaunchKernelGGL((attn_kernel<E, true, 4>), grid, dim3(256), 0, st, a);
   else if (a.tile_q == 256)
-    hipLaunchKernelGGL((attn_kernel<E, false, 8>), grid, dim3(512), 0, st, a);
+    hipLaunchKernelGGL(attn_wide_kernel<E>, grid, dim3(256), 0, st, a);
   else if (a.tile_q == 128)
     hipLaunchKernelGGL((attn_kernel<E, false, 4>), grid, dim3(256), 0, st, a);
   else if (a.key_waves == 8)  // tile_q 32

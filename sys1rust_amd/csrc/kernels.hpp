@@ -90,7 +90,7 @@ struct AttnArgs {
   int ldo = 0;
   float scale = 0.125f;
   int window = -1;  // < 0: global attention; else keys with |i - j| <= window
-  // Queries per tile. Global attention: 256 or 128 (8 or 4 waves, each with 32 queries and every
+  // Queries per tile. Global attention: 256 or 128 (4 waves, each with 64 or 32 queries and every
   // key), or 32: then key_waves (4 or 8) waves split each tile's keys. Local (window <= 64): 128,
   // or 32, whose keys (the tile's window range) 4 waves split.
   int tile_q = 256;

@@ -336,6 +336,15 @@ def test_attention_varlen(dev, window, lens):
     assert float(err.mean()) <= 2e-3, float(err.mean())
 
 
+# 256-query tiles of the global kernel (at least 16 of them with 16 heads): rows that end at, before
+# and after a wave's 64 queries, a tile's 256 and a chunk's 64 keys, that start at every offset
+# within 8 keys, and tiles in an order of their own (most keys first)
+@pytest.mark.parametrize("lens", [[63, 64, 65, 1, 255, 256, 257, 31, 33, 319, 320, 321, 511, 512, 513, 7, 2],
+                                  [2049] + [1] * 9 + [100, 700], [128] * 20])
+def test_attention_wide_tiles(dev, lens):
+    test_attention_varlen(dev, -1, lens)
+
+
 def test_layernorm(dev):
     say("layernorm")
     M, d = 333, 1024
