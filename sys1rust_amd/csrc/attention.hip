@@ -541,7 +541,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
 // K and V^T take turns in one LDS buffer (38 KiB): K for the logits, then V^T, loaded while the
 // softmax weights are computed. At the 10-request headline that fits four workgroups per CU,
 // all 800 tiles in one round, where K and V^T side by side (71 KiB) fit two and took 1.56
-// rounds (16.4 -> 15.0 µs per launch, the same bits).
+// rounds (16.4 -> 15.0 µs per launch, the same bits). The results leave as whole rows through
+// LDS: 48 rows of 215 to 2038 tokens 108 -> 92 µs, 10 of 547 to 579 16.5 -> 15.5 (the same bits).
 constexpr int LQ = 128;                 // queries per workgroup: 4 waves x 32
 constexpr int LMAXW = 64;               // largest window this kernel stages
 constexpr int LMAXK = LQ + 2 * LMAXW + 8;  // staged keys: the range plus 8-alignment slack
@@ -585,7 +586,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
   const int wq0 = tl.q0 + wave * 32;
   const bool wact = wq0 < tl.q1;
   const int qi = wq0 + col;
-  const bool qvalid = qi < tl.q1;
   const int qk = min(qi, tl.q1 - 1);
   v8 qf[4];
 #pragma unroll
@@ -687,7 +687,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
-  if (!wact) return;  // no barrier follows
+  if (!wact) return;  // a wave that has ended takes no part in the barrier that follows
   f32x16 o[2];
 #pragma unroll
   for (int e = 0; e < 16; ++e) { o[0][e] = 0.0f; o[1][e] = 0.0f; }
@@ -708,21 +708,28 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
       }
     }
   }
-  const float lt = half_sum(psum);
-  if (!qvalid) return;
-  const float inv = 1.0f / lt;
-  uint16_t* orow = a.out + size_t(qi) * a.ldo + head * 64;
+  // The wave's 32 rows leave through its own 4 KiB of the buffer once every wave has read V^T, so
+  // that a store writes whole 128-byte rows: chunk c of row r at slot c ^ (r % 8).
+  const float inv = 1.0f / half_sum(psum);
+  __syncthreads();
+  uint16_t* st = sbuf + wave * 32 * 64;
 #pragma unroll
   for (int dt = 0; dt < 2; ++dt)
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int dim = dt * 32 + g * 8 + hl * 4;
-      uint2 w;
-      w.x = E::pack2(o[dt][g * 4 + 0] * inv, o[dt][g * 4 + 1] * inv);
-      w.y = E::pack2(o[dt][g * 4 + 2] * inv, o[dt][g * 4 + 3] * inv);
-      *reinterpret_cast<uint2*>(orow + dim) = w;
-    }
+    for (int g = 0; g < 4; ++g)
+      *reinterpret_cast<uint2*>(st + col * 64 + ((dt * 4 + g) ^ (col & 7)) * 8 + hl * 4) =
+          make_uint2(E::pack2(o[dt][g * 4 + 0] * inv, o[dt][g * 4 + 1] * inv),
+                     E::pack2(o[dt][g * 4 + 2] * inv, o[dt][g * 4 + 3] * inv));
+  const int r8 = lane >> 3, slot = lane & 7;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = i * 8 + r8;
+    const uint4 v = *reinterpret_cast<const uint4*>(st + r * 64 + (slot ^ (r & 7)) * 8);
+    if (wq0 + r < tl.q1) *reinterpret_cast<uint4*>(a.out + size_t(wq0 + r) * a.ldo + head * 64 + slot * 8) = v;
+  }
 }
+
+
 
 // Global attention for a short batch (one request): a workgroup of KW waves takes 32 queries of
 // one row and head, and wave w visits the row's key chunks w, w + KW, ... with softmax statistics
