@@ -1525,11 +1525,11 @@ void Model::run_encoder32(const Plan& p, const Acts32& a) {
   const float eps = float(cfg.eps);
   const int* ids = dmeta + p.off_ids;
   const int* pos = dmeta + p.off_pos;
-  // h = LN(tok_emb[ids]) (lib.rs:1534-1551)
+  // h = LN(tok_emb[ids]) (lib.rs:1534-1551), and the first layer's input, if there is a layer
   op("embed", [&] {
     gather_f32_launch(w32(tok_emb), ids, T, d, a.att, stream);
-    layernorm_launch(a.att, nullptr, emb_norm, nullptr, eps, T, d, a.x, a.h, nullptr, nullptr, nullptr, stream, ELEM_F32,
-                     layers[0].s_qkv.a);
+    layernorm_launch(a.att, nullptr, emb_norm, nullptr, eps, T, d, layers.empty() ? nullptr : a.x, a.h, nullptr, nullptr,
+                     nullptr, stream, ELEM_F32, layers.empty() ? 1.0f : layers[0].s_qkv.a);
   });
   for (int l = 0; l < cfg.layers; ++l) {
     const LayerWeights& L = layers[l];

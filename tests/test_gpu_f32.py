@@ -107,6 +107,21 @@ def test_f32_short_rows_and_no_markers(small):
     m.close()
 
 
+@pytest.mark.parametrize("layers", [0, 1])
+def test_f32_encoder_depths(small, layers):
+    """An encoder without layers (the embeddings, the final norm and the head), and one with one."""
+    cfg, agent, _, b = small
+    cfg = dict(cfg, num_hidden_layers=layers)
+    st = synth_checkpoint(json.dumps(cfg), json.dumps(agent), 9, 256, 2, True)
+    o = O.Oracle(st, cfg, agent)
+    ref = o.encoder_hidden(b)
+    lg, pl = o.forward(b, ref)
+    for settings in ("dtype=f32", DEFAULT_TUNING + ",dtype=f32"):
+        m = HipBackend(st, json.dumps(cfg), json.dumps(agent), settings=settings)
+        gate_f32(m, b, ref, lg, pl, ActHead.from_weights(o.w), f"f32 layers={layers} {settings[-30:]!r}")
+        m.close()
+
+
 def test_f32_modernbert_large_512_tokens():
     """The 28-layer ModernBERT-large shape over a 512-token state with one question, and a padded
     600-position batch at every position (chunked local attention for the padding), against the
