@@ -982,8 +982,9 @@ __global__ __launch_bounds__(256) void attn_far_kernel(FallbackArgs a) {
   f32x16 o[2];
 #pragma unroll
   for (int e = 0; e < 16; ++e) o[0][e] = o[1][e] = 0.0f;
+  uint32_t up = 0, down = 0;  // output elements that a value of +inf, of -inf (NaN: both) reaches
   // 32-key tiles start 8-aligned, so V^T is read in aligned pieces of 4 keys; pieces past the range
-  // repeat the one of its last key (finite values that meet weights of 0).
+  // repeat the one of its last key (values that meet weights of 0).
   const int first[2] = {tile[2] & ~7, tile[4] & ~7}, end[2] = {tile[3], tile[5]};
   const int na = (end[0] - first[0] + 31) >> 5, nb = (end[1] - first[1] + 31) >> 5;
   for (int t = wave; t < na + nb; t += KW) {
@@ -1030,13 +1031,28 @@ __global__ __launch_bounds__(256) void attn_far_kernel(FallbackArgs a) {
       o[0][e] *= alpha;
       o[1][e] *= alpha;
     }
+    // A weight of 0 times a value that is not finite is NaN: such a value goes into the product as the
+    // largest finite one (NaN: the lowest), and the lanes whose query names its key note it.
+    float most = 0.0f;
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
 #pragma unroll
       for (int dt = 0; dt < 2; ++dt) {
         const uint32_t w = (e & 2) ? vr[dt][e >> 2].y : vr[dt][e >> 2].x;
-        const float v = E::f32(uint16_t((e & 1) ? w >> 16 : w));
+        const float v = __builtin_amdgcn_fmed3f(E::f32(uint16_t((e & 1) ? w >> 16 : w)), -__FLT_MAX__, __FLT_MAX__);
+        most = fmaxf(most, fabsf(v));
         o[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(v, s[e], o[dt], 0, 0, 0);
+      }
+    }
+    if (__any(most == __FLT_MAX__)) {
+      for (int key = kb; key < min(kb + 32, last + 1); ++key) {
+        const bool seen = key >= r0 && key < r1;
+        for (int e = 0; e < 32; ++e) {
+          const float v = E::f32(Vt[size_t((e >> 2) * 8 + 4 * hl + (e & 3)) * a.ldv + key]);
+          if (!seen || fabsf(v) < __builtin_huge_valf()) continue;
+          if (v != NEG_INF) up |= 1u << e;
+          if (v != -NEG_INF) down |= 1u << e;
+        }
       }
     }
   }
@@ -1056,7 +1072,8 @@ __global__ __launch_bounds__(256) void attn_far_kernel(FallbackArgs a) {
   mt[wave * 64 + lane] = m;
   lt[wave * 64 + lane] = l;
 #pragma unroll
-  for (int e = 0; e < 32; ++e) ot[(wave * 32 + e) * 64 + lane] = o[e >> 4][e & 15];
+  for (int e = 0; e < 32; ++e)
+    ot[(wave * 32 + e) * 64 + lane] = o[e >> 4][e & 15] + ((up >> e & 1) ? -NEG_INF : 0.0f) + ((down >> e & 1) ? NEG_INF : 0.0f);
   __syncthreads();
   // Wave w combines and stores dims 8 w .. 8 w + 7 of both halves' pieces: g = w of each 32 dims.
   if (e0 + col >= e1) return;

@@ -7,6 +7,8 @@ final hidden states within 2e-2 relative per real token (||gpu - ref|| / ||ref||
 """
 from __future__ import annotations
 
+import json
+
 import numpy as np
 
 from sys1rust_amd.decode import decode_answers
@@ -178,3 +180,27 @@ def random_batch(rng, vocab: int, pad_id: int) -> Batch:
         mp[r, :k] = np.sort(rng.choice(ln, size=k, replace=False))
     return Batch(n, L, kmax, ids.reshape(-1), am.reshape(-1), lens.astype(np.uint64), mp.reshape(-1), mc,
                  rng.integers(0, 3, size=n).astype(np.uint32))
+
+
+def local_model(layers: int = 1):
+    """A small model of local layers alone (window 16 to each side): config, agent, weights."""
+    from sys1rust_amd.backend import synth_checkpoint
+    from sys1rust_amd.workloads import AGENT, small_config
+
+    cfg = small_config(layers=layers, vocab=1024, local_attention=32)
+    cfg.update(pad_token_id=1002, layer_types=["sliding_attention"] * layers)
+    return cfg, AGENT, synth_checkpoint(json.dumps(cfg), json.dumps(AGENT), seed=21, scorer_width=256)
+
+
+def with_embedding(st: bytes, token: int, value: float) -> bytes:
+    """The checkpoint with every element of a token's embedding replaced."""
+    import struct
+
+    n = struct.unpack("<Q", st[:8])[0]
+    t = json.loads(st[8:8 + n])["encoder.embeddings.tok_embeddings.weight"]
+    assert t["dtype"] == "BF16"
+    d, out = t["shape"][1], bytearray(st)
+    at = 8 + n + t["data_offsets"][0] + token * d * 2
+    bits = np.float32(value).reshape(1).view(np.uint32)[0] >> 16
+    out[at:at + d * 2] = np.full(d, bits, np.uint16).tobytes()
+    return bytes(out)

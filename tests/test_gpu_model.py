@@ -137,6 +137,42 @@ def test_encoder_hidden_far_padding_tiles(small_model, settings):
     m.close()
 
 
+@pytest.mark.parametrize("settings", ["", "mask=bool,dense_upto=0", "band=1,fuserope,dtype=f16", "dtype=f32"])
+def test_far_padding_ignores_nonfinite_keys_it_does_not_name(settings):
+    """A token whose value is NaN (one local layer): in the row before a far padding query's own, which the
+    kernel's aligned loads reach; among the real tokens; and among the padding, where only some queries of
+    a tile name it. Far queries that do not (those whose result does not depend on the token) keep
+    their bits."""
+    from gates import local_model, with_embedding
+
+    cfg, agent, st = local_model()
+    W, L = cfg["local_attention"] // 2, 133
+    lens, at = [L, 4, 50, 3], [L - 1, 70, 10, 130]
+    n = len(lens)
+    rng = np.random.default_rng(23)
+    ids = rng.integers(10, 1000, (n, L)).astype(np.uint32)
+    am = (np.arange(L)[None, :] < np.array(lens)[:, None]).astype(np.uint32)
+    far = np.arange(L)[None, :] >= np.array([l if "bool" in settings else l + W for l in lens])[:, None]
+    m = HipBackend(with_embedding(st, 7, np.nan), json.dumps(cfg), json.dumps(agent), settings=settings)
+
+    def hidden(rows, token):
+        x = ids.copy()
+        for r in rows:
+            x[r, at[r]] = token
+        return m.encoder_hidden(Batch(n, L, 0, x.reshape(-1), am.reshape(-1), np.array(lens, np.uint64),
+                                      np.zeros(0, np.uint32), np.zeros(n, np.uint64), np.zeros(n, np.uint32))).reshape(n, L, -1)
+
+    for rows in ([0], [1], [2], [3], [0, 1, 2, 3]):
+        say(f"far padding {settings!r}: NaN in rows {rows}")
+        one, other, nan = hidden(rows, 8), hidden(rows, 9), hidden(rows, 7)
+        sees = (one != other).any(-1)
+        changed = (one != nan).any(-1)
+        assert bool((far & ~sees).any()) and (len(rows) == 1 or bool((far & sees).any()))
+        assert int((changed & far & ~sees).sum()) == 0
+        assert int((np.isfinite(nan).all(-1) & far & sees).sum()) == 0
+    m.close()
+
+
 @pytest.mark.parametrize("rows", [31, 32, 33, 130])
 def test_encoder_hidden_download_pieces(small_model, rows):
     """encoder_hidden's output around the size from which it is downloaded in 2 MiB pieces by several
