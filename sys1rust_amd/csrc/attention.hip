@@ -977,7 +977,7 @@ __global__ __launch_bounds__(256) void attn_far_kernel(FallbackArgs a) {
   const float sl2 = a.scale * 1.4426950408889634f;
   // Repeated keys: the weight of n copies is exp2(s + log2 n).
   const int klo = f0.y, khi = (f1.x > f0.w ? f1.x : f0.z) - 1;
-  const float llo = __builtin_amdgcn_logf(float(1 + f1.y)), lhi = __builtin_amdgcn_logf(float(1 + f1.z));
+  const float llo = log2f(float(1 + f1.y)), lhi = log2f(float(1 + f1.z));
   float m = NEG_INF, l = 0.0f;
   f32x16 o[2];
 #pragma unroll
@@ -1058,7 +1058,7 @@ __global__ __launch_bounds__(256) void attn_far_kernel(FallbackArgs a) {
   }
   l = half_sum(l);
   if (wave == 0 && f1.w > 0) {  // zero slots: score 0, value 0, weight `zeros`
-    const float sz = __builtin_amdgcn_logf(float(f1.w));
+    const float sz = log2f(float(f1.w));
     const float mn = fmaxf(m, sz);
     const float alpha = __builtin_amdgcn_exp2f(m - mn);
     l = l * alpha + __builtin_amdgcn_exp2f(sz - mn);
