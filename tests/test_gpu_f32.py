@@ -298,3 +298,34 @@ def test_f32_wide_operand_range(span):
            ((outs[0][0], outs[1][0]), (outs[0][1].pooled, outs[1][1].pooled), (outs[0][1].logits, outs[1][1].logits))]
     say(f"f32 operands over 2^{2 * span}: hidden, pooled, logits rel {rel}")
     assert max(rel) <= 2e-5, rel
+
+
+@pytest.mark.parametrize("rows,length", [(3, 33), (6, 97), (24, 97), (70, 130)])
+def test_f32_nonfinite_keys_stay_in_their_window(rows, length):
+    """A token whose value is NaN, within and at both sides of the 32-key tiles (one local layer, window
+    16; 32-, 64- and 128-query work tiles): the queries that see it get no finite result, and every
+    other one the same bits as with any other token in its place."""
+    from gates import local_model, with_embedding
+    from sys1rust_amd.workloads import Batch
+
+    cfg, agent, st = local_model()
+    W = cfg["local_attention"] // 2
+    rng = np.random.default_rng(rows)
+    ids = rng.integers(10, 1000, (rows, length)).astype(np.uint32)
+    at = rng.integers(0, length, rows)
+    at[:3] = (0, min(31, length - 1), length - 1)
+
+    def batch(token):
+        x = ids.copy()
+        x[np.arange(rows), at] = token
+        return Batch(rows, length, 0, x.reshape(-1), np.ones(x.size, np.uint32), np.full(rows, length, np.uint64),
+                     np.zeros(0, np.uint32), np.zeros(rows, np.uint64), np.zeros(rows, np.uint32))
+
+    m = HipBackend(with_embedding(st, 7, np.nan), json.dumps(cfg), json.dumps(agent), settings="dtype=f32", device=0)
+    say(f"f32 NaN keys in {rows} rows of {length}")
+    plain, nan = (m.encoder_hidden(batch(t)).reshape(rows, length, -1) for t in (8, 7))
+    sees = np.abs(np.arange(length)[None, :] - at[:, None]) <= W
+    changed = (plain != nan).any(-1)
+    assert int((changed & ~sees).sum()) == 0
+    assert int((np.isfinite(nan).all(-1) & sees).sum()) == 0
+    m.close()
