@@ -526,6 +526,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
         *reinterpret_cast<uint2*>(st + (qh * 32 + col) * 64 + ((dt * 4 + g) ^ (col & 7)) * 8 + hl * 4) = w;
       }
   }
+  wave_lds_fence();
 #pragma unroll
   for (int i = 0; i < QH * 4; ++i) {
     const int r = i * 8 + r8;
@@ -720,6 +721,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
       *reinterpret_cast<uint2*>(st + col * 64 + ((dt * 4 + g) ^ (col & 7)) * 8 + hl * 4) =
           make_uint2(E::pack2(o[dt][g * 4 + 0] * inv, o[dt][g * 4 + 1] * inv),
                      E::pack2(o[dt][g * 4 + 2] * inv, o[dt][g * 4 + 3] * inv));
+  wave_lds_fence();
   const int r8 = lane >> 3, slot = lane & 7;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {

@@ -94,6 +94,14 @@ __device__ __forceinline__ void store4_split(void* m, size_t e, const float* v, 
   *reinterpret_cast<uint2*>(o + 32) = make_uint2(lo[0], lo[1]);
 }
 
+// Between LDS writes and reads of what other lanes of the same wave wrote: a wave's LDS accesses take
+// effect in order, so this only keeps the compiler, which knows one lane's accesses, from reordering them.
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // 8 elements of type E held in a uint4 <-> floats.
 template <class E>
 __device__ __forceinline__ void unpack8(const uint4& v, float* f) {
