@@ -195,7 +195,8 @@ int s1k_split_rope(const void* qkv, int M, int d, const int32_t* pos, double the
 
 /* Attention over packed rows: q, k [H, T, 64] bf16, v transposed [H, 64, v_ld] bf16 (v_ld >=
  * T rounded up to 8, plus 64), seq_starts [nseq + 1] int32 (host memory), window < 0 for
- * global, else |i - j| <= window; out [T, H*64] bf16. */
+ * global, else |i - j| <= window; out [T, H*64] bf16. q, k and v are aligned to 16 bytes, out
+ * to 8. */
 int s1k_attention(const void* q, const void* k, const void* v, int v_ld, int T, int H,
                   const int32_t* seq_starts, int nseq, int window, float scale, void* out,
                   void* stream);

@@ -318,6 +318,10 @@ void attn_kernel(AttnArgs a) {
     }
 }
 
+// 16 bytes of a result row: a caller's out is aligned to 8 only.
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef u32x4 u32x4_a8 __attribute__((aligned(8)));
+
 // Global layers of batches that fill the GPU: a wave owns 64 queries, as two halves of 32, and a
 // workgroup of 4 waves the same 256 queries that 8 waves of 32 would. Each K and V^T fragment read
 // from LDS then feeds two MFMAs, and half 1's softmax weights are computed beside half 0's V^T P^T
@@ -530,8 +534,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
 #pragma unroll
   for (int i = 0; i < QH * 4; ++i) {
     const int r = i * 8 + r8;
-    const uint4 v = *reinterpret_cast<const uint4*>(st + r * 64 + (slot ^ (r & 7)) * 8);
-    if (wq0 + r < tl.q1) *reinterpret_cast<uint4*>(a.out + size_t(wq0 + r) * a.ldo + head * 64 + slot * 8) = v;
+    const u32x4 v = *reinterpret_cast<const u32x4*>(st + r * 64 + (slot ^ (r & 7)) * 8);
+    if (wq0 + r < tl.q1) *reinterpret_cast<u32x4_a8*>(a.out + size_t(wq0 + r) * a.ldo + head * 64 + slot * 8) = v;
   }
 }
 
@@ -726,8 +730,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void a
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int r = i * 8 + r8;
-    const uint4 v = *reinterpret_cast<const uint4*>(st + r * 64 + (slot ^ (r & 7)) * 8);
-    if (wq0 + r < tl.q1) *reinterpret_cast<uint4*>(a.out + size_t(wq0 + r) * a.ldo + head * 64 + slot * 8) = v;
+    const u32x4 v = *reinterpret_cast<const u32x4*>(st + r * 64 + (slot ^ (r & 7)) * 8);
+    if (wq0 + r < tl.q1) *reinterpret_cast<u32x4_a8*>(a.out + size_t(wq0 + r) * a.ldo + head * 64 + slot * 8) = v;
   }
 }
 

@@ -308,7 +308,7 @@ def attention_ref(q, k, v, starts, window, scale):
 @pytest.mark.parametrize("window", [-1, 64, 16, 100])
 @pytest.mark.parametrize("lens", [[1, 37, 129, 300, 600], [8, 200], [700, 1], [513], [2048], [5, 3, 250, 1, 700, 9],
                                   [600] * 24, [1, 2, 130, 7, 64, 600, 3] * 4])
-def test_attention_varlen(dev, window, lens):
+def test_attention_varlen(dev, window, lens, out_at=0):
     say(f"attention window={window} lens={lens}")
     H = 16
     starts = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
@@ -323,7 +323,8 @@ def test_attention_varlen(dev, window, lens):
     vt = torch.full((H, 64, ldv), -1, dtype=torch.int16, device=dev)
     vt[:, :, :T] = vb.transpose(1, 2)
     vt[:, :, T:(T + 7) // 8 * 8] = 0
-    out = torch.zeros(T, H * 64, dtype=torch.int16, device=dev)
+    buf = torch.full((T * H * 64 + 8,), 77, dtype=torch.int16, device=dev)
+    out = buf[out_at:out_at + T * H * 64].view(T, H * 64).zero_()
     st = np.ascontiguousarray(starts)
     L.check(L.lib().s1k_attention(ptr(qb), ptr(kb), ptr(vt), ldv, T, H, st.ctypes.data_as(L.i32p), len(lens),
                                   window, 0.125, ptr(out), stream()))
@@ -334,6 +335,14 @@ def test_attention_varlen(dev, window, lens):
     err = (got - ref).abs()
     assert float(err.max()) <= 2e-2, float(err.max())
     assert float(err.mean()) <= 2e-3, float(err.mean())
+    assert bool((buf[:out_at] == 77).all()) and bool((buf[out_at + T * H * 64:] == 77).all())
+
+
+# out at 8 bytes from a 16-byte boundary: tiles of 256, 128 and 32 queries, global and local
+@pytest.mark.parametrize("window", [-1, 64])
+@pytest.mark.parametrize("lens", [[600] * 24 + [7], [513, 300], [40, 9]])
+def test_attention_out_aligned_to_8(dev, window, lens):
+    test_attention_varlen(dev, window, lens, out_at=4)
 
 
 # 256-query tiles of the global kernel (at least 16 of them with 16 heads): rows that end at, before
