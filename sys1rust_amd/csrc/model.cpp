@@ -709,6 +709,14 @@ void Model::upload(const Plan& p) {
   hip_check(hipMemcpyAsync(dmeta, hmeta, bytes, hipMemcpyHostToDevice, stream), "upload batch");
 }
 
+// Whether p is plain host memory, which the GPU's copies cannot reach by themselves.
+static bool pageable(const void* p) {
+  hipPointerAttribute_t a{};
+  if (hipPointerGetAttributes(&a, p) == hipSuccess) return a.type == hipMemoryTypeUnregistered;
+  (void)hipGetLastError();  // a pointer the runtime does not know
+  return true;
+}
+
 // The runtime's own copy to pageable memory moves a piece at a time: DMA to its pinned buffer, then one
 // thread's copy, which also takes the page faults of memory that the caller has just allocated. Here
 // kCopiers threads first touch their pieces' pages, while the GPU still computes (as an OR with 0, so
@@ -717,9 +725,9 @@ void Model::upload(const Plan& p) {
 // 20.7 MB (encoder_hidden of 5064 positions, d 1024), the whole call: 2170 -> 1332 us, of which the GPU
 // computes 650. With pieces of 1 MiB 1415
 // (12 us between two copies), 1323 at 4; 6 or 8 threads 1320-1340. Below two pieces the threads' start
-// costs more than they save.
+// costs more than they save, and pinned memory takes the copy directly.
 void Model::download(void* dst, const void* src, size_t bytes, const char* what) {
-  if (bytes < 2 * kPiece) {
+  if (bytes < 2 * kPiece || !pageable(dst)) {
     hip_check(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream), what);
     hip_check(hipStreamSynchronize(stream), what);
     return;

@@ -20,9 +20,11 @@ from pathlib import Path
 
 import numpy as np
 import pytest
+import torch
 
 from oracle import oracle as O
-from sys1rust_amd.backend import DEFAULT_TUNING, HipBackend, S1Error, synth_checkpoint
+from sys1rust_amd import _lib
+from sys1rust_amd.backend import DEFAULT_TUNING, HipBackend, S1Error, _batch_arrays, check, synth_checkpoint
 from sys1rust_amd.decode import ActHead
 from sys1rust_amd.workloads import AGENT, MODERNBERT_LARGE, Batch, workload
 
@@ -178,7 +180,8 @@ def test_encoder_hidden_download_pieces(small_model, rows):
     """encoder_hidden's output around the size from which it is downloaded in 2 MiB pieces by several
     threads (4 MiB), and past a second round of pieces: every row is that of the batch of one, alone,
     wherever its piece falls, within the 16-bit layers' gate (a batch may take other tiles), and the same
-    call again is the same bits."""
+    call again is the same bits, also into pinned memory (a copy of its own) and at an odd offset into
+    plain memory, with nothing written beside it."""
     cfg, agent, st, _, _ = small_model
     d, L = cfg["hidden_size"], (4 << 20) // 4 // 32 // cfg["hidden_size"]
     rng = np.random.default_rng(5)
@@ -189,6 +192,13 @@ def test_encoder_hidden_download_pieces(small_model, rows):
     say(f"download of {rows} rows x {L} x {d}")
     hid = m.encoder_hidden(batch(ids)).reshape(rows, L, d)
     assert np.array_equal(hid, m.encoder_hidden(batch(ids)).reshape(rows, L, d))
+    args = _batch_arrays(batch(ids))
+    for buf in (torch.full((hid.size + 8,), 5.0).pin_memory(), torch.full((hid.size + 8,), 5.0)):
+        out = buf.numpy()
+        check(_lib.lib().s1_encoder_hidden(m._h, rows, L, 0, *(a.ctypes.data_as(_lib.u64p if a.dtype == np.uint64 else _lib.u32p)
+                                                               for a in args), out[3:].ctypes.data_as(_lib.f32p)))
+        assert np.array_equal(out[3:3 + hid.size], hid.reshape(-1))
+        assert (out[:3] == 5.0).all() and (out[3 + hid.size:] == 5.0).all()
     for r in (0, rows // 2, rows - 1):
         one = m.encoder_hidden(batch(ids[r: r + 1])).reshape(L, d)
         rel = np.linalg.norm(hid[r] - one, axis=-1) / np.linalg.norm(one, axis=-1)
