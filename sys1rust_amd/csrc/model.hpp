@@ -161,11 +161,12 @@ struct Model {
   size_t hout_cap = 0;
   int* dmeta = nullptr;
   size_t dmeta_cap = 0;
-  // pinned staging of a large download: a piece for each of kCopiers threads
+  // pinned staging of a large download: a piece and an event for each of kCopiers threads, and an
+  // event for the end of the work before it
   static constexpr size_t kPiece = size_t(2) << 20;
   static constexpr int kCopiers = 4;
   void* hring = nullptr;
-  hipEvent_t ring_ev[kCopiers] = {};
+  hipEvent_t ring_ev[kCopiers + 1] = {};
 
   // per-kernel timing (Settings::ops)
   struct OpRec {
