@@ -1154,20 +1154,27 @@ int attn_global_tile(const int* row_start, int n, int heads) { return global_til
 int attn_plan_tiles(const int* row_start, int n, int heads, int window, std::vector<int>& out, const int* q_end,
                     const int* k_end) {
   const int qb = window >= 0 ? local_tile(row_start, q_end, n, heads, window) : global_tile(row_start, q_end, n, heads);
-  std::vector<AttnTile> tiles;
+  const size_t first = out.size();
   for (int r = 0; r < n; ++r) {
     const int rs = row_start[r], qe = q_end ? q_end[r] : row_start[r + 1], ke = k_end ? k_end[r] : row_start[r + 1];
     const int step = attn_row_step(qe - rs, qb);
     for (int q0 = rs; q0 < qe; q0 += step) {
       const int q1 = std::min(q0 + step, qe);
       const bool win = window >= 0 && qb == 32;
-      tiles.push_back({q0, q1, win ? std::max(rs, q0 - window) : rs, win ? std::min(ke, q1 + window) : ke});
+      out.push_back(q0);
+      out.push_back(q1);
+      out.push_back(win ? std::max(rs, q0 - window) : rs);
+      out.push_back(win ? std::min(ke, q1 + window) : ke);
     }
   }
-  if (window < 0 && qb == WQ)  // attn_wide_kernel: most keys first
+  if (window < 0 && qb == WQ) {  // attn_wide_kernel: most keys first
+    std::vector<AttnTile> tiles;
+    for (size_t i = first; i < out.size(); i += 4) tiles.push_back({out[i], out[i + 1], out[i + 2], out[i + 3]});
     std::stable_sort(tiles.begin(), tiles.end(),
                      [](const AttnTile& x, const AttnTile& y) { return x.k1 - x.k0 > y.k1 - y.k0; });
-  for (const AttnTile& t : tiles) out.insert(out.end(), {t.q0, t.q1, t.k0, t.k1});
+    out.resize(first);
+    for (const AttnTile& t : tiles) out.insert(out.end(), {t.q0, t.q1, t.k0, t.k1});
+  }
   return qb;
 }
 
