@@ -62,7 +62,8 @@ constexpr size_t kMaxSpan = (size_t(1) << 32) - 1;
 // as one 8-byte (bf16) or 16-byte (f32) access after a packed conversion. !TR: D = A . W^T, a
 // lane holds one column and four consecutive rows per g; only the transposed v output of the
 // q|k|v epilogue ([H, 64, ldv], rows = tokens contiguous) wants that.
-template <class E, int BM, int BN, int BK, int STAGES, int WM, int WN, int EPI, bool TR, int KG, bool PIPE = false>
+template <class E, int BM, int BN, int BK, int STAGES, int WM, int WN, int EPI, bool TR, int KG, bool PIPE = false,
+          bool ODDK = false>
 __device__ __forceinline__ void gemm_tile(const GemmArgs& g, char* smem0, int m0, int n0, int kt0, int NK, int split) {
   constexpr int NW = WM * WN;                // waves; each owns a TM x TN sub-tile
   constexpr int TM = BM / WM, TN = BN / WN;
@@ -80,15 +81,20 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, char* smem0, int m0
   static_assert((STAGES - 2) * LPW < 64, "vmcnt range");
 
   // KG > 1 (k-groups): the workgroup holds KG groups of NW waves; group k runs k-tiles
-  // [kt0 + k NK / KG, kt0 + (k + 1) NK / KG) on stage buffers of its own (a group with a k-tile
-  // less passes the last one's barrier all the same), and group 0 adds the other groups' accumulators, in
+  // [kt0 + k NK / KG, kt0 + (k + 1) NK / KG) on stage buffers of its own, and group 0 adds the
+  // other groups' accumulators, in
   // group order, from LDS and runs the epilogue alone. A short GEMM's chain of dependent k-tiles
-  // is then KG times shorter on the same tiles.
+  // is then KG times shorter on the same tiles. NK divides by KG, so that every group passes the same
+  // barriers, or with ODDK need not: a group with a k-tile less passes the last one's barrier all the
+  // same (a kernel of its own, since the uneven ranges cost each launch of the even one 0.06 µs).
   const int grp = KG > 1 ? __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6) / NW : 0;
   const int tid = threadIdx.x - grp * NW * 64;
   char* const smem = smem0 + grp * STAGES * STAGE_BYTES;
   const int NKmax = (NK + KG - 1) / KG;
-  if constexpr (KG > 1) {
+  if constexpr (KG > 1 && !ODDK) {
+    kt0 += grp * (NK / KG);
+    NK /= KG;
+  } else if constexpr (KG > 1) {
     const int b = grp * NK / KG;
     kt0 += b;
     NK = (grp + 1) * NK / KG - b;
@@ -266,7 +272,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, char* smem0, int m0
   }
 
   if constexpr (KG > 1) {
-    if (NK < NKmax) barrier_lds();
+    if (ODDK && NK < NKmax) barrier_lds();
     // Groups 1.. leave their accumulators in their own stage buffers, in register order (float4
     // e4 of fragment (i, j) of wave w at ((w FM + i) FN + j) 4 + e4, 64 lanes apart), and end;
     // waves that have ended take no part in the barriers that follow.
@@ -601,7 +607,7 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, char* smem0, int m0
   }
 }
 
-template <class E, int BM, int BN, int BK, int STAGES, int WM, int WN, int EPI, int KG, bool PIPE = false>
+template <class E, int BM, int BN, int BK, int STAGES, int WM, int WN, int EPI, int KG, bool PIPE = false, bool ODDK = false>
 __global__ __launch_bounds__(WM * WN * 64 * KG) void gemm_kernel(GemmArgs g) {
   // STAGES k-tiles of A [BM][BK] and W [BN][BK], bf16, rows of BK * 2 bytes. The 16-byte chunk c
   // of row r sits at slot c ^ ((r / SW) % CH): the 16 lanes of one LDS access phase (16
@@ -632,17 +638,18 @@ __global__ __launch_bounds__(WM * WN * 64 * KG) void gemm_kernel(GemmArgs g) {
 
   if constexpr (EPI == EPI_ROPE) {
     if (n0 >= 2 * g.rope_d) {
-      gemm_tile<E, BM, BN, BK, STAGES, WM, WN, EPI, false, KG>(g, smem, m0, n0, kt0, NK, split);
+      gemm_tile<E, BM, BN, BK, STAGES, WM, WN, EPI, false, KG, false, ODDK>(g, smem, m0, n0, kt0, NK, split);
       return;
     }
   }
-  gemm_tile<E, BM, BN, BK, STAGES, WM, WN, EPI, true, KG, PIPE>(g, smem, m0, n0, kt0, NK, split);
+  gemm_tile<E, BM, BN, BK, STAGES, WM, WN, EPI, true, KG, PIPE, ODDK>(g, smem, m0, n0, kt0, NK, split);
 }
 
-template <class E, int BM, int BN, int BK, int STAGES, int WM, int WN, int EPI, int KG = 1, bool PIPE = false>
+template <class E, int BM, int BN, int BK, int STAGES, int WM, int WN, int EPI, int KG = 1, bool PIPE = false,
+          bool ODDK = false>
 void launch_t(const GemmArgs& g, hipStream_t st) {
   const int mt = (g.M + BM - 1) / BM, nt = g.N / BN;
-  hipLaunchKernelGGL((gemm_kernel<E, BM, BN, BK, STAGES, WM, WN, EPI, KG, PIPE>), dim3(mt * nt, g.splits),
+  hipLaunchKernelGGL((gemm_kernel<E, BM, BN, BK, STAGES, WM, WN, EPI, KG, PIPE, ODDK>), dim3(mt * nt, g.splits),
                      dim3(WM * WN * 64 * KG), 0, st, g);
 }
 
@@ -701,9 +708,15 @@ void launch_te(const GemmArgs& g, hipStream_t st) {
       // 64 x 64 tiles fit one workgroup per CU runs them in two k-groups (8 k-tiles each where
       // there were 16): at 174 tokens q|k|v 9.9 -> 8.9 µs and GeGLU 9.8 -> 8.2 µs (GeGLU on twice
       // the workgroups of its 64 x 128 tiles), weights cold in HBM; a residual product of 563 x
-      // 1024 x 2624, a chain of 41 k-tiles on 72 CUs before, 18.5 -> 12.4 µs.
+      // 1024 x 2624, a chain of 41 k-tiles on 72 CUs before, 18.5 -> 12.4 µs. Unsplit residual
+      // products of 300 to 1344 rows, widths 768 and 1024, K 768 to 4096, cold weights: 1.19 (1024 x
+      // 768, 800 rows) to 1.60 times as fast (768 x 4096, 450 rows), none slower.
       constexpr bool KGOK = EPI != EPI_F32;
-      if (KGOK && g.splits == 1 && g.K >= 2 * BK && (long long)((g.M + 63) / 64) * (g.N / 64) <= 256)
+      constexpr bool ODDOK = KGOK && EPI != EPI_ROPE;  // q|k|v: K = N / 3, N a multiple of 128
+      const bool kg = KGOK && g.splits == 1 && g.K >= 2 * BK && (long long)((g.M + 63) / 64) * (g.N / 64) <= 256;
+      if (ODDOK && kg && (g.K / BK) % 2)
+        launch_t<E, 64, 64, 64, 4, 2, 1, EPI, ODDOK ? 2 : 1, false, ODDOK>(g, st);
+      else if (kg)
         launch_t<E, 64, 64, 64, 4, 2, 1, EPI, KGOK ? 2 : 1>(g, st);
       else if (EPI == EPI_ROPE && (long long)((g.M + 63) / 64) * (g.N / 64) * g.splits <= 256)
         launch_t<E, 64, 64, 64, 4, 2, 1, EPI>(g, st);

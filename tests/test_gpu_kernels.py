@@ -140,6 +140,11 @@ def test_gemm_k_groups_of_any_k(dev, M, K):
     h = h0.clone()
     gemm(A, W, M, N, K, epi=1, bias=bias, C_out=h)
     assert float((h - (h0 + ref)).abs().max()) <= 2e-5 * scale + 1e-5
+    # the GeGLU epilogue on W's row blocks of 32, x and gate in turn
+    pair = (as_f32(A).double() @ as_f32(W).double().T).float().reshape(M, N // 64, 2, 32)
+    r = (torch.nn.functional.gelu(pair[:, :, 0]) * pair[:, :, 1]).reshape(M, N // 2)
+    act = as_f32(gemm(A, W, M, N, K, epi=2))
+    assert bool(((act - r).abs() <= r.abs() * 2 ** -7 + 1e-4).all())
 
 
 @pytest.mark.parametrize("M", [5686, 5000])
