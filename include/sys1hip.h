@@ -42,8 +42,9 @@ typedef struct s1_model s1_model;
  * keeps weights and activations in f16, the checkpoints' own type (BackendOptions::f32 = false,
  * backend.rs:25-27, keeps the checkpoint's f16 weights); the default `dtype=bf16` rounds them to
  * bf16. Accumulation, LayerNorm, softmax and the residual stream are f32 either way. `dtype=f32`
- * is BackendOptions::f32 = true: f32 weights and compute on plain f32 kernels (no fused kernels,
- * a numerics mode, not the serving path). */
+ * is BackendOptions::f32 = true: f32 weights, activations and sums (no fused kernels, a numerics
+ * mode, not the serving path). Its matrix products take both operands at 23 significant bits, one
+ * less than f32's, on the 16-bit matrix instructions; attention multiplies in f32. */
 int s1_model_create(const char* safetensors_path, const char* encoder_config_json,
                     const char* agent_config_json, const char* settings, int device_ordinal,
                     s1_model** out);

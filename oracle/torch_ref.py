@@ -31,6 +31,12 @@ class TorchOracle:
         self.w = {k: torch.from_numpy(np.ascontiguousarray(v)).to(self.dev) for k, v in o.w.items()}
         self.tables = {k: tuple(torch.from_numpy(t).to(self.dev) for t in v) for k, v in o.tables.items()}
 
+    def double(self) -> "TorchOracle":
+        """The same forward in float64 (encoder_hidden and forward), rounded to float32 at the end."""
+        self.w = {k: v.double() for k, v in self.w.items()}
+        self.tables = {k: tuple(t.double() for t in v) for k, v in self.tables.items()}
+        return self
+
     # ---- the oracle's helpers (oracle.layer_norm, gelu, rope, sdpa)
     @staticmethod
     def layer_norm(x, w, b, eps: float):
@@ -83,7 +89,7 @@ class TorchOracle:
             return self.sdpa(q, k, v, scale, mask[None])
         H, hd = q.shape[0], q.shape[2]
         nc = -(-L // S)
-        qp = torch.zeros((H, nc * S, hd), device=self.dev)
+        qp = torch.zeros((H, nc * S, hd), dtype=q.dtype, device=self.dev)
         qp[:, :L] = q
         qp = qp.reshape(H, nc, S, hd)
         pos = torch.from_numpy(O.window_positions(S, nc)).to(self.dev)

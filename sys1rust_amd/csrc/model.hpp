@@ -48,7 +48,7 @@ struct Settings {
   bool fuseln = true;      // a split-K Wo / Wo2 finishes in the kernel of the LayerNorm after it
   bool graphs = true;      // replay each repeated batch shape from a captured HIP graph
   bool f16 = false;        // dtype=f16: weights and activations in f16 (the checkpoint's type), not bf16
-  bool f32 = false;        // dtype=f32: f32 weights and compute (BackendOptions::f32), the plain f32 kernels
+  bool f32 = false;        // dtype=f32: f32 weights and compute (BackendOptions::f32), f32path.hip's kernels
   static Settings parse(const std::string& spec);
 };
 
