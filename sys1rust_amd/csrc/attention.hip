@@ -9,8 +9,8 @@
 // so a hard mask over the row's own keys computes the same values; padding never enters the
 // packed layout at all.
 //
-// Work split: a workgroup of NW wavefronts takes up to 32 NW queries of one sequence and one
-// head; each wave owns 32 queries (64 in attn_wide_kernel, the global layers of batches that fill
+// Work split: a workgroup of 4 wavefronts takes up to 128 queries of one sequence and one head;
+// each wave owns 32 queries (64 in attn_wide_kernel, the global layers of batches that fill
 // the GPU). Keys stream through LDS in chunks of 64 (double-buffered on global layers): K as [key][dim] and V as [dim][key], copied with 16-byte accesses from the
 // transposed v buffer. On local layers waves skip chunks, and 32-key halves, outside their
 // window, and only chunks that cross a window or row edge pay for masking. Short batches (fewer
@@ -62,10 +62,11 @@ __device__ __forceinline__ int2 tile_head(int ntiles) {
 }
 
 // Three waves per SIMD for the local kernel (register budget 168), four for the global one.
-template <class E, bool LOCAL, int NW>
-__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(LOCAL ? 3 : 4)))
+template <class E, bool LOCAL>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(LOCAL ? 3 : 4)))
 void attn_kernel(AttnArgs a) {
   typedef typename E::v8 v8;
+  constexpr int NW = 4;  // wavefronts
   // K and V^T double buffers, [K0 | K1 | V0 | V1], 8 KiB each.
   __shared__ __attribute__((aligned(1024))) uint16_t smem[4 * KC * 64];
   auto sK = [&](int buf) { return smem + buf * KC * 64; };
@@ -325,9 +326,9 @@ typedef u32x4 u32x4_a8 __attribute__((aligned(8)));
 // Global layers of batches that fill the GPU: a wave owns 64 queries, as two halves of 32, and a
 // workgroup of 4 waves the same 256 queries that 8 waves of 32 would. Each K and V^T fragment read
 // from LDS then feeds two MFMAs, and half 1's softmax weights are computed beside half 0's V^T P^T
-// products. Two waves per SIMD: by counters a SIMD spends 477k cycles on VALU issue (an exp2 costs
-// two FMAs) and 262k on MFMAs at 8192 keys and 16 heads, and at equal priority a launch took their
-// sum. The priority raised over the weights and the V^T P^T products lets one wave's vector work
+// products. Two waves per SIMD: by counters a SIMD spends 475k cycles on VALU issue (an exp2 costs
+// two FMAs) and 262k on MFMAs at 8192 keys and 16 heads; at equal priority a launch took their
+// sum, 709k (counted before V^T went through registers), and takes 592k now. The priority raised over the weights and the V^T P^T products lets one wave's vector work
 // go ahead while the other's K Q^T products run (raised over K Q^T, or from the row maximum on, it
 // gains nothing). With this and the order of the tiles, against 8 waves of 32 queries, 16 heads:
 // 8192 keys 336 -> 310 µs (890 TFLOP/s), 10 rows of 547 to 579 tokens 34.1 -> 30.6, 12 of 300 to
@@ -958,7 +959,7 @@ __global__ __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
 // is the lane's own weight). Loads go straight to registers: the sets are a few hundred keys that
 // the tiles of a row share through L2, and what bounds the kernel is each wave's chain of about
 // three key tiles. Measured at 1780 entries of 64 to 320 keys, 16 heads, against one wave per
-// (entry, head) on vector FMAs: 156 -> 21.3 us at 1780 entries.
+// (entry, head) on vector FMAs: 156 -> 22.4 us (20.9 without the care for values that are not finite).
 template <class E>
 __global__ __launch_bounds__(256) void attn_far_kernel(FallbackArgs a) {
   typedef typename E::v8 v8;
@@ -1186,11 +1187,11 @@ void attn_launch_t(const AttnArgs& a, hipStream_t st) {
   else if (a.window >= 0 && a.window <= LMAXW && !a.qkey)
     hipLaunchKernelGGL(attn_local_kernel<E>, grid, dim3(256), 0, st, a);  // tiles of <= LQ queries
   else if (a.window >= 0)
-    hipLaunchKernelGGL((attn_kernel<E, true, 4>), grid, dim3(256), 0, st, a);
+    hipLaunchKernelGGL((attn_kernel<E, true>), grid, dim3(256), 0, st, a);
   else if (a.tile_q == 256)
     hipLaunchKernelGGL(attn_wide_kernel<E>, grid, dim3(256), 0, st, a);
   else if (a.tile_q == 128)
-    hipLaunchKernelGGL((attn_kernel<E, false, 4>), grid, dim3(256), 0, st, a);
+    hipLaunchKernelGGL((attn_kernel<E, false>), grid, dim3(256), 0, st, a);
   else if (a.key_waves == 8)  // tile_q 32
     hipLaunchKernelGGL((attn_ksplit_kernel<E, 8, false>), grid, dim3(512), 0, st, a);
   else

@@ -548,9 +548,9 @@ Plan Model::plan(uint32_t n, uint32_t len, uint32_t kmax, const uint32_t* ids, c
     while (m.size() % 4) m.push_back(0);
   };
   pad4();
-  // Attention work tiles: query blocks of one row; for global layers 256 queries (one workgroup
-  // of 8 waves), or 128 or 32 for a short batch; for local ones 128 (4 waves; their keys are only
-  // the window), or 32 for a short batch.
+  // Attention work tiles: query blocks of one row; for global layers 256 queries (4 waves of 64),
+  // or 128 or 32 for a short batch; for local ones 128 (4 waves; their keys are only
+  // the window), or 32 for a short batch. (attn32_plan_tiles has sizes of its own.)
   p.off_tiles = m.size();
   const auto tiles = set.f32 ? attn32_plan_tiles : attn_plan_tiles;
   p.gq = tiles(p.row_start.data(), int(n), cfg.heads, -1, m, nullptr, nullptr);
@@ -1471,7 +1471,8 @@ Gemm32Args parts_of(Gemm32Args g) {
 // activations a bound that holds for every input. A LayerNorm's output is z * w + b with
 // |z|_2 <= sqrt(d), so each element and each product of it with a weight row is bounded
 // (weight_bound_launch); attention returns averages of v rows; |gelu(x) g| <= |x| |g|. Operands that stay
-// far below their bound lose nothing: a split value keeps f32's precision down to 2^-27 of it.
+// far below their bound lose nothing further: a split value keeps its 23 bits down to 2^-27 of it. (Bounds
+// outside 2^-40 to 2^60 take the scale of the nearer end.)
 void Model::split_weights32() {
   const int d = cfg.d, I = cfg.inter;
   const size_t most = size_t(std::max({3 * d, 2 * I, 4 * d, scorer_width}));
@@ -1615,7 +1616,8 @@ void Model::forward32(const Plan& p, float* logits_out, float* pooled_out) {
     layernorm_launch(a.h, nullptr, final_norm, nullptr, float(cfg.eps), T, d, nullptr, a.enc, type_emb, dmeta + p.off_seg,
                      a.hh, stream, elem);
   });
-  // head_forward (lib.rs:1698-1765): pre-norm layers with biases, ReLU FFN, every row
+  // head_forward (lib.rs:1698-1765): pre-norm layers with biases, ReLU FFN, over every row up to the
+  // last layer's keys and values
   for (int j = 0; j < cfg.head_layers; ++j) {
     const HeadWeights& Hw = head[j];
     if (j == 0)
