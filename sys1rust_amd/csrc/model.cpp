@@ -722,13 +722,14 @@ static bool pageable(const void* p) {
 // The runtime's own copy to pageable memory moves a piece at a time: DMA to its pinned buffer, then one
 // thread's copy, which also takes the page faults of memory that the caller has just allocated. Here
 // kCopiers threads first touch their pieces' pages, while the GPU still computes (as an OR with 0, so
-// that a call that fails leaves the caller's bytes), and then each waits
-// for its pieces in turn and copies them out of its pinned buffer while the others' are on their way.
-// While the GPU computes only the calling thread waits in the runtime; the others sleep.
-// 20.7 MB (encoder_hidden of 5064 positions, d 1024), the whole call: 2170 -> 1332 us, of which the GPU
-// computes 650. With pieces of 1 MiB 1415
-// (12 us between two copies), 1323 at 4; 6 or 8 threads 1320-1340. Below two pieces the threads' start
-// costs more than they save, and pinned memory takes the copy directly.
+// that a call that fails leaves the caller's bytes), and then each waits for its pieces in turn and
+// copies them out of its pinned buffer while the others' are on their way. While the GPU computes only
+// the calling thread waits in the runtime; the others sleep. 20.7 MB (encoder_hidden of 5064 positions,
+// d 1024), the whole call: 2170 -> 1332 us, of which the GPU computes 650, and 2.3 -> 2.9 ms of CPU time; a
+// handle's first call gains 4 to 8%, since it allocates the pieces and memory that is new to the process
+// takes its page faults. With pieces of 1 MiB 1415 us (12 us between two copies), 1323 at 4; 6 or 8 threads
+// 1320-1340. Below two pieces the threads' start costs more than they save, and pinned memory takes
+// the copy directly (1290 -> 1054).
 void Model::download(void* dst, const void* src, size_t bytes, const char* what) {
   if (bytes < 2 * kPiece || !pageable(dst)) {
     hip_check(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream), what);
