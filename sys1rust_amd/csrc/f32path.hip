@@ -156,11 +156,11 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm32_kernel(Gemm32Args g) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         float4* o = reinterpret_cast<float4*>(orow + j * 32 + q * 8);
-        const float4 inv = *reinterpret_cast<const float4*>(g.inv + n0 + wn * TN + 4 * lh + j * 32 + q * 8);
-        const float iv[4] = {inv.x, inv.y, inv.z, inv.w};
+        const int4 wexp = *reinterpret_cast<const int4*>(g.wexp + n0 + wn * TN + 4 * lh + j * 32 + q * 8);
+        const int ex[4] = {wexp.x + g.aexp, wexp.y + g.aexp, wexp.z + g.aexp, wexp.w + g.aexp};
         float v[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) v[r] = fmaf(acx[i][j][4 * q + r], 1.0f / 2048.0f, acc[i][j][4 * q + r]) * iv[r];
+        for (int r = 0; r < 4; ++r) v[r] = ldexpf(fmaf(acx[i][j][4 * q + r], 1.0f / 2048.0f, acc[i][j][4 * q + r]), ex[r]);
         if (!part) {
           if (g.bias) {
             const float4 b = *reinterpret_cast<const float4*>(g.bias + n0 + wn * TN + 4 * lh + j * 32 + q * 8);
@@ -220,17 +220,18 @@ __global__ __launch_bounds__(256) void splitk32_kernel(Gemm32Args g) {
 
 // A weight matrix into split f32 in place, each row times the power of two that puts its largest
 // element (bounds[2 row]) at 2^14 to 2^15: a wave reads its 64 elements of one row, then writes their
-// bytes. inv[row] undoes the row's scale and the input's.
+// bytes. wexp[row] is the exponent that undoes the row's scale.
 __global__ __launch_bounds__(256) void split_weight_kernel(float* w, size_t n, int K, const float* __restrict__ bounds,
-                                                           float a, float* __restrict__ inv) {
+                                                           int* __restrict__ wexp) {
   const size_t e = size_t(blockIdx.x) * 256 + threadIdx.x;
   if (e >= n) return;
   const size_t row = e / K;
   const float m = bounds[2 * row];
   int ex = 0;
   if (m > 0.0f && m < __builtin_huge_valf()) (void)frexpf(m, &ex);
-  const float sc = ldexpf(1.0f, 15 - min(max(ex, -40), 60));  // products of two scales stay normal
-  if (e % K == 0) inv[row] = 1.0f / (sc * a);
+  ex = max(ex, -111) - 15;  // the scale is at most 2^126
+  const float sc = ldexpf(1.0f, -ex);
+  if (e % K == 0) wexp[row] = ex;
   const float x[2] = {w[e], 0.0f};
   uint32_t hi, lo;
   split_f16<2>(x, sc, &hi, &lo);
@@ -240,24 +241,31 @@ __global__ __launch_bounds__(256) void split_weight_kernel(float* w, size_t n, i
 }
 
 // One wave per row of W (weight_bound_launch): |W_r . (z * lw + lb) + bias| <= sqrt(K) |W_r * lw|_2 +
-// |W_r . lb + bias| by the Cauchy-Schwarz inequality.
+// |W_r . lb + bias| by the Cauchy-Schwarz inequality. The squares are taken of elements scaled by their largest.
 __global__ __launch_bounds__(64) void weight_bound_kernel(const float* __restrict__ W, const float* __restrict__ lw,
                                                           const float* __restrict__ lb, const float* __restrict__ bias, int K,
                                                           float* __restrict__ out) {
   const float* row = W + size_t(blockIdx.x) * K;
-  float mx = 0.0f, sq = 0.0f, dot = 0.0f;
+  float mx = 0.0f, most = 0.0f, sq = 0.0f, dot = 0.0f;
   for (int k = threadIdx.x; k < K; k += 64) {
-    const float w = row[k], x = lw ? w * lw[k] : w;
+    const float w = row[k];
     mx = fmaxf(mx, fabsf(w));
-    sq = fmaf(x, x, sq);
+    most = fmaxf(most, fabsf(lw ? w * lw[k] : w));
     if (lb) dot = fmaf(w, lb[k], dot);
   }
   mx = wave_max(mx);
-  sq = wave_sum(sq);
+  most = wave_max(most);
   dot = wave_sum(dot);
+  int ex = 0;
+  if (most > 0.0f && most < __builtin_huge_valf()) (void)frexpf(most, &ex);
+  for (int k = threadIdx.x; k < K; k += 64) {
+    const float x = ldexpf(lw ? row[k] * lw[k] : row[k], -ex);
+    sq = fmaf(x, x, sq);
+  }
+  sq = wave_sum(sq);
   if (threadIdx.x) return;
   out[2 * blockIdx.x] = mx;
-  out[2 * blockIdx.x + 1] = sqrtf(float(K)) * sqrtf(sq) + fabsf(dot + (bias ? bias[blockIdx.x] : 0.0f));
+  out[2 * blockIdx.x + 1] = ldexpf(sqrtf(float(K)) * sqrtf(sq), ex) + fabsf(dot + (bias ? bias[blockIdx.x] : 0.0f));
 }
 
 // qkv [T, 3d] -> q, k, v [H, T, 64], with the half-split RoPE rotation of q and k at pos[t] when
@@ -608,7 +616,7 @@ const char* gemm32_check(const Gemm32Args& g) {
   if (g.K % 32 || g.N % 128 || g.lda % 32 || g.ldw % 32 || g.ldc % 32) return "f32 GEMM: K and leading dimensions must be multiples of 32, N of 128";
   if (g.lda < g.K || g.ldw < g.K) return "f32 GEMM: bad leading dimension";
   if ((reinterpret_cast<uintptr_t>(g.A) | reinterpret_cast<uintptr_t>(g.W) | reinterpret_cast<uintptr_t>(g.C) |
-       reinterpret_cast<uintptr_t>(g.bias) | reinterpret_cast<uintptr_t>(g.ws) | reinterpret_cast<uintptr_t>(g.inv)) % 16)
+       reinterpret_cast<uintptr_t>(g.bias) | reinterpret_cast<uintptr_t>(g.ws) | reinterpret_cast<uintptr_t>(g.wexp)) % 16)
     return "f32 GEMM: operands must be 16-byte aligned";
   if (size_t(std::max(g.lda, g.ldw)) * 128 * 4 > 0xffffffffu) return "f32 GEMM: a tile's rows must span less than 4 GiB";
   if (g.splits < 1 || g.splits > g.K / 32) return "f32 GEMM: splits must be in 1..K/32";
@@ -688,9 +696,9 @@ void attn32_launch(const Attn32Args& a, hipStream_t st) {
   else hipLaunchKernelGGL(attn32_tile_kernel<4>, grid, dim3(256), 0, st, a);
 }
 
-void split_weight_launch(float* W, int N, int K, const float* bounds, float a, float* inv, hipStream_t st) {
+void split_weight_launch(float* W, int N, int K, const float* bounds, int* wexp, hipStream_t st) {
   const size_t n = size_t(N) * K;
-  hipLaunchKernelGGL(split_weight_kernel, dim3(unsigned((n + 255) / 256)), dim3(256), 0, st, W, n, K, bounds, a, inv);
+  hipLaunchKernelGGL(split_weight_kernel, dim3(unsigned((n + 255) / 256)), dim3(256), 0, st, W, n, K, bounds, wexp);
 }
 
 void weight_bound_launch(const float* W, const float* lw, const float* lb, const float* bias, int N, int K, float* out,

@@ -197,7 +197,7 @@ void rowdot_launch(const uint16_t* x, const float* w, const float* b, int R, int
 // ---- The dtype=f32 path (BackendOptions::f32): f32 weights and activations. The products' operands
 // are split f32 (device.hpp's split_f16), activations times a power of two, weights a row each.
 
-// C[M, N] (+)= act(A[M, K] . W[N, K]^T * inv + bias): A and W split, inv[n] = 1 / (A's scale, W row n's),
+// C[M, N] (+)= act(A[M, K] . W[N, K]^T * 2^(aexp + wexp[n]) + bias): A and W split, the exponents undo their scales,
 // C f32, or with cs > 0 split times cs; accumulate adds to an f32 C (the residual).
 struct Gemm32Args {
   const float* A = nullptr;  // [M, lda]
@@ -205,7 +205,8 @@ struct Gemm32Args {
   float* C = nullptr;        // [M, ldc]; null: a split product whose consumer sums the parts
   const float* bias = nullptr;
   int M = 0, N = 0, K = 0, lda = 0, ldw = 0, ldc = 0;
-  const float* inv = nullptr;  // [N]
+  const int* wexp = nullptr;  // [N]
+  int aexp = 0;
   float cs = 0.0f;
   int act = ACT_NONE;
   bool accumulate = false;
@@ -225,8 +226,8 @@ void gemm32_launch(const Gemm32Args& g, hipStream_t st);
 void split32_launch(const float* qkv, int splits, const float* bias, int T, int d, const int* pos, const float* cos_t,
                     const float* sin_t, float* q, float* k, float* v, hipStream_t st);
 // Splits W [N, K] (K a multiple of 64) in place, each row times a power of two by its largest element
-// in `bounds` (weight_bound_launch's), and fills inv [N] for inputs that are held times a.
-void split_weight_launch(float* W, int N, int K, const float* bounds, float a, float* inv, hipStream_t st);
+// in `bounds` (weight_bound_launch's), and fills wexp [N] with the exponents that undo them.
+void split_weight_launch(float* W, int N, int K, const float* bounds, int* wexp, hipStream_t st);
 // Bounds for the scales: for each row r of W [N, K] f32, out[2 r] = its largest |element| and
 // out[2 r + 1] = the most |W_r . x + bias_r| can be over all x = z * lw + lb with |z|_2 <= sqrt(K), what a
 // LayerNorm with weight lw and bias lb (or none) gives.

@@ -7,6 +7,7 @@
 #include "model.hpp"
 #include "selfcheck.hpp"
 
+#include <cfloat>
 #include <chrono>
 #include <condition_variable>
 #include <cstdio>
@@ -1439,7 +1440,8 @@ namespace {
 Gemm32Args gemm32_args(const Scales32& sc, const float* A, int lda, const float* W, int ldw, float* C, int ldc,
                        const float* bias, int M, int N, int K, int act, bool accumulate, float* ws, float cs = 0.0f) {
   Gemm32Args g;
-  g.inv = sc.inv;
+  g.wexp = sc.wexp;
+  g.aexp = sc.aexp;
   g.cs = cs;
   g.A = A;
   g.W = W;
@@ -1472,20 +1474,20 @@ Gemm32Args parts_of(Gemm32Args g) {
 // activations a bound that holds for every input. A LayerNorm's output is z * w + b with
 // |z|_2 <= sqrt(d), so each element and each product of it with a weight row is bounded
 // (weight_bound_launch); attention returns averages of v rows; |gelu(x) g| <= |x| |g|. Operands that stay
-// far below their bound lose nothing further: a split value keeps its 23 bits down to 2^-27 of it. (Bounds
-// outside 2^-40 to 2^60 take the scale of the nearer end.)
+// far below their bound lose nothing further: a split value keeps its 23 bits down to 2^-27 of it.
 void Model::split_weights32() {
   const int d = cfg.d, I = cfg.inter;
   const size_t most = size_t(std::max({3 * d, 2 * I, 4 * d, scorer_width}));
   const size_t rows = size_t(cfg.layers) * (5 * d + 2 * I) + size_t(cfg.head_layers) * 9 * d + scorer_width;
   hip_check(hipMalloc(&imem, (rows + most * 2) * 4), "hipMalloc(scales)");
-  float* inv = static_cast<float*>(imem);
-  float* const db = inv + rows;  // bounds of the weight at hand
+  int* wexp = static_cast<int*>(imem);
+  float* const db = static_cast<float*>(imem) + rows;  // bounds of the weight at hand
   std::vector<float> b(most * 2), hw(d), hb(d);
-  auto pow2 = [](double bound) {
+  auto exponent = [](double bound) {  // of the least power of two that is not below it
     int e = 0;
-    if (bound > 0.0 && std::isfinite(bound)) (void)std::frexp(bound, &e);  // bound <= 2^e
-    return float(std::ldexp(1.0, 15 - std::min(std::max(e, -40), 60)));
+    if (bound > double(FLT_MAX)) return 128;
+    if (bound > 0.0) (void)std::frexp(bound, &e);
+    return std::max(e, -111);
   };
   // What LayerNorm (lw, lb) can give, per element.
   auto norm = [&](const float* lw, const float* lb) {
@@ -1498,15 +1500,16 @@ void Model::split_weights32() {
   // Splits w [N, K], whose input is held times a, after reading its rows' bounds on an input of
   // LayerNorm (lw, lb) into b.
   auto weight = [&](uint16_t* w, int N, int K, double bound, const float* lw, const float* lb, const float* bias) {
-    Scales32 sc{pow2(bound), inv};
+    const int e = exponent(bound) - 15;
+    Scales32 sc{float(std::ldexp(1.0, -e)), e, wexp};
     float* W = const_cast<float*>(w32(w));
     weight_bound_launch(W, lw, lb, bias, N, K, db, stream);
     hip_check(hipGetLastError(), "weight bounds");
     hip_check(hipMemcpyAsync(b.data(), db, size_t(N) * 8, hipMemcpyDeviceToHost, stream), "read bounds");
-    split_weight_launch(W, N, K, db, sc.a, inv, stream);
+    split_weight_launch(W, N, K, db, wexp, stream);
     hip_check(hipGetLastError(), "split weight");
     hip_check(hipStreamSynchronize(stream), "split weight");
-    inv += N;
+    wexp += N;
     return sc;
   };
   auto most_of = [&](int r0, int r1) {

@@ -52,11 +52,12 @@ struct Settings {
   static Settings parse(const std::string& spec);
 };
 
-// dtype=f32: the power of two that a product's input is held times (split f32), and per output column
-// what undoes it and the weight row's.
+// dtype=f32: the power of two that a product's input is held times (split f32), the exponent that
+// undoes it, and per output column the one that undoes the weight row's.
 struct Scales32 {
   float a = 1.0f;
-  const float* inv = nullptr;
+  int aexp = 0;
+  const int* wexp = nullptr;
 };
 
 struct LayerWeights {
@@ -152,7 +153,7 @@ struct Model {
   size_t acap = 0;
   // the dtype=f32 path's activation arena
   void* fmem = nullptr;
-  void* imem = nullptr;  // the f32 products' inv arrays
+  void* imem = nullptr;  // the f32 products' wexp arrays
   size_t fcap = 0;
   // pinned host staging
   void* hmeta = nullptr;

@@ -257,10 +257,10 @@ def test_f32_tile_edges(lens, kmax):
     assert max(rel) <= REL_F64 and dl <= REL_F64, (rel, dl)  # logits are below 1
 
 
-def _rescaled(st: bytes, cfg: dict, span: int) -> bytes:
-    """The same model in exact arithmetic, its operands spread over 2 * span powers of two: channel k
-    of mlp_norm times 2^e_k and column k of Wi divided by it, gate row j of Wi times 2^f_j and column
-    j of Wo divided by it."""
+def _rescaled(st: bytes, cfg: dict, span: int, norm: int, gate: int) -> bytes:
+    """The same model in exact arithmetic, its operands spread over 2 * span powers of two around 2^norm
+    and 2^gate: channel k of mlp_norm times 2^e_k and column k of Wi divided by it, gate row j of Wi times
+    2^f_j and column j of Wo divided by it."""
     import struct
 
     n = struct.unpack("<Q", st[:8])[0]
@@ -277,18 +277,18 @@ def _rescaled(st: bytes, cfg: dict, span: int) -> bytes:
     inter = cfg["intermediate_size"]
     for l in range(cfg["num_hidden_layers"]):
         p = f"encoder.layers.{l}.mlp"
-        e = 2.0 ** rng.integers(-span, span + 1, cfg["hidden_size"])
-        f = 2.0 ** rng.integers(-span, span + 1, inter)
+        e = 2.0 ** (norm + rng.integers(-span, span + 1, cfg["hidden_size"]))
+        f = 2.0 ** (gate + rng.integers(-span, span + 1, inter))
         scale(p + "_norm.weight", e)
         scale(p + ".Wi.weight", np.concatenate([np.ones(inter), f])[:, None] / e[None, :])
         scale(p + ".Wo.weight", 1.0 / f[None, :])
     return bytes(out)
 
 
-@pytest.mark.parametrize("span", [6, 10])
-def test_f32_wide_operand_range(span):
+@pytest.mark.parametrize("span,norm,gate", [(6, 0, 0), (10, 0, 0), (6, -100, 0), (6, 70, 0), (6, 0, 80), (6, 0, -100)])
+def test_f32_wide_operand_range(span, norm, gate):
     """The split operands keep their precision over a wide range of magnitudes: a model whose MLP
-    operands are spread over 2^12 and 2^20 gives the plain model's results. Each operand is held to 2^-23
+    operands are spread over 2^12 and 2^20, or lie around a far power of two, gives the plain model's results. Each operand is held to 2^-23
     of its value either way, a product of two to 2^-21 (5e-7), and a sum of K = 1024 rounds to at most
     K 2^-24, typically its root (2e-6); three layers of two such products, doubled for the two models:
     2e-5 relative. An operand rounded to one f16 would be off by 2e-4 or more."""
@@ -300,13 +300,13 @@ def test_f32_wide_operand_range(span):
     b = collate([(rng.integers(0, 1000, L).tolist(), [1, L // 2], 0) for L in (70, 200, 33)], pad_id=1002)
     st = synth_checkpoint(json.dumps(cfg), json.dumps(AGENT), seed=6, scorer_width=256)
     outs = []
-    for image in (st, _rescaled(st, cfg, span)):
+    for image in (st, _rescaled(st, cfg, span, norm, gate)):
         m = HipBackend(image, json.dumps(cfg), json.dumps(AGENT), settings=DEFAULT_TUNING + ",dtype=f32", device=0)
         outs.append((m.encoder_hidden(b), m.forward(b)))
         m.close()
     rel = [float(np.linalg.norm(x - y) / np.linalg.norm(x)) for x, y in
            ((outs[0][0], outs[1][0]), (outs[0][1].pooled, outs[1][1].pooled), (outs[0][1].logits, outs[1][1].logits))]
-    say(f"f32 operands over 2^{2 * span}: hidden, pooled, logits rel {rel}")
+    say(f"f32 operands over 2^{2 * span} around 2^{norm}, 2^{gate}: hidden, pooled, logits rel {rel}")
     assert max(rel) <= 2e-5, rel
 
 
