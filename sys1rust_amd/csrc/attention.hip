@@ -328,9 +328,10 @@ typedef u32x4 u32x4_a8 __attribute__((aligned(8)));
 // from LDS then feeds two MFMAs, and half 1's softmax weights are computed beside half 0's V^T P^T
 // products. Two waves per SIMD: by counters a SIMD spends 475k cycles on VALU issue (an exp2 costs
 // two FMAs) and 262k on MFMAs at 8192 keys and 16 heads; at equal priority a launch took their
-// sum, 709k (counted before V^T went through registers), and takes 592k now. The priority raised over the weights and the V^T P^T products lets one wave's vector work
-// go ahead while the other's K Q^T products run (raised over K Q^T, or from the row maximum on, it
-// gains nothing). With this and the order of the tiles, against 8 waves of 32 queries, 16 heads:
+// sum, 709k (counted before V^T went through registers), and takes 592k now. The priority raised
+// over the weights and the V^T P^T products lets one wave's vector work go ahead while the other's
+// K Q^T products run (raised over K Q^T, or from the row maximum on, it gains nothing). With this
+// and the order of the tiles, against 8 waves of 32 queries, 16 heads:
 // 8192 keys 336 -> 310 µs (890 TFLOP/s), 10 rows of 547 to 579 tokens 34.1 -> 30.6, 12 of 300 to
 // 1100 61.3 -> 51.8, 48 of 215 to 2038 510 -> 481. The same work with 32 queries per wave and four
 // waves per SIMD (128 registers, 10 spilled) is 2 to 7% slower, and V^T in its own order in LDS, by direct loads, with a

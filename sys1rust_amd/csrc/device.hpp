@@ -67,13 +67,12 @@ struct F16 {
 };
 
 // A split f32 value: hi + lo / 2048, two f16 (hi the value rounded, lo what that leaves, scaled up so
-// that it keeps its bits below the smallest hi): 23 significant bits, one less than f32. Three quarters
-// of the f32 values are held exactly and the others to 2^-23 (4.2e-8 in the root mean square over a binade), for
-// values down to 2^-28 of f16's largest; weights that come from f16 or bf16 are exact.
-// (The split and its scaling by 2^11: Ootomo and Yokota, "Recovering single precision accuracy from Tensor
-// Cores while surpassing the FP32 theoretical peak performance", 2022.)
-// Operands of the f32 products are held so, times a power of two that keeps
-// them in range; a row keeps its bytes, [32 hi | 32 lo] for every 32 elements: element e of a
+// that it keeps its bits below the smallest hi): 23 significant bits, one less than f32. Three
+// quarters of the f32 values are held exactly and the others to 2^-23 (4.2e-8 in the root mean
+// square over a binade), for values down to 2^-28 of f16's largest; weights that come from f16 or
+// bf16 are exact. (The split and its scaling by 2^11: Ootomo and Yokota, "Recovering single
+// precision accuracy from Tensor Cores while surpassing the FP32 theoretical peak performance",
+// 2022.) Operands of the f32 products are held so, times a power of two that keeps them in range; a row keeps its bytes, [32 hi | 32 lo] for every 32 elements: element e of a
 // matrix (rows a multiple of 32) has hi at 16-bit index split_at(e) and lo 32 after it.
 __host__ __device__ inline size_t split_at(size_t e) { return (e & ~size_t(31)) * 2 + (e & 31); }
 template <int N>  // N consecutive values (a multiple of 2), scaled by sc

@@ -23,13 +23,13 @@ __device__ __forceinline__ float act32(float v, int act) {
 // C[M, N] = A[M, K] . W[N, K]^T of split operands: hi hi + (hi lo + lo hi) / 2048 on
 // v_mfma_f32_32x32x16_f16, each of the three exact and summed in f32, the two orders of magnitude in
 // accumulators of their own; lo lo, up to 2^-22 of a term, is left out. A term is then off by up to
-// 2^-21 (8e-8 in the root mean square; an f32 FMA: 2^-24 and 2.5e-8), but the sum is rounded a sixteenth as
-// often: of K terms of one size, normal values, relative root mean square against one FMA after the other, K 1: 7.9e-8
-// against 2.5e-8, 4: 8.3e-8, 4.0e-8, 16: 8.4e-8, 7.3e-8, 32: 8.6e-8, 1.0e-7, 256: 1.1e-7, 2.9e-7, 1024: 1.7e-7,
-// 5.7e-7. A sum that a few terms outweigh is less exact than by FMAs, the sums over the widths of
-// this model's layers (768 and more) more exact. Three 16-deep instructions take 96 clocks of a SIMD where the f32 matrix
-// instruction takes 512; what bounds these products is the power that they draw (the same launch on
-// zeros runs 1.4 times as fast). Against v_mfma_f32_32x32x2_f32 on the same tiles, M 5707:
+// 2^-21, 7.9e-8 in the root mean square (an f32 FMA: 2^-24 and 2.5e-8), but the sum is rounded a
+// sixteenth as often. Sums of K products of normal values, relative root mean square, here and by one
+// FMA after the other (emulated): K 4 8.3e-8, 4.0e-8; 16 8.4e-8, 7.3e-8; 32 8.6e-8, 1.0e-7; 256 1.1e-7, 2.9e-7;
+// 1024 1.7e-7, 5.7e-7. So a sum that a few terms outweigh is less exact than by FMAs, and the sums over
+// the widths of this model's layers (768 and more) are more exact. Three 16-deep instructions take 96
+// clocks of a SIMD where the f32 matrix instruction takes 512; what bounds these products is the power
+// that they draw (the same launch on zeros runs 1.4 times as fast). Against v_mfma_f32_32x32x2_f32 on the same tiles, M 5707:
 // N 3072, K 1024 330 -> 119 us (302 TFLOP/s); 1024, 1024 112 -> 39; 5248, 1024 524 -> 224; 1024, 2624
 // 279 -> 92; 4096, 1024 417 -> 168; 1024, 4096 425 -> 149, and the error against float64 from 5.7e-7 to
 // 2.2e-7 at K 1024, 1.2e-6 to 4.3e-7 at 4096 (fewer roundings of the sum). Splitting into three bf16
@@ -326,8 +326,8 @@ __global__ __launch_bounds__(256) void split32_kernel(const float* __restrict__ 
 // and its 16 KiB, shared by the waves of the workgroup through L1, are well within what that
 // allows, so there is nothing to stage and no barrier in the loop. The next tile's K is loaded
 // before this tile's softmax. The weights are exp2 of fma(s, log2 e, -max): the argument is rounded as
-// s - max would be, and a weight below 2^-126 of the row's largest is 0. Measured at 5707 tokens in 10 rows, 16 heads, against one wave per
-// (query, head) on vector FMAs: global 1720 -> 245 us, local
+// s - max would be, and a weight below 2^-126 of the row's largest is 0. Measured at 5707 tokens in
+// 10 rows, 16 heads, against one wave per (query, head) on vector FMAs: global 1720 -> 245 us, local
 // 402 -> 74 us.
 template <int KW>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void attn32_tile_kernel(Attn32Args a) {

@@ -82,11 +82,11 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, char* smem0, int m0
 
   // KG > 1 (k-groups): the workgroup holds KG groups of NW waves; group k runs k-tiles
   // [kt0 + k NK / KG, kt0 + (k + 1) NK / KG) on stage buffers of its own, and group 0 adds the
-  // other groups' accumulators, in
-  // group order, from LDS and runs the epilogue alone. A short GEMM's chain of dependent k-tiles
-  // is then KG times shorter on the same tiles. NK divides by KG, so that every group passes the same
-  // barriers, or with ODDK need not: a group with a k-tile less passes the last one's barrier all the
-  // same (a kernel of its own, since the uneven ranges cost each launch of the even one 0.06 µs).
+  // other groups' accumulators, in group order, from LDS and runs the epilogue alone. A short
+  // GEMM's chain of dependent k-tiles is then KG times shorter on the same tiles. NK divides by
+  // KG, so that every group passes the same barriers, or with ODDK need not: a group with a k-tile
+  // less passes the last one's barrier all the same (a kernel of its own, since the uneven ranges
+  // cost each launch of the even one 0.06 µs).
   const int grp = KG > 1 ? __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6) / NW : 0;
   const int tid = threadIdx.x - grp * NW * 64;
   char* const smem = smem0 + grp * STAGES * STAGE_BYTES;
