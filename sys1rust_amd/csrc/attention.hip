@@ -960,7 +960,7 @@ __global__ __launch_bounds__(KW * 64) __attribute__((amdgpu_waves_per_eu(2))) vo
 // is the lane's own weight). Loads go straight to registers: the sets are a few hundred keys that
 // the tiles of a row share through L2, and what bounds the kernel is each wave's chain of about
 // three key tiles. Measured at 1780 entries of 64 to 320 keys, 16 heads, against one wave per
-// (entry, head) on vector FMAs: 156 -> 22.4 us (20.9 without the care for values that are not finite).
+// (entry, head) on vector FMAs: 156 -> 20.7 us (20.3 without the care for values that are not finite).
 template <class E>
 __global__ __launch_bounds__(256) void attn_far_kernel(FallbackArgs a) {
   typedef typename E::v8 v8;
@@ -990,7 +990,7 @@ __global__ __launch_bounds__(256) void attn_far_kernel(FallbackArgs a) {
   f32x16 o[2];
 #pragma unroll
   for (int e = 0; e < 16; ++e) o[0][e] = o[1][e] = 0.0f;
-  uint32_t up = 0, down = 0;  // output elements that a value of +inf, of -inf (NaN: both) reaches
+  float most = 0.0f;  // the largest |value| met
   // 32-key tiles start 8-aligned, so V^T is read in aligned pieces of 4 keys; pieces past the range
   // repeat the one of its last key (values that meet weights of 0).
   const int first[2] = {tile[2] & ~7, tile[4] & ~7}, end[2] = {tile[3], tile[5]};
@@ -1040,8 +1040,7 @@ __global__ __launch_bounds__(256) void attn_far_kernel(FallbackArgs a) {
       o[1][e] *= alpha;
     }
     // A weight of 0 times a value that is not finite is NaN: such a value goes into the product as the
-    // largest finite one (NaN: the lowest), and the lanes whose query names its key note it.
-    float most = 0.0f;
+    // largest finite one (NaN: the lowest), and to the queries that name its key after the loop.
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
 #pragma unroll
@@ -1052,8 +1051,14 @@ __global__ __launch_bounds__(256) void attn_far_kernel(FallbackArgs a) {
         o[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(v, s[e], o[dt], 0, 0, 0);
       }
     }
-    if (__any(most == __FLT_MAX__)) {
-      for (int key = kb; key < min(kb + 32, last + 1); ++key) {
+  }
+  uint32_t up = 0, down = 0;  // output elements that a value of +inf, of -inf (NaN: both) reaches
+  if (__any(most == __FLT_MAX__)) {
+    for (int t = wave; t < na + nb; t += KW) {
+      const bool isb = t >= na;
+      const int kb = isb ? first[1] + (t - na) * 32 : first[0] + t * 32, stop = isb ? end[1] : end[0];
+      const int r0 = isb ? f0.w : f0.y, r1 = isb ? f1.x : f0.z;
+      for (int key = kb; key < min(kb + 32, stop); ++key) {
         const bool seen = key >= r0 && key < r1;
         for (int e = 0; e < 32; ++e) {
           const float v = E::f32(Vt[size_t((e >> 2) * 8 + 4 * hl + (e & 3)) * a.ldv + key]);
@@ -1080,8 +1085,10 @@ __global__ __launch_bounds__(256) void attn_far_kernel(FallbackArgs a) {
   mt[wave * 64 + lane] = m;
   lt[wave * 64 + lane] = l;
 #pragma unroll
-  for (int e = 0; e < 32; ++e)
-    ot[(wave * 32 + e) * 64 + lane] = o[e >> 4][e & 15] + ((up >> e & 1) ? -NEG_INF : 0.0f) + ((down >> e & 1) ? NEG_INF : 0.0f);
+  for (int e = 0; e < 32; ++e) ot[(wave * 32 + e) * 64 + lane] = o[e >> 4][e & 15];
+  if (__any((up | down) != 0))
+    for (int e = 0; e < 32; ++e)
+      ot[(wave * 32 + e) * 64 + lane] += ((up >> e & 1) ? -NEG_INF : 0.0f) + ((down >> e & 1) ? NEG_INF : 0.0f);
   __syncthreads();
   // Wave w combines and stores dims 8 w .. 8 w + 7 of both halves' pieces: g = w of each 32 dims.
   if (e0 + col >= e1) return;

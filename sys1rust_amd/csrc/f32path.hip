@@ -330,7 +330,7 @@ __global__ __launch_bounds__(256) void split32_kernel(const float* __restrict__ 
 // 10 rows, 16 heads, against one wave per (query, head) on vector FMAs: global 1720 -> 245 us, local
 // 402 -> 74 us.
 template <int KW>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void attn32_tile_kernel(Attn32Args a) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void attn32_tile_kernel(Attn32Args a) {
   constexpr float NEG_INF = -__builtin_huge_valf();
   __shared__ float mt[KW > 1 ? 4 * 64 : 1], lt[KW > 1 ? 4 * 64 : 1], ot[KW > 1 ? 4 * 32 * 64 : 1];
   const int lid = xcd_remap(blockIdx.x, gridDim.x);
@@ -364,7 +364,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void a
   f32x16 o[2];
 #pragma unroll
   for (int e = 0; e < 16; ++e) o[0][e] = o[1][e] = 0.0f;
-  uint32_t up = 0, down = 0;  // output elements that a value of +inf, of -inf (NaN: both) reaches
+  float most = 0.0f;  // the largest |value| met where keys are masked
   f32x4 kf[8];
   auto loadk = [&](int kb) __attribute__((always_inline)) {  // rows past the range repeat its last key
     const float* kr = Kh + size_t(min(kb + col, k1 - 1)) * 64 + hl * 4;
@@ -429,9 +429,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void a
       }
     }
     // Where keys are masked, a weight of 0 times a value that is not finite would be NaN: such a value
-    // goes into the product as the largest finite one (NaN: the lowest), and the lanes whose query
-    // sees its key note it.
-    float most = 0.0f;
+    // goes into the product as the largest finite one (NaN: the lowest), and to the queries that see
+    // its key after the loop.
     if (edge) {
 #pragma unroll
       for (int dt = 0; dt < 2; ++dt)
@@ -446,10 +445,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void a
       o[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(v[0][e], s[e], o[0], 0, 0, 0);
       o[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(v[1][e], s[e], o[1], 0, 0, 0);
     }
-    if (__any(most == __FLT_MAX__)) {
-      for (int j = 0; j < min(32, k1 - kb); ++j) {
-        const float* vk = Vh + size_t(kb + j) * 64 + 4 * hl;
-        const bool seen = a.window < 0 || abs(kb + j - qk) <= a.window;
+  }
+  uint32_t up = 0, down = 0;  // output elements that a value of +inf, of -inf (NaN: both) reaches
+  if (__any(most == __FLT_MAX__)) {
+    for (int kb = k0 + wk * 32; kb < k1; kb += KW * 32) {
+      for (int key = kb; key < min(kb + 32, k1); ++key) {
+        const float* vk = Vh + size_t(key) * 64 + 4 * hl;
+        const bool seen = a.window < 0 || abs(key - qk) <= a.window;
         for (int e = 0; e < 32; ++e) {
           const float x = vk[(e >> 2) * 8 + (e & 3)];
           if (!seen || fabsf(x) < -NEG_INF) continue;
@@ -459,8 +461,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void a
       }
     }
   }
-  auto sum = [&](int e) __attribute__((always_inline)) {
-    return o[e >> 4][e & 15] + ((up >> e & 1) ? -NEG_INF : 0.0f) + ((down >> e & 1) ? NEG_INF : 0.0f);
+  auto reached = [&](int e) __attribute__((always_inline)) {
+    return ((up >> e & 1) ? -NEG_INF : 0.0f) + ((down >> e & 1) ? NEG_INF : 0.0f);
   };
   l = half_sum(l);
   float L = l, f[KW];
@@ -468,7 +470,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void a
     mt[wave * 64 + lane] = m;
     lt[wave * 64 + lane] = l;
 #pragma unroll
-    for (int e = 0; e < 32; ++e) ot[(wave * 32 + e) * 64 + lane] = sum(e);
+    for (int e = 0; e < 32; ++e) ot[(wave * 32 + e) * 64 + lane] = o[e >> 4][e & 15];
+    if (__any((up | down) != 0))
+      for (int e = 0; e < 32; ++e) ot[(wave * 32 + e) * 64 + lane] += reached(e);
     __syncthreads();
     if (wk != 0) return;
     float M = m;
@@ -493,7 +497,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void a
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int e = g * 4 + r;
-        float acc = sum(dt * 16 + e);
+        float acc = o[dt][e] + reached(dt * 16 + e);
         if constexpr (KW > 1) {
           acc *= f[0];
 #pragma unroll
